@@ -82,7 +82,8 @@ int rqc_set_autotune(int on);
    fused qubits K per pass) and the most gates per pass (8 or 6) on the evaluation itself and keeps
    the fastest for that structure; on = 2 also forgets the choices made so far */
 int rqc_set_eval_autotune(int on);
-/* tile shape (2^rows x 2^cols amplitudes) and most gates per pass of the last evaluation */
+/* tile shape (2^rows x 2^cols amplitudes; 2^cols the elements of a contiguous run) and most gates
+   per pass of the last evaluation */
 int rqc_last_tiles(int* tile_rows_log2, int* tile_cols_log2, int* gates_per_pass);
 
 /* device workspace: upper bound in bytes (0 = automatic, about 85% of free HBM);
@@ -110,6 +111,9 @@ int rqc_profile_query(int kind, double* total_ms, long* launches, double* alg_by
    that pass's), and the flops the matrix cores issue for them: the reverse passes' state
    recovery besides, in the forms the kernels use (FP64 dual: forward 72, reverse 240, with three
    real products per complex gate product; FP32 the real 16 x 16 form: forward 128, reverse 384).
+   FP64 evaluations over the whole of a dense target sweep one array (U^dagger with the circuit's
+   gates on either side): its forward products count as forward (96, issued 72), a gate's
+   conjugation as reverse, by what it issues (144).
    No reference counterpart: the library's own measurement. */
 int rqc_profile_query_flops(int kind, double* alg_flops, double* issued_flops);
 

@@ -13,11 +13,13 @@
 // (src/quantum_circuit.c:147-236) evaluated for all columns of the block, with
 // the tangent-forward folded into the forward sweep (dual numbers).
 // The column blocks cover all N columns; B is the largest power of two whose
-// checkpoints fit the device workspace.
+// checkpoints fit the device workspace.  FP64 evaluations over the whole of a dense target that
+// has room for its arrays sweep the product U^dagger W itself instead (rqc_cyc_plan.hpp).
 
 #include <algorithm>
 #include <cstring>
 #include <functional>
+#include <list>
 #include <map>
 #include <string>
 #include <set>
@@ -27,6 +29,7 @@
 #include "rqc_eval.hpp"
 #include "rqc_kernels.hpp"
 #include "rqc_tile_kernels.hpp"
+#include "rqc_cyc_kernels.hpp"
 #include "mat4.hpp"
 #include "rqcopt/gate.h"
 #include "rqcopt/statevector.h"
@@ -711,6 +714,9 @@ struct TilePlan
 	size_t lds_fwd = 0, lds_rev = 0;
 	size_t lds_rev_seed = 0;        // the seed pass: also the fused forward pass's G, Z
 	size_t partial_doubles = 0;
+	// cyclic-product sweeps (EvalPlan::cyc): the launches and their grids
+	CycPlan cyc;
+	std::vector<unsigned> cyc_grid;
 };
 
 // Forward-pass tile: the forward pass holds half the states of the reverse pass
@@ -845,6 +851,119 @@ static std::shared_ptr<TilePlan> plan_tiles(const Context& dev, const Circuit& C
 	return tp;
 }
 
+// ---------------------------------------------------------------- cyclic-product sweeps
+typedef void (*CycKernel)(const CycArgs, const cx<double>*, zc*, long, zc*, const int*);
+
+// Waves of a workgroup (log2): 16 for the 64 x 64 tiles of dual sweeps (one workgroup per CU, four
+// waves per SIMD: L = 14, depth 9 HVP 64.5 ms against 66.6 with 8), 8 for those of plain sweeps (64 KiB
+// of LDS: two workgroups per CU cover each other's loads; L = 12, depth 7 gradient 1.03 ms against 1.17).
+constexpr int cyc_log_waves(int K, bool dual) { return K == 5 ? 2 : dual ? 4 : 3; }
+
+template <int K>
+static CycKernel cyc_kernel(bool dual, bool out)
+{
+	if (dual) { return out ? k_cyc_sweep<K, true, double, true, cyc_log_waves(K, true)> : k_cyc_sweep<K, true, double, false, cyc_log_waves(K, true)>; }
+	return out ? k_cyc_sweep<K, false, double, true, cyc_log_waves(K, false)> : k_cyc_sweep<K, false, double, false, cyc_log_waves(K, false)>;
+}
+
+static CycKernel cyc_kernel(int K, bool dual, bool out)
+{
+	return (K == 5) ? cyc_kernel<5>(dual, out) : cyc_kernel<6>(dual, out);
+}
+
+static int cyc_nthreads(int K, bool dual) { return 64 << cyc_log_waves(K, dual); }
+
+static size_t cyc_lds(int K, bool dual)
+{
+	if (K == 5) { return dual ? cyc_lds_bytes<5, true>() : cyc_lds_bytes<5, false>(); }
+	return dual ? cyc_lds_bytes<6, true>() : cyc_lds_bytes<6, false>();
+}
+
+// Tile qubits: 64 x 64 tiles fuse most gates per pass (L = 12, depth 7 HVP 2.40 ms, 32 x 32 tiles
+// 3.21 ms); below 10 qubits they leave most CUs idle (L = 8, depth 7: 16 tiles, 220 us against 64
+// tiles, 179 us; L = 9 gradient 134 us against 109 us; equal at 10 qubits).
+static int cyc_tile_qubits(int L) { return L >= 10 ? 6 : 5; }
+
+// Plans by circuit structure.  A program evaluates one structure many times with new gates; the
+// search costs up to a few milliseconds, as much as an evaluation of 10 qubits.  The last kMost
+// plans are kept (host memory only); the key holds the whole structure, nothing of the gates.
+class PlanCache
+{
+public:
+	std::shared_ptr<const TilePlan> get(const std::vector<int>& key, const std::function<std::shared_ptr<const TilePlan>()>& make)
+	{
+		std::lock_guard<std::mutex> lk(mu_);
+		for (auto it = plans_.begin(); it != plans_.end(); ++it) {
+			if (it->first == key) {
+				plans_.splice(plans_.begin(), plans_, it);
+				return it->second;
+			}
+		}
+		plans_.emplace_front(key, make());
+		if (plans_.size() > kMost) { plans_.pop_back(); }
+		return plans_.front().second;
+	}
+
+private:
+	static constexpr size_t kMost = 64;
+	std::mutex mu_;
+	std::list<std::pair<std::vector<int>, std::shared_ptr<const TilePlan>>> plans_;
+};
+
+static std::vector<int> structure_ints(const Circuit& C, std::initializer_list<int> head)
+{
+	std::vector<int> key(head);
+	key.push_back(C.L);
+	key.insert(key.end(), C.wi.begin(), C.wi.end());
+	key.insert(key.end(), C.wj.begin(), C.wj.end());
+	return key;
+}
+
+static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const Circuit& C, bool dual, bool target_only, int K)
+{
+	auto tp = std::make_shared<TilePlan>();
+	std::vector<int> gi(C.ngates), gj(C.ngates), bi, bj;
+	for (int k = 0; k < C.ngates; k++) {
+		gi[k] = C.L - 1 - C.wi[k];
+		gj[k] = C.L - 1 - C.wj[k];
+	}
+	// a circuit inside one tile: two passes of at most kCycOps gates suit the two directions
+	const int gmax = (C.L <= K) ? std::min(kCycOps, std::max(1, (C.ngates + 1) / 2)) : kCycOps;
+	std::vector<CycPass> passes = plan_cyc_passes(C.L, gi, gj, K, gmax);
+	for (CycPass& p : passes) {
+		for (int& k : p.slots) {
+			tp->order.push_back(k);
+			bi.push_back(gi[k]);
+			bj.push_back(gj[k]);
+			k = (int)tp->order.size() - 1;
+		}
+	}
+	tp->cyc = make_cyc_plan(C.L, K, passes, bi, bj, target_only, dual, kMatG, kMatGinv);
+	const size_t lds = cyc_lds(K, dual);
+	int occ = 0;
+	for (bool out : {false, true}) {
+		const CycKernel kf = cyc_kernel(K, dual, out);
+		allow_lds(kf, lds);
+		RQC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(kf), cyc_nthreads(K, dual), lds));
+	}
+	for (const CycLaunch& l : tp->cyc.launches) {
+		long n = 0;
+		for (int j = 0; j < l.njobs; j++) { n = std::max(n, 1L << l.job[j].ngen); }
+		// a power of two (the kernel steps its tiles by index bits)
+		long g = 1;
+		while (2 * g <= std::min<long>(n, (long)std::max(1, occ) * dev.cu_count)) { g *= 2; }
+		tp->cyc_grid.push_back((unsigned)g);
+	}
+	tp->passes.resize(passes.size());
+	return tp;
+}
+
+static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circuit& C, bool dual, bool target_only, int K)
+{
+	static PlanCache cache;
+	return cache.get(structure_ints(C, {K, dual, target_only, dev.device}), [&] { return make_cyc_tiles(dev, C, dual, target_only, K); });
+}
+
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, bool fp32, bool project, bool unitary,
@@ -873,6 +992,33 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	bool tiles = dev.engine == RQC_ENGINE_TILE_PASS && C.L <= 30 && (mode == Mode::Target || unitary);
 	TileShape ts{0, 0};
 	std::vector<Pass> passes;
+	// cyclic-product sweeps: the whole trace of a dense target, when its arrays fit
+	if (tiles && !pl.sampled && !fp32 && C.L >= 5 && 2 * (C.L - 6) <= kCycGens) {
+		const int K = cyc_tile_qubits(C.L);
+		const bool dual = (mode == Mode::Hvp);
+		auto tp = plan_cyc(dev, C, dual, mode == Mode::Target, K);
+		const int nst = tp->cyc.nbuf * (dual ? 2 : 1);
+		// (arrays that fit the held workspace need no look at the free memory)
+		const size_t need = (size_t)nst * pl.N * pl.N * elem;
+		size_t room = budget;
+		if (room == 0 && need <= held) { room = need; }
+		if (room == 0) {
+			size_t fr = 0, tot = 0;
+			RQC_HIP(hipMemGetInfo(&fr, &tot));
+			room = (size_t)(0.85 * (double)(fr + held));
+		}
+		if (need <= room) {
+			pl.tiles = pl.cyc = true;
+			pl.tp = tp;
+			pl.nst = nst;
+			pl.B = pl.N;
+			pl.passes = (int)tp->passes.size();
+			pl.tile_K = K;
+			pl.tile_logC = 4;   // runs of 16 elements in HBM
+			pl.gmax = kCycOps;
+			tiles = false;
+		}
+	}
 	if (tiles) {
 		ts = fp32 ? tile_shape<float>(C.L, pl.N, logE_c) : tile_shape<double>(C.L, pl.N, logE_c);
 		tiles = ts.usable();
@@ -892,7 +1038,7 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 		pl.tile_logC = ts.logC;
 		pl.gmax = gmax;
 		pl.tp = fp32 ? plan_tiles<float>(dev, C, pl, passes, ts) : plan_tiles<double>(dev, C, pl, passes, ts);
-	} else {
+	} else if (!pl.cyc) {
 		pl.nst = states_needed(mode, C.ngates);
 		pl.B = choose_block(pl.N, pl.nst, elem, budget, held, Bmax);
 		pl.passes = C.ngates;
@@ -902,7 +1048,12 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	pl.gtr = reduce_grid(pl.N * pl.B);
 	pl.n_acc = 1 + 32 * (size_t)pl.G;
 	size_t npart = pl.gtr;
-	if (pl.tiles) {
+	if (pl.cyc) {
+		// every gate's recorded partial traces, or the trace parts of a target evaluation
+		const CycPlan& cp = pl.tp->cyc;
+		npart = (mode == Mode::Target) ? (size_t)cp.ntrace * (cyc_nthreads(cp.K, false) / 64)
+		                               : (size_t)pl.G * cyc_parts(cp.L, cp.K) * (mode == Mode::Hvp ? 32 : 16);
+	} else if (pl.tiles) {
 		// outer-product partials, the chunk sums of the first reduction stage, then the trace
 		// partials of a first reverse pass that takes the target's trace
 		npart = std::max(npart, (pl.tp->partial_doubles + (size_t)kReduceChunks * kMaxTileGates * 256 + 1) / 2 +
@@ -910,7 +1061,10 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	}
 	else { npart = std::max(npart, (size_t)pl.grev_pg * kWidth); }
 	pl.n_part = npart;
-	if (pl.tiles) {
+	if (pl.cyc) {
+		pl.mats_bytes = align256((size_t)pl.G * kMats * 16 * sizeof(zc));
+		pl.terms_bytes = align256((size_t)pl.G * 2 * sizeof(int));   // each slot's gate and side
+	} else if (pl.tiles) {
 		pl.mats_bytes = align256((size_t)pl.G * kMats * 16 * elem);
 		pl.terms_bytes = align256((size_t)pl.G * sizeof(GateTerms));
 		if (!pl.tp->terms_fwd.empty()) { pl.terms_bytes += pl.tp->fterms_off; }   // the forward terms follow
@@ -966,6 +1120,10 @@ static void fill_tables(const EvalPlan& pl, const Circuit& C, char* host)
 				m4_transpose(m6[kMatGinv], rm);
 				m4_transpose(m6[kMatW], rm + 16);
 			}
+		}
+		if (pl.cyc) {
+			int* od = reinterpret_cast<int*>(host + pl.mats_bytes);
+			for (int x = 0; x < pl.G; x++) { od[2 * x] = tp.order[x]; od[2 * x + 1] = tp.cyc.up[x]; }
 		}
 		std::memcpy(host + pl.mats_bytes, tp.terms.data(), tp.terms.size() * sizeof(GateTerms));
 		if (!tp.terms_fwd.empty()) {
@@ -1194,6 +1352,53 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 	}
 }
 
+// cyclic-product sweeps of a dense target (rqc_cyc_plan.hpp)
+static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_partial, const char* tab, char* S,
+	const int* skip)
+{
+	const CycPlan& cp = pl.tp->cyc;
+	const bool dual = (pl.mode == Mode::Hvp);
+	const cx<double>* mats = reinterpret_cast<const cx<double>*>(tab);
+	const int* order = reinterpret_cast<const int*>(tab + pl.mats_bytes);
+	const zc* rmats = reinterpret_cast<const zc*>(tab + pl.rmats_off);
+	const size_t sz = (size_t)pl.N * pl.N * sizeof(cx<double>);
+	const int ns = dual ? 2 : 1;
+	const long nparts = cyc_parts(cp.L, cp.K);
+	const size_t lds = cyc_lds(cp.K, dual);
+	const double E = (double)(1L << (2 * cp.K)), side = dual ? 72.0 : 24.0;
+	for (size_t i = 0; i < cp.launches.size(); i++) {
+		const CycLaunch& l = cp.launches[i];
+		CycArgs a;
+		std::memset(&a, 0, sizeof(a));
+		double bytes = 0, flops = 0;
+		for (int j = 0; j < l.njobs; j++) {
+			a.job[j] = l.job[j];
+			const double amps = (double)(1L << l.job[j].ngen) * E;
+			for (int w = 0; w < ns; w++) {
+				a.in[j][w] = l.in[j] < 0 ? static_cast<const void*>(dU) : S + (size_t)(l.in[j] * ns + w) * sz;
+				a.out[j][w] = l.out[j] < 0 ? nullptr : S + (size_t)(l.out[j] * ns + w) * sz;
+			}
+			bytes += amps * sizeof(cx<double>) * ((l.in[j] < 0 ? 1 : ns) + (l.out[j] < 0 ? 0 : ns));
+			flops += amps * l.gate_sides[j] * side;
+		}
+		// algorithmic flops: a forward product in the direct complex form (the issued three-product
+		// form is 3/4 of it); a conjugation by what it issues (it replaces the adjoint update and the
+		// outer products of a gate)
+		LaunchTimer lt(s, l.reverse ? RQC_KERNEL_REVERSE : RQC_KERNEL_FORWARD, bytes, l.reverse ? flops : flops * (4.0 / 3.0),
+			flops);
+		const CycKernel kf = cyc_kernel(cp.K, dual, l.out[0] >= 0);
+		kf<<<dim3(pl.tp->cyc_grid[i], l.njobs), cyc_nthreads(cp.K, dual), lds, s.stream>>>(a, mats, d_partial, nparts, d_partial, skip);
+	}
+	LaunchTimer lt(s, RQC_KERNEL_OTHER);
+	if (pl.mode == Mode::Target) {
+		k_cyc_trace<<<1, kBlock, 0, s.stream>>>(d_partial, cp.ntrace * (cyc_nthreads(cp.K, false) / 64), d_acc, skip);
+	} else if (dual) {
+		k_cyc_reduce<true><<<pl.G, 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, skip);
+	} else {
+		k_cyc_reduce<false><<<pl.G, 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, skip);
+	}
+}
+
 // per-group sums of per-gate gradients / HVPs and the Riemannian projection
 // (reference src/target.c:526-535 and :650-671), one thread per group.
 // res: f, dv[16 ng], hz[16 ng] (complex), grad[16 ng], hvp[16 ng] (double)
@@ -1271,12 +1476,14 @@ void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit
 	s.last_logC = pl.tiles ? pl.tile_logC : 0;
 	s.last_gmax = pl.tiles ? pl.gmax : 0;
 	s.last_passes = pl.passes;
-	{
+	if (!pl.cyc) {
 		LaunchTimer lt(s, RQC_KERNEL_OTHER);
 		k_fill_zero<<<nblocks((long)pl.n_acc), kBlock, 0, s.stream>>>(acc, (long)pl.n_acc, skip);
 	}
 	const GateTerms* gterms = reinterpret_cast<const GateTerms*>(tab + pl.mats_bytes);
-	if (pl.fp32) {
+	if (pl.cyc) {
+		run_cyc(s, pl, dU, acc, part, tab, work + pl.off_states, skip);
+	} else if (pl.fp32) {
 		cx<float>* S = reinterpret_cast<cx<float>*>(work + pl.off_states);
 		const cx<float>* Xs = static_cast<const cx<float>*>(X);
 		if (pl.tiles) { run_tiles<float>(s, pl, dU, acc, part, reinterpret_cast<const cx<float>*>(tab), gterms, S, skip, Xs, W, be); }
@@ -1348,7 +1555,7 @@ static TileChoice tune_eval(Context& c, const Circuit& C, Mode mode, int per, bo
 		} catch (const Error&) {
 			continue;   // a candidate that does not fit is skipped
 		}
-		if (!pl.tiles) { break; }   // no tile-pass plan: nothing to tune
+		if (!pl.tiles || pl.cyc) { break; }   // no tile shape to tune
 		std::vector<char> tab(pl.tab_bytes);
 		fill_eval_tables(pl, C, tab.data());
 		c.work.reserve(pl.bytes);

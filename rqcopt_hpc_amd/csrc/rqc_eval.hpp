@@ -61,6 +61,7 @@ struct EvalPlan
 	bool fp32 = false;     // complex FP32 sweeps (mixed precision)
 	bool project = false;  // Riemannian projection of gradient and HVP
 	bool tiles = false;    // tile-pass engine (else one gate per pass)
+	bool cyc = false;      // cyclic-product sweeps (with tiles; rqc_cyc_plan.hpp)
 	int L = 0, G = 0, per = 1, ng = 0;
 	long N = 0, B = 0;     // 2^L and the column-block width
 	bool sampled = false;  // columns are given states (stochastic trace), not the basis

@@ -1,0 +1,84 @@
+"""Cyclic-product sweeps (rqc_cyc_kernels.hpp): target, gradient and HVP of dense targets against
+the oracle and the per-gate engine, at the sizes where plans and tiles change.
+
+5 qubits is the smallest tile, 9 / 10 the change of the tile size, and the gate counts cover one
+gate (no conjugation), passes of one gate, full passes of 8 and the next pass's first gate; random
+wires give passes with one-sided launches, any wire order and gates that repeat a pair.  FP64 sums
+of up to 2^22 products of magnitude 1 / N rounded at 2^-53 stay within 1e-12 of either engine.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+import rqcopt_hpc_amd as R
+from helpers import brickwall_perms, crandn, haar_unitary, reldiff
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+@pytest.fixture(autouse=True)
+def fp64():
+    R.require_gpu()
+    R.set_precision(R.PRECISION_FP64)
+    yield
+    R.set_sweep_engine(R.ENGINE_TILE_PASS)
+    R.set_workspace_limit(0)
+
+
+def _all(T, g, z, w, L):
+    return (R.circuit_unitary_target(T, g, w, L), R.circuit_unitary_target_and_gradient(T, g, w, L),
+            R.circuit_unitary_target_hessian_vector_product(T, g, z, w, L))
+
+
+def _check(a, f, dg, hg):
+    assert reldiff(a[0], f) < TOL
+    assert reldiff(a[1][0], f) < TOL and reldiff(a[1][1], dg) < TOL
+    assert reldiff(a[2][0], f) < TOL and reldiff(a[2][1], dg) < TOL
+    if np.max(np.abs(hg)) > 0:
+        assert reldiff(a[2][2], hg) < TOL
+    else:
+        assert np.max(np.abs(a[2][2])) < TOL * np.max(np.abs(dg))
+
+
+@pytest.mark.parametrize("L,ngates", [(5, 1), (5, 8), (5, 17), (6, 2), (6, 9), (7, 1), (7, 33), (8, 16), (9, 25), (10, 9),
+                                      (10, 40), (11, 23)])
+def test_random_circuits_match_oracle(L, ngates):
+    print("qubits", L, "gates", ngates, flush=True)
+    rng = np.random.default_rng(100 * L + ngates)
+    g = np.stack([haar_unitary(rng) for _ in range(ngates)])
+    z = crandn(rng, (ngates, 4, 4))
+    w = np.array([rng.choice(L, 2, replace=False) for _ in range(ngates)], dtype=np.int32)
+    U = crandn(rng, (1 << L, 1 << L)) / (1 << (L // 2))
+    T = R.DeviceTarget.dense(U)
+    a = _all(T, g, z, w, L)
+    assert R.last_sweep()[0] == R.ENGINE_TILE_PASS and R.last_column_block() == 1 << L
+    if L <= 8:
+        _check(a, *O.circuit_unitary_target_hvp(O.Ufunc.dense(U), g, z, w, L))
+    R.set_sweep_engine(R.ENGINE_PER_GATE)
+    b = _all(T, g, z, w, L)
+    _check(a, b[0], b[1][1], b[2][2])
+
+
+@pytest.mark.parametrize("L,depth", [(6, 1), (10, 4), (12, 2), (12, 5)])
+def test_brickwalls_match_the_column_sweeps(L, depth):
+    """The same evaluation with and without room for the N x N arrays (column blocks of the tile
+    passes), and repeated: bitwise equal."""
+    print("qubits", L, "layers", depth, flush=True)
+    rng = np.random.default_rng(7 * L + depth)
+    V = np.stack([haar_unitary(rng) for _ in range(depth)])
+    Z = crandn(rng, (depth, 4, 4))
+    P = brickwall_perms(L, depth)
+    T = R.DeviceTarget.brickwall(np.stack([haar_unitary(rng) for _ in range(3)]), brickwall_perms(L, 3))
+    a = R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+    b = R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    ft = R.brickwall_unitary_target(T, V, P)
+    R.set_workspace_limit(max(1 << 20, (1 << (2 * L)) * 16 // 4))
+    c = R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+    assert R.last_column_block() < 1 << L or L == 6
+    assert reldiff(ft, a[0]) < TOL
+    for x, y in zip(a, c):
+        assert reldiff(x, y) < TOL
