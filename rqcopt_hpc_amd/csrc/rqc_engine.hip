@@ -1400,7 +1400,11 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 }
 
 // per-group sums of per-gate gradients / HVPs and the Riemannian projection
-// (reference src/target.c:526-535 and :650-671), one thread per group.
+// (reference src/target.c:526-535 and :650-671; m4_project_grad_hvp), one
+// workgroup per group, an entry of a 4x4 matrix per thread.  One thread per
+// group, with the sums and the six 4x4 products in series, took 28 us at 3
+// groups of 3 gates and 60 us at 9 groups of 7; the entries' loads are
+// independent here (4 and 6 us).
 // res: f, dv[16 ng], hz[16 ng] (complex), grad[16 ng], hvp[16 ng] (double)
 // fcorr (FP32 sweeps with a gradient): the sweeps applied the gates rounded to
 // complex float, fl(V), so the accumulated f is f(fl(V)).  f(V) = f(fl(V)) +
@@ -1408,46 +1412,85 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 // holomorphic in the gates for the trace targets: fcorr 1 corrects the complex
 // f; the block-encoding f is real with df = Re sum dv dV: fcorr 2 corrects its
 // real part).  Every gate of a group is the group's gate vlist[l].
-__global__ void k_finalize(const zc* __restrict__ acc, int ngroups, int per, const zc* __restrict__ vlist,
-	const zc* __restrict__ vdirs, zc* __restrict__ res, int want_grad, int project, int want_hvp, int fcorr,
-	const int* skip)
+__global__ __launch_bounds__(kBlock) void k_finalize(const zc* __restrict__ acc, int ngroups, int per,
+	const zc* __restrict__ vlist, const zc* __restrict__ vdirs, zc* __restrict__ res, int want_grad, int project, int want_hvp,
+	int fcorr, const int* skip)
 {
 	if (skipped(skip)) { return; }
-	const int l = blockIdx.x * blockDim.x + threadIdx.x;
+	const int l = blockIdx.x, t = threadIdx.x;
+	// entry e of group g's sums (e < 16: gradient, else HVP), over its gates in order
+	auto group_sum = [&](int g, int e) {
+		zc s = {0, 0};
+#pragma unroll 8
+		for (int k = 0; k < per; k++) { s += acc[1 + 32L * ((long)g * per + k) + e]; }
+		return s;
+	};
 	if (l == 0) {
-		zc f = acc[0];
+		zc c[1] = {{0, 0}};
+		__shared__ zc corr[1];
 		if (want_grad && fcorr != 0) {
-			zc c = {0, 0};
-			for (int g = 0; g < ngroups; g++) {
-				for (int e = 0; e < 16; e++) {
-					const zc v = vlist[16 * g + e];
-					const zc dv = {v.x - (double)(float)v.x, v.y - (double)(float)v.y};
-					zc s = {0, 0};
-					for (int k = 0; k < per; k++) { s += acc[1 + 32L * ((long)g * per + k) + e]; }
-					c.x += s.x * dv.x - s.y * dv.y;
-					c.y += s.x * dv.y + s.y * dv.x;
-				}
+			for (int i = t; i < 16 * ngroups; i += kBlock) {
+				const zc v = vlist[i];
+				const zc dv = {v.x - (double)(float)v.x, v.y - (double)(float)v.y};
+				const zc s = group_sum(i >> 4, i & 15);
+				c[0].x += s.x * dv.x - s.y * dv.y;
+				c[0].y += s.x * dv.y + s.y * dv.x;
 			}
-			f.x += c.x;
-			if (fcorr == 1) { f.y += c.y; }
+			block_sum_store<1>(c, corr);
+			__syncthreads();
+			c[0] = corr[0];
 		}
-		res[0] = f;
+		if (t == 0) {
+			zc f = acc[0];
+			f.x += c[0].x;
+			if (fcorr == 1) { f.y += c[0].y; }
+			res[0] = f;
+		}
 	}
 	if (!want_grad || l >= ngroups) { return; }
 	zc* dv_out = res + 1;
 	zc* hz_out = dv_out + 16L * ngroups;
 	double* grad = reinterpret_cast<double*>(hz_out + 16L * ngroups);
 	double* hvp = grad + 16L * ngroups;
-	zc dv[16], hz[16];
-	for (int e = 0; e < 16; e++) { dv[e] = {0, 0}; hz[e] = {0, 0}; }
-	for (int k = 0; k < per; k++) {
-		const zc* a = acc + 1 + 32L * ((long)l * per + k);
-		for (int e = 0; e < 16; e++) { dv[e] += a[e]; hz[e] += a[16 + e]; }
+	__shared__ zc V[16], Z[16], A[2][16], U[2][16], W[2][16];   // A: conj of the sums (gradient, HVP)
+	const int h = (t >> 4) & 1, e = t & 15, r = e >> 2, c = e & 3;
+	const bool on = t < 32;
+	if (on) {
+		const zc s = group_sum(l, t);
+		(h ? hz_out : dv_out)[16 * l + e] = s;
+		A[h][e] = conj(s);
+		if (h) { Z[e] = want_hvp ? vdirs[16 * l + e] : zc{0, 0}; }
+		else { V[e] = vlist[16 * l + e]; }
 	}
-	for (int e = 0; e < 16; e++) { dv_out[16 * l + e] = dv[e]; hz_out[16 * l + e] = hz[e]; }
-	if (project) {
-		m4_project_grad_hvp(vlist + 16 * l, want_hvp ? vdirs + 16 * l : nullptr, dv, hz, grad + 16 * l,
-			want_hvp ? hvp + 16 * l : nullptr);
+	if (!project) { return; }
+	__syncthreads();
+	// the symmetric triple product (Z g^dagger V + V g^dagger Z) / 2 of the HVP's correction
+	if (on) {
+		const zc* X = h ? V : Z;
+		zc s = {0, 0};
+		for (int k = 0; k < 4; k++) { s += X[4 * r + k] * conj(A[0][4 * c + k]); }
+		U[h][e] = s;
+	}
+	__syncthreads();
+	if (on) {
+		const zc* X = h ? Z : V;
+		zc s = {0, 0};
+		for (int k = 0; k < 4; k++) { s += U[h][4 * r + k] * X[4 * k + c]; }
+		W[h][e] = s;
+	}
+	__syncthreads();
+	if (on && h) { A[1][e] -= 0.5 * (W[0][e] + W[1][e]); }
+	__syncthreads();
+	// tangent coordinates: the skew-Hermitian part of V^dagger A, Re + Im by entry
+	if (on) {
+		zc s = {0, 0};
+		for (int k = 0; k < 4; k++) { s += conj(V[4 * k + r]) * A[h][4 * k + c]; }
+		U[h][e] = s;
+	}
+	__syncthreads();
+	if (on && (!h || want_hvp)) {
+		const zc a = U[h][e], b = conj(U[h][4 * c + r]);
+		(h ? hvp : grad)[16 * l + e] = (r == c) ? a.y : (0.5 * (a - b)).x + (0.5 * (a - b)).y;
 	}
 }
 
@@ -1495,7 +1538,7 @@ void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit
 		else { run_gates<double>(s, pl, C, dU, acc, part, S, skip, Xs, W, be); }
 	}
 	LaunchTimer lt(s, RQC_KERNEL_OTHER);
-	k_finalize<<<std::max(1, (pl.ng + 63) / 64), 64, 0, s.stream>>>(acc, pl.ng, pl.per, vin, vin + 16 * (size_t)pl.ng, res,
+	k_finalize<<<pl.mode != Mode::Target ? pl.ng : 1, kBlock, 0, s.stream>>>(acc, pl.ng, pl.per, vin, vin + 16 * (size_t)pl.ng, res,
 		pl.mode != Mode::Target ? 1 : 0, pl.project ? 1 : 0, pl.mode == Mode::Hvp ? 1 : 0,
 		pl.fp32 ? (be != nullptr ? 2 : 1) : 0, skip);
 }
