@@ -507,6 +507,48 @@ static std::vector<Pass> plan_passes(const Circuit& C, int K, int gmax)
 	return out;
 }
 
+// Plans by circuit structure.  A program evaluates one structure many times with new gates; the
+// search costs up to a few milliseconds, as much as an evaluation of 10 qubits.  The last kMost
+// plans are kept (host memory only); the key holds the whole structure, nothing of the gates.
+template <typename P>
+class PlanCache
+{
+public:
+	std::shared_ptr<const P> get(const std::vector<int>& key, const std::function<std::shared_ptr<const P>()>& make)
+	{
+		std::lock_guard<std::mutex> lk(mu_);
+		for (auto it = plans_.begin(); it != plans_.end(); ++it) {
+			if (it->first == key) {
+				plans_.splice(plans_.begin(), plans_, it);
+				return it->second;
+			}
+		}
+		plans_.emplace_front(key, make());
+		if (plans_.size() > kMost) { plans_.pop_back(); }
+		return plans_.front().second;
+	}
+
+private:
+	static constexpr size_t kMost = 64;
+	std::mutex mu_;
+	std::list<std::pair<std::vector<int>, std::shared_ptr<const P>>> plans_;
+};
+
+static std::vector<int> structure_ints(const Circuit& C, std::initializer_list<int> head)
+{
+	std::vector<int> key(head);
+	key.push_back(C.L);
+	key.insert(key.end(), C.wi.begin(), C.wi.end());
+	key.insert(key.end(), C.wj.begin(), C.wj.end());
+	return key;
+}
+
+static std::vector<Pass> cached_passes(const Circuit& C, int K, int gmax)
+{
+	static PlanCache<std::vector<Pass>> cache;
+	return *cache.get(structure_ints(C, {K, gmax}), [&] { return std::make_shared<const std::vector<Pass>>(plan_passes(C, K, gmax)); });
+}
+
 // Kernel arguments of a pass.  Tile-bit order: the two least used bits of the
 // pass go to the top tile positions (wave ownership of quads changes, and a
 // barrier is needed, only between consecutive gates whose two highest non-gate
@@ -884,41 +926,6 @@ static size_t cyc_lds(int K, bool dual)
 // tiles, 179 us; L = 9 gradient 134 us against 109 us; equal at 10 qubits).
 static int cyc_tile_qubits(int L) { return L >= 10 ? 6 : 5; }
 
-// Plans by circuit structure.  A program evaluates one structure many times with new gates; the
-// search costs up to a few milliseconds, as much as an evaluation of 10 qubits.  The last kMost
-// plans are kept (host memory only); the key holds the whole structure, nothing of the gates.
-class PlanCache
-{
-public:
-	std::shared_ptr<const TilePlan> get(const std::vector<int>& key, const std::function<std::shared_ptr<const TilePlan>()>& make)
-	{
-		std::lock_guard<std::mutex> lk(mu_);
-		for (auto it = plans_.begin(); it != plans_.end(); ++it) {
-			if (it->first == key) {
-				plans_.splice(plans_.begin(), plans_, it);
-				return it->second;
-			}
-		}
-		plans_.emplace_front(key, make());
-		if (plans_.size() > kMost) { plans_.pop_back(); }
-		return plans_.front().second;
-	}
-
-private:
-	static constexpr size_t kMost = 64;
-	std::mutex mu_;
-	std::list<std::pair<std::vector<int>, std::shared_ptr<const TilePlan>>> plans_;
-};
-
-static std::vector<int> structure_ints(const Circuit& C, std::initializer_list<int> head)
-{
-	std::vector<int> key(head);
-	key.push_back(C.L);
-	key.insert(key.end(), C.wi.begin(), C.wi.end());
-	key.insert(key.end(), C.wj.begin(), C.wj.end());
-	return key;
-}
-
 static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const Circuit& C, bool dual, bool target_only, int K)
 {
 	auto tp = std::make_shared<TilePlan>();
@@ -960,7 +967,7 @@ static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const 
 
 static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circuit& C, bool dual, bool target_only, int K)
 {
-	static PlanCache cache;
+	static PlanCache<TilePlan> cache;
 	return cache.get(structure_ints(C, {K, dual, target_only, dev.device}), [&] { return make_cyc_tiles(dev, C, dual, target_only, K); });
 }
 
@@ -1024,7 +1031,7 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 		tiles = ts.usable();
 	}
 	if (tiles) {
-		passes = plan_passes(C, ts.K, gmax);
+		passes = cached_passes(C, ts.K, gmax);
 		const int P = (int)passes.size();
 		pl.nst = (mode == Mode::Target) ? 2 : (mode == Mode::Grad) ? P + 2 : 2 * P + 4;
 		pl.B = choose_block(pl.N, pl.nst, elem, budget, held, Bmax);
