@@ -773,6 +773,7 @@ static void batch_optimize_device(Batch& bt, const struct mat4x4* const* vstart,
 			d.ng = pl.ng;
 			d.mode = (int)pl.mode;
 			d.fp32 = pl.fp32 ? 1 : 0;
+			d.round_gates = (pl.fp32 && pl.cyc) ? 1 : 0;
 		}
 	}
 	const DeviceTableDesc* d_desc = reinterpret_cast<const DeviceTableDesc*>(bt.dmem + bt.off_desc);

@@ -901,16 +901,19 @@ typedef void (*CycKernel)(const CycArgs, const cx<double>*, zc*, long, zc*, cons
 // of LDS: two workgroups per CU cover each other's loads; L = 12, depth 7 gradient 1.03 ms against 1.17).
 constexpr int cyc_log_waves(int K, bool dual) { return K == 5 ? 2 : dual ? 4 : 3; }
 
-template <int K>
+template <int K, typename TS>
 static CycKernel cyc_kernel(bool dual, bool out)
 {
-	if (dual) { return out ? k_cyc_sweep<K, true, double, true, cyc_log_waves(K, true)> : k_cyc_sweep<K, true, double, false, cyc_log_waves(K, true)>; }
-	return out ? k_cyc_sweep<K, false, double, true, cyc_log_waves(K, false)> : k_cyc_sweep<K, false, double, false, cyc_log_waves(K, false)>;
+	constexpr int LD = cyc_log_waves(K, true), LP = cyc_log_waves(K, false);
+	if (dual) { return out ? k_cyc_sweep<K, true, TS, true, LD> : k_cyc_sweep<K, true, TS, false, LD>; }
+	return out ? k_cyc_sweep<K, false, TS, true, LP> : k_cyc_sweep<K, false, TS, false, LP>;
 }
 
-static CycKernel cyc_kernel(int K, bool dual, bool out)
+// fp32: the arrays between launches in complex FP32 (mixed precision)
+static CycKernel cyc_kernel(int K, bool dual, bool fp32, bool out)
 {
-	return (K == 5) ? cyc_kernel<5>(dual, out) : cyc_kernel<6>(dual, out);
+	if (fp32) { return (K == 5) ? cyc_kernel<5, float>(dual, out) : cyc_kernel<6, float>(dual, out); }
+	return (K == 5) ? cyc_kernel<5, double>(dual, out) : cyc_kernel<6, double>(dual, out);
 }
 
 static int cyc_nthreads(int K, bool dual) { return 64 << cyc_log_waves(K, dual); }
@@ -926,7 +929,7 @@ static size_t cyc_lds(int K, bool dual)
 // tiles, 179 us; L = 9 gradient 134 us against 109 us; equal at 10 qubits).
 static int cyc_tile_qubits(int L) { return L >= 10 ? 6 : 5; }
 
-static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const Circuit& C, bool dual, bool target_only, int K)
+static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const Circuit& C, bool dual, bool fp32, bool target_only, int K)
 {
 	auto tp = std::make_shared<TilePlan>();
 	std::vector<int> gi(C.ngates), gj(C.ngates), bi, bj;
@@ -949,7 +952,7 @@ static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const 
 	const size_t lds = cyc_lds(K, dual);
 	int occ = 0;
 	for (bool out : {false, true}) {
-		const CycKernel kf = cyc_kernel(K, dual, out);
+		const CycKernel kf = cyc_kernel(K, dual, fp32, out);
 		allow_lds(kf, lds);
 		RQC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(kf), cyc_nthreads(K, dual), lds));
 	}
@@ -965,10 +968,11 @@ static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const 
 	return tp;
 }
 
-static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circuit& C, bool dual, bool target_only, int K)
+static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circuit& C, bool dual, bool fp32, bool target_only, int K)
 {
 	static PlanCache<TilePlan> cache;
-	return cache.get(structure_ints(C, {K, dual, target_only, dev.device}), [&] { return make_cyc_tiles(dev, C, dual, target_only, K); });
+	return cache.get(structure_ints(C, {K, dual, fp32, target_only, dev.device}),
+		[&] { return make_cyc_tiles(dev, C, dual, fp32, target_only, K); });
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1000,10 +1004,10 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	TileShape ts{0, 0};
 	std::vector<Pass> passes;
 	// cyclic-product sweeps: the whole trace of a dense target, when its arrays fit
-	if (tiles && !pl.sampled && !fp32 && C.L >= 5 && 2 * (C.L - 6) <= kCycGens) {
+	if (tiles && !pl.sampled && C.L >= 5 && 2 * (C.L - 6) <= kCycGens) {
 		const int K = cyc_tile_qubits(C.L);
 		const bool dual = (mode == Mode::Hvp);
-		auto tp = plan_cyc(dev, C, dual, mode == Mode::Target, K);
+		auto tp = plan_cyc(dev, C, dual, fp32, mode == Mode::Target, K);
 		const int nst = tp->cyc.nbuf * (dual ? 2 : 1);
 		// (arrays that fit the held workspace need no look at the free memory)
 		const size_t need = (size_t)nst * pl.N * pl.N * elem;
@@ -1090,6 +1094,8 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	return pl;
 }
 
+RQC_HD static zc round_float(zc v) { return zc{(double)(float)v.x, (double)(float)v.y}; }
+
 template <typename T>
 static void fill_tables(const EvalPlan& pl, const Circuit& C, char* host)
 {
@@ -1100,7 +1106,12 @@ static void fill_tables(const EvalPlan& pl, const Circuit& C, char* host)
 		for (size_t x = 0; x < tp.order.size(); x++) {
 			const int k = tp.order[x];
 			// G, Z, G^-1, -G^-1 Z G^-1, G^T, Z^T (kMats matrices, zero where unused)
-			const zc* g = &C.gates[16 * (size_t)k];
+			zc gr[16];
+			std::memcpy(gr, &C.gates[16 * (size_t)k], sizeof(gr));
+			// (mixed cyclic-product sweeps: FP64 products of the gates rounded to complex float, which
+			// is what the correction of f in k_finalize assumes)
+			if (pl.cyc && pl.fp32) { for (zc& v : gr) { v = round_float(v); } }
+			const zc* g = gr;
 			zc m6[kMats][16];
 			std::memset(m6, 0, sizeof(m6));
 			std::memcpy(m6[kMatG], g, sizeof(m6[0]));
@@ -1149,7 +1160,7 @@ static void fill_tables(const EvalPlan& pl, const Circuit& C, char* host)
 void fill_eval_tables(const EvalPlan& pl, const Circuit& C, char* host)
 {
 	std::memset(host, 0, pl.tab_bytes);
-	if (pl.fp32) { fill_tables<float>(pl, C, host); }
+	if (pl.fp32 && !pl.cyc) { fill_tables<float>(pl, C, host); }
 	else { fill_tables<double>(pl, C, host); }
 }
 
@@ -1172,7 +1183,11 @@ __device__ void fill_slots_device(const DeviceTableDesc& d)
 	cx<T>* hm = reinterpret_cast<cx<T>*>(d.tab);
 	for (int x = threadIdx.x; x < d.G; x += blockDim.x) {
 		const int l = d.slot_group[x];
-		const zc* g = d.gates + 16 * (size_t)l;
+		zc g[16];
+		for (int e = 0; e < 16; e++) {
+			g[e] = d.gates[16 * (size_t)l + e];
+			if (d.round_gates) { g[e] = round_float(g[e]); }
+		}
 		zc m6[kMats][16];
 		for (int w = 0; w < kMats; w++) { m4_zero(m6[w]); }
 		for (int e = 0; e < 16; e++) { m6[kMatG][e] = g[e]; }
@@ -1208,7 +1223,7 @@ __global__ __launch_bounds__(64) void k_fill_tables(const DeviceTableDesc* __res
 {
 	const DeviceTableDesc& d = descs[blockIdx.x];
 	if (d.skip != nullptr && *d.skip != 0) { return; }
-	if (d.fp32) { fill_slots_device<float>(d); }
+	if (d.fp32 && !d.round_gates) { fill_slots_device<float>(d); }
 	else { fill_slots_device<double>(d); }
 }
 
@@ -1368,7 +1383,7 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 	const cx<double>* mats = reinterpret_cast<const cx<double>*>(tab);
 	const int* order = reinterpret_cast<const int*>(tab + pl.mats_bytes);
 	const zc* rmats = reinterpret_cast<const zc*>(tab + pl.rmats_off);
-	const size_t sz = (size_t)pl.N * pl.N * sizeof(cx<double>);
+	const size_t elem = pl.fp32 ? sizeof(cx<float>) : sizeof(cx<double>), sz = (size_t)pl.N * pl.N * elem;
 	const int ns = dual ? 2 : 1;
 	const long nparts = cyc_parts(cp.L, cp.K);
 	const size_t lds = cyc_lds(cp.K, dual);
@@ -1385,7 +1400,7 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 				a.in[j][w] = l.in[j] < 0 ? static_cast<const void*>(dU) : S + (size_t)(l.in[j] * ns + w) * sz;
 				a.out[j][w] = l.out[j] < 0 ? nullptr : S + (size_t)(l.out[j] * ns + w) * sz;
 			}
-			bytes += amps * sizeof(cx<double>) * ((l.in[j] < 0 ? 1 : ns) + (l.out[j] < 0 ? 0 : ns));
+			bytes += amps * ((l.in[j] < 0 ? sizeof(zc) : ns * elem) + (l.out[j] < 0 ? 0 : ns * elem));
 			flops += amps * l.gate_sides[j] * side;
 		}
 		// algorithmic flops: a forward product in the direct complex form (the issued three-product
@@ -1393,7 +1408,7 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 		// outer products of a gate)
 		LaunchTimer lt(s, l.reverse ? RQC_KERNEL_REVERSE : RQC_KERNEL_FORWARD, bytes, l.reverse ? flops : flops * (4.0 / 3.0),
 			flops);
-		const CycKernel kf = cyc_kernel(cp.K, dual, l.out[0] >= 0);
+		const CycKernel kf = cyc_kernel(cp.K, dual, pl.fp32, l.out[0] >= 0);
 		kf<<<dim3(pl.tp->cyc_grid[i], l.njobs), cyc_nthreads(cp.K, dual), lds, s.stream>>>(a, mats, d_partial, nparts, d_partial, skip);
 	}
 	LaunchTimer lt(s, RQC_KERNEL_OTHER);

@@ -111,6 +111,7 @@ struct DeviceTableDesc
 	int* bad = nullptr;             // set to 1 when a gate is singular
 	size_t mats_bytes = 0, terms_bytes = 0, rmats_off = 0;
 	int G = 0, ng = 0, mode = 0, fp32 = 0;
+	int round_gates = 0;            // FP64 matrices of the gates rounded to complex float (mixed cyclic sweeps)
 };
 // group of every execution slot of a tile-pass plan
 std::vector<int> table_slot_groups(const EvalPlan& pl);

@@ -82,3 +82,24 @@ def test_brickwalls_match_the_column_sweeps(L, depth):
     assert reldiff(ft, a[0]) < TOL
     for x, y in zip(a, c):
         assert reldiff(x, y) < TOL
+
+
+@pytest.mark.parametrize("L,ngates", [(5, 3), (6, 17), (9, 12), (10, 31), (11, 20)])
+def test_mixed_precision_rounds_between_launches_only(L, ngates):
+    """Mixed precision keeps the arrays between launches in complex FP32 and multiplies in FP64: an
+    entry is rounded (2^-24 relative) once per launch, at most about 20 times, so gradients and HVPs
+    stay within 2e-6 of FP64 (20 roundings of one sign: 1.2e-6), f within that of sqrt(N)."""
+    print("qubits", L, "gates", ngates, flush=True)
+    rng = np.random.default_rng(31 * L + ngates)
+    g = np.stack([haar_unitary(rng) for _ in range(ngates)])
+    z = crandn(rng, (ngates, 4, 4))
+    w = np.array([rng.choice(L, 2, replace=False) for _ in range(ngates)], dtype=np.int32)
+    U = np.linalg.qr(crandn(rng, (1 << L, 1 << L)))[0]
+    T = R.DeviceTarget.dense(U)
+    a = _all(T, g, z, w, L)
+    R.set_precision(R.PRECISION_MIXED)
+    m = _all(T, g, z, w, L)
+    assert R.last_sweep()[0] == R.ENGINE_TILE_PASS
+    for f in (m[0], m[1][0], m[2][0]):
+        assert abs(f - a[0]) < 2e-6 * 2 ** (L / 2)
+    assert reldiff(m[1][1], a[1][1]) < 2e-6 and reldiff(m[2][1], a[2][1]) < 2e-6 and reldiff(m[2][2], a[2][2]) < 2e-6
