@@ -41,6 +41,14 @@ template <int K, bool DUAL> constexpr int cyc_lds_bytes()
 	return cyc_state_bytes<K, DUAL>() + kCycOps * cyc_mats_per_op(DUAL) * 256;
 }
 
+// the pointer's counterpart in copy i of its region
+template <typename P>
+__device__ __forceinline__ P* copy_of(P* p, long stride, int i)
+{
+	typedef typename std::conditional<std::is_const<P>::value, const char, char>::type byte;
+	return reinterpret_cast<P*>(reinterpret_cast<byte*>(p) + stride * i);
+}
+
 // XOR of the terms selected by the bits of x (masks, so that the terms' loads are unconditional)
 template <typename T>
 __device__ __forceinline__ T cyc_select(const T* terms, int n, long x)
@@ -61,9 +69,13 @@ __device__ __forceinline__ long lane_value(long v, int l)
 // the next tile's loads alone, not for the stores issued after them (one counter, in order).
 template <int K, bool DUAL, typename TS, bool OUT, int LW = 2 * (K - 4)>
 __global__ __launch_bounds__(64 << LW, LW >= 2 * (K - 4) ? 4 : 2) void k_cyc_sweep(const CycArgs A, const cx<double>* __restrict__ mats,
-	zc* __restrict__ part, long nparts, zc* __restrict__ trace, const int* skip)
+	zc* __restrict__ part, long nparts, zc* __restrict__ trace, long stride, const int* skip)
 {
 	if (skipped(skip)) { return; }
+	// evaluation blockIdx.z of several of one plan, `stride` bytes apart (tables, parts and arrays; U shared)
+	mats = copy_of(mats, stride, blockIdx.z);
+	part = copy_of(part, stride, blockIdx.z);
+	trace = copy_of(trace, stride, blockIdx.z);
 	extern __shared__ __align__(16) char lds_raw[];
 	constexpr int LT = 6 + LW, NT = 1 << LT, NW = NT / 64;
 	constexpr int LE = 2 * K - LT, NE = 1 << LE;   // elements per thread (the highest index bits)
@@ -77,12 +89,13 @@ __global__ __launch_bounds__(64 << LW, LW >= 2 * (K - 4) ? 4 : 2) void k_cyc_swe
 	if ((long)blockIdx.x >= ntiles) { return; }
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-	const vec2* in0 = static_cast<const vec2*>(A.in[blockIdx.y][0]);
-	const vec2* in1 = static_cast<const vec2*>(A.in[blockIdx.y][1]);
-	const lds_d2* inU = static_cast<const lds_d2*>(A.in[blockIdx.y][0]);
-	vec2* out0 = static_cast<vec2*>(A.out[blockIdx.y][0]);
-	vec2* out1 = static_cast<vec2*>(A.out[blockIdx.y][1]);
 	const int flags = J.flags;
+	const long in_stride = (flags & kCycReadU) ? 0 : stride;
+	const vec2* in0 = copy_of(static_cast<const vec2*>(A.in[blockIdx.y][0]), in_stride, blockIdx.z);
+	const vec2* in1 = copy_of(static_cast<const vec2*>(A.in[blockIdx.y][1]), in_stride, blockIdx.z);
+	const lds_d2* inU = static_cast<const lds_d2*>(A.in[blockIdx.y][0]);
+	vec2* out0 = copy_of(static_cast<vec2*>(A.out[blockIdx.y][0]), stride, blockIdx.z);
+	vec2* out1 = copy_of(static_cast<vec2*>(A.out[blockIdx.y][1]), stride, blockIdx.z);
 
 	// the gate matrices of the products: left factors transposed, right ones as they are, so that
 	// a lane's operand entry is at 4 (lane >> 4) + (lane & 3) in both
@@ -323,9 +336,12 @@ __global__ __launch_bounds__(64 << LW, LW >= 2 * (K - 4) ? 4 : 2) void k_cyc_swe
 // order: circuit gate of the slot and its side.  Slot 0 writes f = -Tr M.
 template <bool DUAL>
 __global__ __launch_bounds__(256) void k_cyc_reduce(const zc* __restrict__ part, long nparts, const int* __restrict__ order,
-	const zc* __restrict__ rmats, zc* __restrict__ acc, const int* skip)
+	const zc* __restrict__ rmats, zc* __restrict__ acc, long stride, const int* skip)
 {
 	if (skipped(skip)) { return; }
+	part = copy_of(part, stride, blockIdx.y);
+	rmats = copy_of(rmats, stride, blockIdx.y);
+	acc = copy_of(acc, stride, blockIdx.y);
 	constexpr int NE = DUAL ? 32 : 16, NS = 256 / NE;
 	__shared__ zc red[NS][NE];
 	const int x = blockIdx.x, e = threadIdx.x & (NE - 1), p0 = threadIdx.x / NE;
@@ -364,6 +380,40 @@ __global__ __launch_bounds__(256) void k_cyc_reduce(const zc* __restrict__ part,
 			}
 		}
 		acc[1 + 32L * order[2 * x] + 16 * h + 4 * c + r] = zc{-v.x, -v.y};
+	}
+}
+
+// Tables of the HVPs along the unit directions E_rc on every gate of one group (the columns of a
+// Hessian): column c0 + blockIdx.y (group (c0 + y) / 16, entry (c0 + y) mod 16), at tab + y stride
+// bytes, from the table of the circuit without directions.  One thread per 4x4 entry of a slot:
+// Z = E_rc, W = -G^-1 E_rc G^-1 = -(column r of G^-1) (row c of it), zero for the other groups' gates.
+__global__ __launch_bounds__(kBlock) void k_cyc_unit_tables(const char* __restrict__ base, char* __restrict__ tab, long stride,
+	long bytes, long rmats_off, long order_off, int G, int per, int c0)
+{
+	char* t = tab + stride * blockIdx.y;
+	const long first = (long)blockIdx.x * kBlock + threadIdx.x, step = (long)gridDim.x * kBlock;
+	const int col = c0 + blockIdx.y, group = col >> 4, r = (col >> 2) & 3, c = col & 3;
+	const int* order = reinterpret_cast<const int*>(base + order_off);
+	const zc* mats = reinterpret_cast<const zc*>(base);
+	const long nm = (long)G * kMats * 16, nr = (long)G * 32, r0 = rmats_off / (long)sizeof(zc);
+	for (long i = first; i < bytes / (long)sizeof(zc); i += step) {
+		zc v = reinterpret_cast<const zc*>(base)[i];
+		const bool in_m = i < nm, in_r = i >= r0 && i < r0 + nr;
+		if (in_m || in_r) {
+			const long k = in_m ? i : i - r0;
+			const int x = (int)(in_m ? k / (16 * kMats) : k / 32), w = (int)((k >> 4) % (in_m ? kMats : 2)), e = (int)(k & 15);
+			if (order[2 * x] / per == group) {
+				const zc* gi = mats + ((long)x * kMats + kMatGinv) * 16;
+				const int a = e >> 2, b = e & 3;
+				auto wm = [&](int i2, int j2) { return -(gi[4 * i2 + r] * gi[4 * c + j2]); };
+				const zc one = {1, 0}, zero = {0, 0};
+				if (in_r) { if (w == 1) { v = wm(b, a); } }
+				else if (w == kMatZ) { v = (a == r && b == c) ? one : zero; }
+				else if (w == kMatZT) { v = (b == r && a == c) ? one : zero; }
+				else if (w == kMatW) { v = wm(a, b); }
+			}
+		}
+		reinterpret_cast<zc*>(t)[i] = v;
 	}
 }
 

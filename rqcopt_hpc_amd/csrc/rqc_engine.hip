@@ -894,7 +894,7 @@ static std::shared_ptr<TilePlan> plan_tiles(const Context& dev, const Circuit& C
 }
 
 // ---------------------------------------------------------------- cyclic-product sweeps
-typedef void (*CycKernel)(const CycArgs, const cx<double>*, zc*, long, zc*, const int*);
+typedef void (*CycKernel)(const CycArgs, const cx<double>*, zc*, long, zc*, long, const int*);
 
 // Waves of a workgroup (log2): 16 for the 64 x 64 tiles of dual sweeps (one workgroup per CU, four
 // waves per SIMD: L = 14, depth 9 HVP 64.5 ms against 66.6 with 8), 8 for those of plain sweeps (64 KiB
@@ -926,8 +926,9 @@ static size_t cyc_lds(int K, bool dual)
 
 // Tile qubits: 64 x 64 tiles fuse most gates per pass (L = 12, depth 7 HVP 2.40 ms, 32 x 32 tiles
 // 3.21 ms); below 10 qubits they leave most CUs idle (L = 8, depth 7: 16 tiles, 220 us against 64
-// tiles, 179 us; L = 9 gradient 134 us against 109 us; equal at 10 qubits).
-static int cyc_tile_qubits(int L) { return L >= 10 ? 6 : 5; }
+// tiles, 179 us; L = 9 gradient 134 us against 109 us; equal at 10 qubits), unless several
+// evaluations share a launch.
+static int cyc_tile_qubits(int L, int copies) { return (L >= 10 || (L >= 6 && copies >= 1 << (20 - 2 * L))) ? 6 : 5; }
 
 static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const Circuit& C, bool dual, bool fp32, bool target_only, int K)
 {
@@ -978,7 +979,7 @@ static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circui
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, bool fp32, bool project, bool unitary,
-	size_t budget, size_t held, const TileChoice* choice, long ncols)
+	size_t budget, size_t held, const TileChoice* choice, long ncols, int copies)
 {
 	const int logE_c = (choice != nullptr) ? choice->logE : 0;
 	const int gmax = (choice != nullptr && choice->gmax > 0) ? std::min(choice->gmax, (int)kMaxTileGates) : tile_gmax();
@@ -1005,7 +1006,7 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	std::vector<Pass> passes;
 	// cyclic-product sweeps: the whole trace of a dense target, when its arrays fit
 	if (tiles && !pl.sampled && C.L >= 5 && 2 * (C.L - 6) <= kCycGens) {
-		const int K = cyc_tile_qubits(C.L);
+		const int K = cyc_tile_qubits(C.L, copies);
 		const bool dual = (mode == Mode::Hvp);
 		auto tp = plan_cyc(dev, C, dual, fp32, mode == Mode::Target, K);
 		const int nst = tp->cyc.nbuf * (dual ? 2 : 1);
@@ -1376,7 +1377,7 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 
 // cyclic-product sweeps of a dense target (rqc_cyc_plan.hpp)
 static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_partial, const char* tab, char* S,
-	const int* skip)
+	const int* skip, const EvalCopies& cps)
 {
 	const CycPlan& cp = pl.tp->cyc;
 	const bool dual = (pl.mode == Mode::Hvp);
@@ -1406,18 +1407,21 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 		// algorithmic flops: a forward product in the direct complex form (the issued three-product
 		// form is 3/4 of it); a conjugation by what it issues (it replaces the adjoint update and the
 		// outer products of a gate)
+		bytes *= cps.n;
+		flops *= cps.n;
 		LaunchTimer lt(s, l.reverse ? RQC_KERNEL_REVERSE : RQC_KERNEL_FORWARD, bytes, l.reverse ? flops : flops * (4.0 / 3.0),
 			flops);
 		const CycKernel kf = cyc_kernel(cp.K, dual, pl.fp32, l.out[0] >= 0);
-		kf<<<dim3(pl.tp->cyc_grid[i], l.njobs), cyc_nthreads(cp.K, dual), lds, s.stream>>>(a, mats, d_partial, nparts, d_partial, skip);
+		kf<<<dim3(pl.tp->cyc_grid[i], l.njobs, cps.n), cyc_nthreads(cp.K, dual), lds, s.stream>>>(a, mats, d_partial, nparts,
+			d_partial, cps.stride, skip);
 	}
 	LaunchTimer lt(s, RQC_KERNEL_OTHER);
 	if (pl.mode == Mode::Target) {
 		k_cyc_trace<<<1, kBlock, 0, s.stream>>>(d_partial, cp.ntrace * (cyc_nthreads(cp.K, false) / 64), d_acc, skip);
 	} else if (dual) {
-		k_cyc_reduce<true><<<pl.G, 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, skip);
+		k_cyc_reduce<true><<<dim3(pl.G, cps.n), 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, cps.stride, skip);
 	} else {
-		k_cyc_reduce<false><<<pl.G, 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, skip);
+		k_cyc_reduce<false><<<dim3(pl.G, cps.n), 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, cps.stride, skip);
 	}
 }
 
@@ -1436,9 +1440,11 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 // real part).  Every gate of a group is the group's gate vlist[l].
 __global__ __launch_bounds__(kBlock) void k_finalize(const zc* __restrict__ acc, int ngroups, int per,
 	const zc* __restrict__ vlist, const zc* __restrict__ vdirs, zc* __restrict__ res, int want_grad, int project, int want_hvp,
-	int fcorr, const int* skip)
+	int fcorr, long stride, long res_stride, const int* skip)
 {
 	if (skipped(skip)) { return; }
+	acc = copy_of(acc, stride, blockIdx.y);
+	res = copy_of(res, res_stride, blockIdx.y);
 	const int l = blockIdx.x, t = threadIdx.x;
 	// entry e of group g's sums (e < 16: gradient, else HVP), over its gates in order
 	auto group_sum = [&](int g, int e) {
@@ -1517,9 +1523,11 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const zc* __restrict__ acc,
 }
 
 void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit& C, const zc* dU, char* work,
-	char* tab, char* res_dev, const char* host_tab, const int* skip, const void* X, const zc* W, const BlockEnc* be)
+	char* tab, char* res_dev, const char* host_tab, const int* skip, const void* X, const zc* W, const BlockEnc* be,
+	const EvalCopies& cps)
 {
 	(void)dev;
+	if (cps.n != 1 && !pl.cyc) { throw Error(-3, "several evaluations per launch need a cyclic-product plan"); }
 	if (skip != nullptr && !pl.tiles) { throw Error(-3, "skip flags need the tile-pass engine"); }
 	if (pl.sampled && (X == nullptr || (W == nullptr && be == nullptr))) {
 		throw Error(-3, "a sampled evaluation needs its sample and seed blocks");
@@ -1547,7 +1555,7 @@ void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit
 	}
 	const GateTerms* gterms = reinterpret_cast<const GateTerms*>(tab + pl.mats_bytes);
 	if (pl.cyc) {
-		run_cyc(s, pl, dU, acc, part, tab, work + pl.off_states, skip);
+		run_cyc(s, pl, dU, acc, part, tab, work + pl.off_states, skip, cps);
 	} else if (pl.fp32) {
 		cx<float>* S = reinterpret_cast<cx<float>*>(work + pl.off_states);
 		const cx<float>* Xs = static_cast<const cx<float>*>(X);
@@ -1560,9 +1568,9 @@ void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit
 		else { run_gates<double>(s, pl, C, dU, acc, part, S, skip, Xs, W, be); }
 	}
 	LaunchTimer lt(s, RQC_KERNEL_OTHER);
-	k_finalize<<<pl.mode != Mode::Target ? pl.ng : 1, kBlock, 0, s.stream>>>(acc, pl.ng, pl.per, vin, vin + 16 * (size_t)pl.ng, res,
+	k_finalize<<<dim3(pl.mode != Mode::Target ? pl.ng : 1, cps.n), kBlock, 0, s.stream>>>(acc, pl.ng, pl.per, vin, vin + 16 * (size_t)pl.ng, res,
 		pl.mode != Mode::Target ? 1 : 0, pl.project ? 1 : 0, pl.mode == Mode::Hvp ? 1 : 0,
-		pl.fp32 ? (be != nullptr ? 2 : 1) : 0, skip);
+		pl.fp32 ? (be != nullptr ? 2 : 1) : 0, cps.stride, cps.res_stride, skip);
 }
 
 void unpack_result(const EvalPlan& pl, const char* res, EvalResult& R)
@@ -3049,6 +3057,46 @@ static EvalResult eval_blockenc(const Circuit& C, linear_func hfunc, void* hdata
 	return R;
 }
 
+// HVP columns of a Hessian on a cyclic-product plan: several evaluations per launch, their tables expanded on the GPU from one.  48 columns of 8 qubits and 3 layers as 48
+// evaluations took 2.55 ms, launch after launch of 64 small tiles; together 0.33 ms (both with the
+// host side).
+static void hessian_columns(Context& c, const EvalPlan& pl, const Circuit& C, const zc* dU, int m, char* hres, size_t rs)
+{
+	const size_t stride = align256(pl.bytes), res_off = align256(pl.tab_bytes), base = res_off + (size_t)m * rs;
+	// enough tiles to fill the device 16 times over and no more (2 GiB of arrays in FP64)
+	const long tiles = 1L << (2 * (pl.L - pl.tile_K));
+	int chunk = (int)std::max<long>(1, std::min<long>(m, 4096 / tiles));
+	if (base + (size_t)chunk * stride > c.work.bytes) {
+		size_t room = c.ws_limit;
+		if (room == 0) {
+			size_t fr = 0, tot = 0;
+			RQC_HIP(hipMemGetInfo(&fr, &tot));
+			room = (size_t)(0.85 * (double)(fr + c.work.bytes));
+		}
+		chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)chunk, room > base ? (room - base) / stride : 1));
+	}
+	c.work.reserve(base + (size_t)chunk * stride);
+	char* work = c.work.as<char>();
+	std::vector<char> tab(pl.tab_bytes);
+	fill_eval_tables(pl, C, tab.data());
+	RQC_HIP(hipMemcpyAsync(work, tab.data(), pl.tab_bytes, hipMemcpyHostToDevice, c.stream));
+	for (int c0 = 0; c0 < m; c0 += chunk) {
+		const int n = std::min(chunk, m - c0);
+		char* w = work + base;
+		{
+			LaunchTimer lt(c, RQC_KERNEL_OTHER);
+			const unsigned g = (unsigned)std::min<size_t>(64, (pl.tab_bytes / sizeof(zc) + kBlock - 1) / kBlock);
+			k_cyc_unit_tables<<<dim3(g, n), kBlock, 0, c.stream>>>(work, w + pl.off_tab, (long)stride, (long)pl.tab_bytes,
+				(long)pl.rmats_off, (long)pl.mats_bytes, pl.G, pl.per, c0);
+		}
+		enqueue_eval(c, c, pl, C, dU, w, nullptr, work + res_off + (size_t)c0 * rs, nullptr, nullptr, nullptr, nullptr, nullptr,
+			EvalCopies{n, (long)stride, (long)rs});
+	}
+	RQC_HIP(hipMemcpyAsync(hres, work + res_off, (size_t)m * rs, hipMemcpyDeviceToHost, c.stream));
+	RQC_HIP(hipStreamSynchronize(c.stream));
+	RQC_HIP(hipGetLastError());
+}
+
 // Complex Hessian of the brickwall target (reference src/target.c:687-797).  Column
 // (j, y) is the HVP with the unit direction E_y on every gate of layer j, so the
 // 16 nlayers columns are HVP evaluations of one plan: their tables go up in one
@@ -3067,7 +3115,7 @@ static void eval_hessian(const Circuit& C0, linear_func ufunc, void* udata, int 
 	const bool blockenc = (hess2 != nullptr);
 	const bool unitary = gates_near_unitary(C);
 	const EvalPlan pl = plan_eval(c, C, Mode::Hvp, per, c.precision == RQC_PRECISION_MIXED, false, unitary, c.ws_limit,
-		c.work.bytes, nullptr, blockenc ? (1L << (C.L / 2)) : nsamples);
+		c.work.bytes, nullptr, blockenc ? (1L << (C.L / 2)) : nsamples, m);
 	const zc* dU = nullptr;
 	SampleBlocks sb;
 	BlockEncInputs bi;
@@ -3081,39 +3129,44 @@ static void eval_hessian(const Circuit& C0, linear_func ufunc, void* udata, int 
 		dU = resolve_target(c, ufunc, udata, C0.L);
 	}
 	const double scale = (pl.sampled && !blockenc) ? (double)pl.N / (double)nsamples : 1.0;
-	const size_t ts = align256(pl.tab_bytes), rs = align256(pl.res_bytes()), base = align256(pl.bytes);
-	std::vector<char> htab((size_t)m * ts);
-	std::vector<Circuit> cols((size_t)m, C);
-	for (int col = 0; col < m; col++) {
-		Circuit& Cc = cols[col];
-		const int jl = col / 16, y = col % 16;
-		for (int q = 0; q < per; q++) { Cc.dirs[16 * ((size_t)jl * per + q) + y] = zc{1, 0}; }
-		fill_eval_tables(pl, Cc, htab.data() + (size_t)col * ts);
-	}
-	const size_t gbytes = blockenc ? (size_t)m * m * sizeof(zc) : 0;
-	c.work.reserve(base + (size_t)m * (ts + rs) + gbytes);
-	char* work = c.work.as<char>();
-	char* tabs = work + base;
-	char* ress = tabs + (size_t)m * ts;
-	RQC_HIP(hipMemcpyAsync(tabs, htab.data(), htab.size(), hipMemcpyHostToDevice, c.stream));
-	for (int col = 0; col < m; col++) {
-		const BlockEnc be{bi.H, blockenc ? bi.J + (size_t)col * pl.N : nullptr};
-		enqueue_eval(c, c, pl, cols[col], dU, work, tabs + (size_t)col * ts, ress + (size_t)col * rs, nullptr, nullptr,
-			sb.X, sb.W, blockenc ? &be : nullptr);
-	}
+	const size_t rs = align256(pl.res_bytes());
 	std::vector<char> hres((size_t)m * rs);
-	RQC_HIP(hipMemcpyAsync(hres.data(), ress, hres.size(), hipMemcpyDeviceToHost, c.stream));
-	if (blockenc) {
-		// hess2: Gram matrix of the projected Jacobian columns P^dagger dW P e_b of the m unit directions
-		zc* gram = reinterpret_cast<zc*>(ress + (size_t)m * rs);
-		{
-			LaunchTimer lt(c, RQC_KERNEL_OTHER);
-			k_gram_hermitian<<<dim3(m, m), kBlock, 0, c.stream>>>(bi.J, pl.N, m, gram);
+	if (pl.cyc) {
+		hessian_columns(c, pl, C, dU, m, hres.data(), rs);
+	} else {
+		const size_t ts = align256(pl.tab_bytes), base = align256(pl.bytes);
+		std::vector<char> htab((size_t)m * ts);
+		std::vector<Circuit> cols((size_t)m, C);
+		for (int col = 0; col < m; col++) {
+			Circuit& Cc = cols[col];
+			const int jl = col / 16, y = col % 16;
+			for (int q = 0; q < per; q++) { Cc.dirs[16 * ((size_t)jl * per + q) + y] = zc{1, 0}; }
+			fill_eval_tables(pl, Cc, htab.data() + (size_t)col * ts);
 		}
-		RQC_HIP(hipMemcpyAsync(hess2, gram, gbytes, hipMemcpyDeviceToHost, c.stream));
+		const size_t gbytes = blockenc ? (size_t)m * m * sizeof(zc) : 0;
+		c.work.reserve(base + (size_t)m * (ts + rs) + gbytes);
+		char* work = c.work.as<char>();
+		char* tabs = work + base;
+		char* ress = tabs + (size_t)m * ts;
+		RQC_HIP(hipMemcpyAsync(tabs, htab.data(), htab.size(), hipMemcpyHostToDevice, c.stream));
+		for (int col = 0; col < m; col++) {
+			const BlockEnc be{bi.H, blockenc ? bi.J + (size_t)col * pl.N : nullptr};
+			enqueue_eval(c, c, pl, cols[col], dU, work, tabs + (size_t)col * ts, ress + (size_t)col * rs, nullptr, nullptr,
+				sb.X, sb.W, blockenc ? &be : nullptr);
+		}
+		RQC_HIP(hipMemcpyAsync(hres.data(), ress, hres.size(), hipMemcpyDeviceToHost, c.stream));
+		if (blockenc) {
+			// hess2: Gram matrix of the projected Jacobian columns P^dagger dW P e_b of the m unit directions
+			zc* gram = reinterpret_cast<zc*>(ress + (size_t)m * rs);
+			{
+				LaunchTimer lt(c, RQC_KERNEL_OTHER);
+				k_gram_hermitian<<<dim3(m, m), kBlock, 0, c.stream>>>(bi.J, pl.N, m, gram);
+			}
+			RQC_HIP(hipMemcpyAsync(hess2, gram, gbytes, hipMemcpyDeviceToHost, c.stream));
+		}
+		RQC_HIP(hipStreamSynchronize(c.stream));
+		RQC_HIP(hipGetLastError());
 	}
-	RQC_HIP(hipStreamSynchronize(c.stream));
-	RQC_HIP(hipGetLastError());
 	std::vector<zc> H((size_t)m * m);
 	for (int col = 0; col < m; col++) {
 		EvalResult R;

@@ -91,9 +91,10 @@ struct EvalPlan
 // reverse sweeps only then; see sweep_unitary); `budget`: bytes for the state arrays
 // (0 = automatic, 85% of the free device memory plus `held`); `ncols` > 0: the
 // sweep's columns are that many given states instead of the 2^L basis columns
-// (the column block is then at most the power of two covering them)
+// (the column block is then at most the power of two covering them); `copies`: evaluations of the
+// plan that will share launches (EvalCopies; it only sizes the tiles)
 EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, bool fp32, bool project, bool unitary,
-	size_t budget, size_t held, const TileChoice* choice = nullptr, long ncols = 0);
+	size_t budget, size_t held, const TileChoice* choice = nullptr, long ncols = 0, int copies = 1);
 // host image of the evaluation's table region (pl.tab_bytes bytes at `host`)
 void fill_eval_tables(const EvalPlan& pl, const Circuit& C, char* host);
 
@@ -129,6 +130,15 @@ struct BlockEnc
 	zc* J = nullptr;        // device, or NULL
 };
 
+// several evaluations of one cyclic-product plan in the same launches: copy i has its own
+// workspace (tables in it, filled before) i * stride bytes after the first, its results i *
+// res_stride bytes after the first's
+struct EvalCopies
+{
+	int n = 1;
+	long stride = 0, res_stride = 0;
+};
+
 // enqueue the evaluation on slot s into workspace `work` (pl.bytes).  The table
 // region is at `tab` and the result region at `res` (NULL: their places in the
 // workspace); the table image is uploaded first when host_tab is given.  With
@@ -139,7 +149,7 @@ struct BlockEnc
 // or, with `be`, the block-encoding residual in place of the trace (W unused).
 void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit& C, const zc* dU, char* work,
 	char* tab, char* res, const char* host_tab, const int* skip, const void* X = nullptr, const zc* W = nullptr,
-	const BlockEnc* be = nullptr);
+	const BlockEnc* be = nullptr, const EvalCopies& cps = EvalCopies());
 
 struct EvalResult
 {

@@ -23,6 +23,7 @@ def fp64():
     R.require_gpu()
     R.set_precision(R.PRECISION_FP64)
     yield
+    R.set_precision(R.PRECISION_FP64)
     R.set_sweep_engine(R.ENGINE_TILE_PASS)
     R.set_workspace_limit(0)
 
@@ -82,6 +83,25 @@ def test_brickwalls_match_the_column_sweeps(L, depth):
     assert reldiff(ft, a[0]) < TOL
     for x, y in zip(a, c):
         assert reldiff(x, y) < TOL
+
+
+@pytest.mark.parametrize("L,depth", [(6, 1), (6, 4), (8, 2), (10, 2)])
+def test_hessian_columns_together_match_single_products(L, depth):
+    """The Hessian's columns run as several evaluations per launch (all at once at 6 and 8 qubits, in
+    chunks of 16 at 10): each equals the HVP along its unit direction, which runs alone."""
+    print("qubits", L, "layers", depth, flush=True)
+    rng = np.random.default_rng(13 * L + depth)
+    V = np.stack([haar_unitary(rng) for _ in range(depth)])
+    P = brickwall_perms(L, depth)
+    T = R.DeviceTarget.brickwall(np.stack([haar_unitary(rng) for _ in range(3)]), brickwall_perms(L, 3))
+    f, dv, H = R.brickwall_unitary_target_gradient_hessian(T, V, P)
+    H = np.asarray(H).reshape(16 * depth, 16 * depth)
+    for col in sorted({0, 7, 16 * depth - 1, 8 * depth + 3}):
+        Z = np.zeros((depth, 4, 4), complex)
+        Z[col // 16, (col % 16) // 4, col % 4] = 1
+        f1, dv1, hz = R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+        assert reldiff(f, f1) < TOL and reldiff(dv, dv1) < TOL
+        assert np.max(np.abs(H[:, col] - hz.reshape(-1))) < TOL * np.max(np.abs(H))
 
 
 @pytest.mark.parametrize("L,ngates", [(5, 3), (6, 17), (9, 12), (10, 31), (11, 20)])
