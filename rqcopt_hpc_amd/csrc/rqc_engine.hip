@@ -1810,29 +1810,57 @@ static void launch_forward_dual(Context& c, const zc* G, const zc* Z, int i, int
 		to_gate<double>(Z), wires_of(i, j, L), 1, 0, nq, din == nullptr ? 1 : 0);
 }
 
-// reverse step of one FP64 gate on a single statevector; gradient (and HVP) summed into acc[0..32)
+// workgroups of a reverse step on a single statevector: one quad per thread while that leaves CUs
+// idle (an HVP's gate at 18 qubits: 256 workgroups 11.5 us; four quads per thread, 64 workgroups,
+// with six exchanges for each of the 64 sums took 24 us, and a reduction launch after each gate
+// 4.6 us and a gap)
+static unsigned state_grid(long nq) { return (unsigned)std::max(1L, std::min((nq + kBlock - 1) / kBlock, 512L)); }
+
+// reverse step of one FP64 gate on a single statevector; the workgroups' gradient (and HVP) sums
+// go to part (state_grid x kWidth entries)
 static void launch_reverse(Context& c, const zc* G, const zc* Z, int i, int j, int L, const zc* psi, const zc* dpsi,
-	const zc* phi, const zc* dphi, zc* phi_out, zc* dphi_out, bool dual, zc* acc, zc* part)
+	const zc* phi, const zc* dphi, zc* phi_out, zc* dphi_out, bool dual, zc* part)
 {
 	const long nq = (1L << L) / 4;
-	const unsigned g = reduce_grid(nq);
+	const unsigned g = state_grid(nq);
 	int flags = 0;
 	if (dpsi == nullptr) { flags |= 1; }
 	if (dphi == nullptr) { flags |= 2; }
 	if (phi_out == nullptr) { flags |= 4; }
-	{
-		LaunchTimer lt(c, RQC_KERNEL_REVERSE);
-		if (dual) {
-			k_gate_reverse<double, true><<<g, kBlock, 0, c.stream>>>(psi, dpsi, phi, dphi, phi_out, dphi_out,
-				to_gate<double>(G), to_gate<double>(Z), wires_of(i, j, L), 1, 0, nq, flags, part);
-		} else {
-			k_gate_reverse<double, false><<<g, kBlock, 0, c.stream>>>(psi, nullptr, phi, nullptr, phi_out, nullptr,
-				to_gate<double>(G), to_gate<double>(G), wires_of(i, j, L), 1, 0, nq, flags | 2, part);
-		}
+	LaunchTimer lt(c, RQC_KERNEL_REVERSE);
+	if (dual) {
+		k_gate_reverse<double, true><<<g, kBlock, 0, c.stream>>>(psi, dpsi, phi, dphi, phi_out, dphi_out,
+			to_gate<double>(G), to_gate<double>(Z), wires_of(i, j, L), 1, 0, nq, flags, part);
+	} else {
+		k_gate_reverse<double, false><<<g, kBlock, 0, c.stream>>>(psi, nullptr, phi, nullptr, phi_out, nullptr,
+			to_gate<double>(G), to_gate<double>(G), wires_of(i, j, L), 1, 0, nq, flags | 2, part);
 	}
-	LaunchTimer lt(c, RQC_KERNEL_OTHER);
-	k_reduce_partials<<<kWidth, kBlock, 0, c.stream>>>(part, (int)g, kWidth, acc, nullptr);
 }
+
+// sums of ngates gates on a single statevector: acc (kWidth entries per gate), then a part region
+// for launch_reverse per gate; one launch adds up all of them
+struct StateSums
+{
+	zc* acc;
+	zc* part;
+	unsigned grid;
+	int ngates;
+
+	StateSums(Context& c, int ngates_, int L) : grid(state_grid((1L << L) / 4)), ngates(ngates_)
+	{
+		const size_t n = (size_t)ngates * kWidth;
+		c.small.reserve(n * (1 + grid) * sizeof(zc));
+		acc = c.small.as<zc>();
+		part = acc + n;
+	}
+	zc* part_of(int k) const { return part + (size_t)k * grid * kWidth; }
+	void reduce(Context& c) const
+	{
+		if (ngates == 0) { return; }
+		LaunchTimer lt(c, RQC_KERNEL_OTHER);
+		k_reduce_gates<<<dim3(ngates, kWidth), kBlock, 0, c.stream>>>(part, (int)grid, acc);
+	}
+};
 
 static zc* small_acc(Context& c, size_t n_acc)
 {
@@ -2013,15 +2041,16 @@ extern "C" void apply_gate_backward(const struct mat4x4* gate, const int i, cons
 		Context& c = ctx();
 		std::lock_guard<std::recursive_mutex> lk(c.mu);
 		const size_t bytes = ((size_t)1 << L) * sizeof(zc);
-		zc* acc = small_acc(c, 32);
+		const StateSums sums(c, 1, L);
 		Staging s(c);
 		const int a = s.add(psi->data, bytes, true, false);
 		const int d = s.add(dpsi_out->data, bytes, true, false);
 		const int o = s.add(dpsi->data, bytes, false, true);
 		s.upload();
 		const zc* G = reinterpret_cast<const zc*>(gate->data);
-		launch_reverse(c, G, G, i, j, L, s.dev<zc>(a), nullptr, s.dev<zc>(d), nullptr, s.dev<zc>(o), nullptr, false, acc, acc + 32);
-		copy_out(c, dgate->data, acc, 16 * sizeof(zc));
+		launch_reverse(c, G, G, i, j, L, s.dev<zc>(a), nullptr, s.dev<zc>(d), nullptr, s.dev<zc>(o), nullptr, false, sums.part);
+		sums.reduce(c);
+		copy_out(c, dgate->data, sums.acc, 16 * sizeof(zc));
 		s.download();
 	} catch (const std::exception& e) { fatal("apply_gate_backward", e); }
 }
@@ -2253,8 +2282,8 @@ extern "C" int quantum_circuit_backward(const struct mat4x4 gates[], const int n
 		std::lock_guard<std::recursive_mutex> lk(c.mu);
 		const size_t bytes = ((size_t)1 << L) * sizeof(zc);
 		const size_t n = (size_t)1 << L;
-		zc* acc = small_acc(c, 32 * (size_t)ngates);
-		zc* part = acc + 32 * (size_t)ngates;
+		const StateSums sums(c, ngates, L);
+		zc* acc = sums.acc;
 		Staging s(c);
 		const int st = s.scratch(bytes * ngates);
 		const int d = s.add(dpsi_out->data, bytes, true, false);
@@ -2268,9 +2297,10 @@ extern "C" int quantum_circuit_backward(const struct mat4x4 gates[], const int n
 		for (int k = ngates - 1; k >= 0; k--) {
 			zc* nxt = (k == 0) ? s.dev<zc>(o) : buf[k % 2];
 			const zc* G = &C.gates[16 * (size_t)k];
-			launch_reverse(c, G, G, C.wi[k], C.wj[k], L, S + k * n, nullptr, cur, nullptr, nxt, nullptr, false, acc + 32 * (size_t)k, part);
+			launch_reverse(c, G, G, C.wi[k], C.wj[k], L, S + k * n, nullptr, cur, nullptr, nxt, nullptr, false, sums.part_of(k));
 			cur = nxt;
 		}
+		sums.reduce(c);
 		std::vector<zc> hacc(32 * (size_t)ngates);
 		RQC_HIP(hipMemcpyAsync(hacc.data(), acc, hacc.size() * sizeof(zc), hipMemcpyDeviceToHost, c.stream));
 		s.download();
@@ -2291,8 +2321,8 @@ extern "C" int quantum_circuit_gates_hessian_vector_product(const struct mat4x4 
 		std::lock_guard<std::recursive_mutex> lk(c.mu);
 		const size_t bytes = ((size_t)1 << L) * sizeof(zc);
 		const size_t n = (size_t)1 << L;
-		zc* acc = small_acc(c, 32 * (size_t)ngates);
-		zc* part = acc + 32 * (size_t)ngates;
+		const StateSums sums(c, ngates, L);
+		zc* acc = sums.acc;
 		Staging s(c);
 		const int a = s.add(psi->data, bytes, true, false);
 		const int f = s.add(phi->data, bytes, true, false);
@@ -2300,24 +2330,25 @@ extern "C" int quantum_circuit_gates_hessian_vector_product(const struct mat4x4 
 		const int o = s.add(psi_out->data, bytes, false, true);
 		s.upload();
 		zc* S = s.dev<zc>(st);
-		auto P = [&](int k) { return S + k * n; };               // psi_k, k = 0 .. G
-		auto D = [&](int k) { return S + (ngates + k) * n; };    // dpsi_k, k = 1 .. G
+		auto P = [&](int k) { return k == 0 ? s.dev<zc>(a) : S + k * n; };   // psi_k, k = 0 .. G
+		auto D = [&](int k) { return S + (ngates + k) * n; };                // dpsi_k, k = 1 .. G
 		zc* F[2] = {S + (2 * ngates + 1) * n, S + (2 * ngates + 2) * n};
 		zc* DF[2] = {S + (2 * ngates + 3) * n, S + (2 * ngates + 4) * n};
-		dcopy(c, P(0), s.dev<zc>(a), bytes);
 		for (int k = 0; k < ngates; k++) {
 			launch_forward_dual(c, &C.gates[16 * (size_t)k], &C.dirs[16 * (size_t)k], C.wi[k], C.wj[k], L, P(k), P(k + 1),
 				k > 0 ? D(k) : nullptr, D(k + 1));
 		}
-		dcopy(c, s.dev<zc>(o), P(ngates), bytes);
-		dcopy(c, F[0], s.dev<zc>(f), bytes);
+		const zc* phi_k = s.dev<zc>(f);
 		int cur = 0;
 		for (int k = ngates - 1; k >= 0; k--) {
 			launch_reverse(c, &C.gates[16 * (size_t)k], &C.dirs[16 * (size_t)k], C.wi[k], C.wj[k], L, P(k),
-				k > 0 ? D(k) : nullptr, F[cur], k < ngates - 1 ? DF[cur] : nullptr,
-				k > 0 ? F[1 - cur] : nullptr, k > 0 ? DF[1 - cur] : nullptr, true, acc + 32 * (size_t)k, part);
+				k > 0 ? D(k) : nullptr, phi_k, k < ngates - 1 ? DF[cur] : nullptr,
+				k > 0 ? F[1 - cur] : nullptr, k > 0 ? DF[1 - cur] : nullptr, true, sums.part_of(k));
 			cur = 1 - cur;
+			phi_k = F[cur];
 		}
+		sums.reduce(c);
+		dcopy(c, s.dev<zc>(o), P(ngates), bytes);   // last: psi and psi_out may be one array
 		std::vector<zc> hacc(32 * (size_t)ngates);
 		RQC_HIP(hipMemcpyAsync(hacc.data(), acc, hacc.size() * sizeof(zc), hipMemcpyDeviceToHost, c.stream));
 		s.download();
@@ -2398,14 +2429,14 @@ extern "C" int brickwall_unitary_backward_hessian(const struct mat4x4 vlist[], i
 		std::lock_guard<std::recursive_mutex> lk(c.mu);
 		const size_t n = (size_t)1 << L;
 		const size_t bytes = n * sizeof(zc);
-		// small: gradient accumulators (32 per gate), reverse partials, Hessian m x m
-		c.small.reserve((32 * (size_t)ng + 4096 * (size_t)kWidth + (size_t)m * m) * sizeof(zc));
-		zc* acc = c.small.as<zc>();
-		zc* part = acc + 32 * (size_t)ng;
-		zc* dh = part + 4096 * (size_t)kWidth;
+		// small: Hessian m x m after the gates' sums
+		const size_t nsum = (size_t)ng * kWidth * (1 + state_grid((1L << L) / 4));
+		c.small.reserve((nsum + (size_t)m * m) * sizeof(zc));
+		const StateSums sums(c, ng, L);
+		zc* acc = sums.acc;
+		zc* dh = acc + nsum;
 		{
 			LaunchTimer lt(c, RQC_KERNEL_OTHER);
-			k_fill_zero<<<nblocks(32L * ng), kBlock, 0, c.stream>>>(acc, 32L * ng, nullptr);
 			k_fill_zero<<<nblocks((long)m * m), kBlock, 0, c.stream>>>(dh, (long)m * m, nullptr);
 		}
 		Staging s(c);
@@ -2423,8 +2454,9 @@ extern "C" int brickwall_unitary_backward_hessian(const struct mat4x4 vlist[], i
 			zc* out = (k > 0) ? A + (size_t)(k - 1) * n : s.dev<zc>(o);
 			const zc* G = &C.gates[16 * (size_t)k];
 			launch_reverse(c, G, G, C.wi[k], C.wj[k], L, S + k * n, nullptr, A + (size_t)k * n, nullptr, out, nullptr, false,
-				acc + 32 * (size_t)k, part);
+				sums.part_of(k));
 		}
+		sums.reduce(c);
 		zc* T[2] = {s.dev<zc>(t0), s.dev<zc>(t1)};
 		for (int g = 0; g < ng; g++) {
 			const int i = g / per;
@@ -3057,9 +3089,9 @@ static EvalResult eval_blockenc(const Circuit& C, linear_func hfunc, void* hdata
 	return R;
 }
 
-// HVP columns of a Hessian on a cyclic-product plan: several evaluations per launch, their tables expanded on the GPU from one.  48 columns of 8 qubits and 3 layers as 48
-// evaluations took 2.55 ms, launch after launch of 64 small tiles; together 0.33 ms (both with the
-// host side).
+// HVP columns of a Hessian on a cyclic-product plan: several evaluations per launch, their tables
+// expanded on the GPU from one.  48 columns of 8 qubits and 3 layers as 48 evaluations took
+// 2.55 ms, launch after launch of 64 small tiles; together 0.33 ms (both with the host side).
 static void hessian_columns(Context& c, const EvalPlan& pl, const Circuit& C, const zc* dU, int m, char* hres, size_t rs)
 {
 	const size_t stride = align256(pl.bytes), res_off = align256(pl.tab_bytes), base = res_off + (size_t)m * rs;

@@ -132,28 +132,54 @@ __global__ __launch_bounds__(kBlock) void k_gate_forward(
 }
 
 // ---------------------------------------------------------------------------
-// block-wide fixed-order sum of NV complex FP64 values per thread; thread 0..NV-1
-// of the block end up holding... the results are written to out[0..NV)
+// Wave-wide sums of N values per lane (N a power of two, at most 64), in a fixed order: while more
+// than one value is left, a step adds the lanes of a pair with each keeping half of the values, so
+// that N values take N - 1 exchanges (and log2(64 / N) more for the lanes that then hold the same
+// value) instead of 6 N.  Returns the sum of value `wave_sum_index<N>(lane)`.
+template <int N, int S = 32>
+__device__ __forceinline__ double wave_sum(double (&v)[N])
+{
+	if constexpr (N > 1) {
+		double h[N / 2];
+		const bool up = (threadIdx.x & S) != 0;
+#pragma unroll
+		for (int i = 0; i < N / 2; i++) {
+			const double keep = up ? v[i + N / 2] : v[i], give = up ? v[i] : v[i + N / 2];
+			h[i] = keep + __shfl_xor(give, S, 64);
+		}
+		return wave_sum<N / 2, S / 2>(h);
+	} else {
+		double s = v[0];
+#pragma unroll
+		for (int o = S; o >= 1; o >>= 1) { s += __shfl_xor(s, o, 64); }
+		return s;
+	}
+}
+
+template <int N> __device__ __forceinline__ int wave_sum_index(int lane)
+{
+	constexpr int bits = (N == 64) ? 6 : (N == 32) ? 5 : (N == 8) ? 3 : 1;
+	static_assert((1 << bits) == N, "2, 8, 32 or 64 values");
+	return lane >> (6 - bits);
+}
+
+// block-wide fixed-order sum of NV complex FP64 values per thread; the results are written to
+// out[0 .. NV)
 template <int NV>
 __device__ __forceinline__ void block_sum_store(zc* v, zc* out)
 {
-	__shared__ double red[kBlock / 64][NV][2];
+	constexpr int N = 2 * NV;
+	__shared__ double red[kBlock / 64][N];
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	double d[N];
 #pragma unroll
-	for (int e = 0; e < NV; e++) {
-		double re = v[e].x, im = v[e].y;
-#pragma unroll
-		for (int s = 32; s >= 1; s >>= 1) {
-			re += __shfl_xor(re, s, 64);
-			im += __shfl_xor(im, s, 64);
-		}
-		if (lane == 0) { red[wave][e][0] = re; red[wave][e][1] = im; }
-	}
+	for (int e = 0; e < NV; e++) { d[2 * e] = v[e].x; d[2 * e + 1] = v[e].y; }
+	red[wave][wave_sum_index<N>(lane)] = wave_sum<N>(d);
 	__syncthreads();
-	if (threadIdx.x < NV) {
-		double re = 0, im = 0;
-		for (int k = 0; k < kBlock / 64; k++) { re += red[k][threadIdx.x][0]; im += red[k][threadIdx.x][1]; }
-		out[threadIdx.x] = {re, im};
+	if (threadIdx.x < N) {
+		double s = 0;
+		for (int k = 0; k < kBlock / 64; k++) { s += red[k][threadIdx.x]; }
+		reinterpret_cast<double*>(out)[threadIdx.x] = s;
 	}
 }
 
@@ -425,6 +451,21 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(const zc* __restrict
 	block_sum_store<1>(r, res);
 	__syncthreads();
 	if (threadIdx.x == 0) { acc[e] += res[0]; }
+}
+
+// out[x * kWidth + y] = sum over the parts p of partial[(x * nparts + p) * kWidth + y] in a fixed
+// order: the sums of gate x of a sweep over one statevector, all gates in one launch
+__global__ __launch_bounds__(kBlock) void k_reduce_gates(const zc* __restrict__ partial, int nparts, zc* __restrict__ out)
+{
+	const int e = blockIdx.y;
+	const zc* p = partial + (long)blockIdx.x * nparts * kWidth;
+	zc s = {0, 0};
+	for (int i = threadIdx.x; i < nparts; i += kBlock) { s += p[(long)i * kWidth + e]; }
+	zc r[1] = {s};
+	__shared__ zc res[1];
+	block_sum_store<1>(r, res);
+	__syncthreads();
+	if (threadIdx.x == 0) { out[(long)blockIdx.x * kWidth + e] = res[0]; }
 }
 
 // X[a * B + c] = (a == b0 + c)
