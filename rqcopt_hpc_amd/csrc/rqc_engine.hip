@@ -30,6 +30,7 @@
 #include "rqc_kernels.hpp"
 #include "rqc_tile_kernels.hpp"
 #include "rqc_cyc_kernels.hpp"
+#include "rqc_state_kernels.hpp"
 #include "mat4.hpp"
 #include "rqcopt/gate.h"
 #include "rqcopt/statevector.h"
@@ -1846,7 +1847,9 @@ struct StateSums
 	unsigned grid;
 	int ngates;
 
-	StateSums(Context& c, int ngates_, int L) : grid(state_grid((1L << L) / 4)), ngates(ngates_)
+	// parts_: workgroups per gate (0: those of launch_reverse)
+	StateSums(Context& c, int ngates_, int L, unsigned parts_ = 0)
+		: grid(parts_ != 0 ? parts_ : state_grid((1L << L) / 4)), ngates(ngates_)
 	{
 		const size_t n = (size_t)ngates * kWidth;
 		c.small.reserve(n * (1 + grid) * sizeof(zc));
@@ -1861,6 +1864,90 @@ struct StateSums
 		k_reduce_gates<<<dim3(ngates, kWidth), kBlock, 0, c.stream>>>(part, (int)grid, acc);
 	}
 };
+
+// Passes over a statevector: the pass's gates and its tile, which holds the gates' qubits and the two
+// lowest index bits (64 contiguous bytes)
+struct StatePass
+{
+	std::vector<int> gates;
+	StateTile tile;
+};
+
+static std::vector<StatePass> plan_state(const Circuit& C)
+{
+	const int L = C.L, K = std::min(L, kStateK);
+	// at most 64 gates are taken back from one kept state
+	std::vector<StatePass> plan;
+	for (const Pass& p : cached_passes(C, L <= K ? L : K - 2, 64)) {
+		StatePass sp;
+		sp.gates = p.gates;
+		unsigned m = 3;
+		for (int k : p.gates) { m |= (1u << (L - 1 - C.wi[k])) | (1u << (L - 1 - C.wj[k])); }
+		for (int b = 0; b < L && __builtin_popcount(m) < K; b++) { m |= 1u << b; }
+		std::memset(&sp.tile, 0, sizeof(sp.tile));
+		sp.tile.K = K;
+		sp.tile.L = L;
+		int n = 0;
+		for (int in = 1; in >= 0; in--) {
+			for (int b = 0; b < L; b++) {
+				if ((int)((m >> b) & 1) == in) { sp.tile.bit[n++] = b; }
+			}
+		}
+		plan.push_back(std::move(sp));
+	}
+	return plan;
+}
+
+// the HVP of a statevector in passes: psi_out, and every gate's sums into sums.part; S holds the
+// states between the passes and the tangents after them, then the adjoint and its tangent.  ops is
+// read by a copy on the stream.
+static void state_passes(Context& c, const Circuit& C, const std::vector<StatePass>& plan, const StateSums& sums, const zc* psi,
+	const zc* phi, zc* psi_out, zc* S, std::vector<StateOp>& ops, StateOp* dev_ops)
+{
+	const int L = C.L, P = (int)plan.size(), K = plan[0].tile.K;
+	const size_t n = (size_t)1 << L;
+	std::vector<int> first;
+	for (const StatePass& p : plan) {
+		int pos[32];
+		for (int t = 0; t < K; t++) { pos[p.tile.bit[t]] = t; }
+		first.push_back((int)ops.size());
+		for (int k : p.gates) {
+			StateOp o;
+			std::memcpy(o.g, &C.gates[16 * (size_t)k], sizeof(o.g));
+			std::memcpy(o.z, &C.dirs[16 * (size_t)k], sizeof(o.z));
+			if (m4_inverse(o.g, o.ginv) != 0) { throw Error(-4, "singular gate in the statevector passes"); }
+			zc t[16];
+			m4_mul(o.z, o.ginv, t);
+			m4_mul(o.ginv, t, o.w);
+			o.gate.pi = pos[L - 1 - C.wi[k]];
+			o.gate.pj = pos[L - 1 - C.wj[k]];
+			o.gate.index = k;
+			o.gate.first = ops.empty();
+			ops.push_back(o);
+		}
+	}
+	RQC_HIP(hipMemcpyAsync(dev_ops, ops.data(), ops.size() * sizeof(StateOp), hipMemcpyHostToDevice, c.stream));
+	const int nt = std::max(128, 1 << (K - 1));
+	const size_t lds_f = state_lds_bytes(false), lds_r = state_lds_bytes(true);
+	allow_lds(k_state_pass<false>, lds_f);
+	allow_lds(k_state_pass<true>, lds_r);
+	auto state = [&](int p) { return p == P ? psi_out : S + (p - 1) * n; };      // after p passes, p = 1 .. P
+	auto tangent = [&](int p) { return S + (P - 2 + p) * n; };
+	zc* ad = S + (2 * P - 1) * n;
+	zc* dad = ad + n;
+	const double sb = (double)n * sizeof(zc);
+	for (int p = 0; p < P; p++) {
+		LaunchTimer lt(c, RQC_KERNEL_FORWARD, (p > 0 ? 4 : 3) * sb);
+		k_state_pass<false><<<sums.grid, nt, lds_f, c.stream>>>(dev_ops + first[p], (int)plan[p].gates.size(), plan[p].tile,
+			p > 0 ? state(p) : psi, p > 0 ? tangent(p) : nullptr, nullptr, nullptr, state(p + 1), tangent(p + 1), nullptr);
+	}
+	for (int p = P - 1; p >= 0; p--) {
+		LaunchTimer lt(c, RQC_KERNEL_REVERSE, (3 + (p < P - 1) + 2 * (p > 0)) * sb);
+		k_state_pass<true><<<sums.grid, nt, lds_r, c.stream>>>(dev_ops + first[p], (int)plan[p].gates.size(), plan[p].tile,
+			state(p + 1), tangent(p + 1), p < P - 1 ? ad : phi, p < P - 1 ? dad : nullptr, p > 0 ? ad : nullptr,
+			p > 0 ? dad : nullptr, sums.part);
+	}
+}
 
 static zc* small_acc(Context& c, size_t n_acc)
 {
@@ -2321,34 +2408,42 @@ extern "C" int quantum_circuit_gates_hessian_vector_product(const struct mat4x4 
 		std::lock_guard<std::recursive_mutex> lk(c.mu);
 		const size_t bytes = ((size_t)1 << L) * sizeof(zc);
 		const size_t n = (size_t)1 << L;
-		const StateSums sums(c, ngates, L);
+		const bool passes = c.engine == RQC_ENGINE_TILE_PASS && ngates > 1 && L <= 30 && gates_near_unitary(C);
+		const std::vector<StatePass> plan = passes ? plan_state(C) : std::vector<StatePass>();
+		const StateSums sums(c, ngates, L, passes ? 1u << (L - plan[0].tile.K) : 0);
 		zc* acc = sums.acc;
 		Staging s(c);
 		const int a = s.add(psi->data, bytes, true, false);
 		const int f = s.add(phi->data, bytes, true, false);
-		const int st = s.scratch(bytes * (2 * (size_t)ngates + 5));
+		const int st = s.scratch(bytes * (passes ? 2 * plan.size() + 1 : 2 * (size_t)ngates + 5));
 		const int o = s.add(psi_out->data, bytes, false, true);
+		const int tab = s.scratch(passes ? ngates * sizeof(StateOp) : 0);
 		s.upload();
 		zc* S = s.dev<zc>(st);
-		auto P = [&](int k) { return k == 0 ? s.dev<zc>(a) : S + k * n; };   // psi_k, k = 0 .. G
-		auto D = [&](int k) { return S + (ngates + k) * n; };                // dpsi_k, k = 1 .. G
-		zc* F[2] = {S + (2 * ngates + 1) * n, S + (2 * ngates + 2) * n};
-		zc* DF[2] = {S + (2 * ngates + 3) * n, S + (2 * ngates + 4) * n};
-		for (int k = 0; k < ngates; k++) {
-			launch_forward_dual(c, &C.gates[16 * (size_t)k], &C.dirs[16 * (size_t)k], C.wi[k], C.wj[k], L, P(k), P(k + 1),
-				k > 0 ? D(k) : nullptr, D(k + 1));
-		}
-		const zc* phi_k = s.dev<zc>(f);
-		int cur = 0;
-		for (int k = ngates - 1; k >= 0; k--) {
-			launch_reverse(c, &C.gates[16 * (size_t)k], &C.dirs[16 * (size_t)k], C.wi[k], C.wj[k], L, P(k),
-				k > 0 ? D(k) : nullptr, phi_k, k < ngates - 1 ? DF[cur] : nullptr,
-				k > 0 ? F[1 - cur] : nullptr, k > 0 ? DF[1 - cur] : nullptr, true, sums.part_of(k));
-			cur = 1 - cur;
-			phi_k = F[cur];
+		std::vector<StateOp> ops;
+		if (passes) {
+			state_passes(c, C, plan, sums, s.dev<zc>(a), s.dev<zc>(f), s.dev<zc>(o), S, ops, s.dev<StateOp>(tab));
+		} else {
+			auto P = [&](int k) { return k == 0 ? s.dev<zc>(a) : S + k * n; };   // psi_k, k = 0 .. G
+			auto D = [&](int k) { return S + (ngates + k) * n; };                // dpsi_k, k = 1 .. G
+			zc* F[2] = {S + (2 * ngates + 1) * n, S + (2 * ngates + 2) * n};
+			zc* DF[2] = {S + (2 * ngates + 3) * n, S + (2 * ngates + 4) * n};
+			for (int k = 0; k < ngates; k++) {
+				launch_forward_dual(c, &C.gates[16 * (size_t)k], &C.dirs[16 * (size_t)k], C.wi[k], C.wj[k], L, P(k), P(k + 1),
+					k > 0 ? D(k) : nullptr, D(k + 1));
+			}
+			const zc* phi_k = s.dev<zc>(f);
+			int cur = 0;
+			for (int k = ngates - 1; k >= 0; k--) {
+				launch_reverse(c, &C.gates[16 * (size_t)k], &C.dirs[16 * (size_t)k], C.wi[k], C.wj[k], L, P(k),
+					k > 0 ? D(k) : nullptr, phi_k, k < ngates - 1 ? DF[cur] : nullptr,
+					k > 0 ? F[1 - cur] : nullptr, k > 0 ? DF[1 - cur] : nullptr, true, sums.part_of(k));
+				cur = 1 - cur;
+				phi_k = F[cur];
+			}
+			dcopy(c, s.dev<zc>(o), P(ngates), bytes);   // last: psi and psi_out may be one array
 		}
 		sums.reduce(c);
-		dcopy(c, s.dev<zc>(o), P(ngates), bytes);   // last: psi and psi_out may be one array
 		std::vector<zc> hacc(32 * (size_t)ngates);
 		RQC_HIP(hipMemcpyAsync(hacc.data(), acc, hacc.size() * sizeof(zc), hipMemcpyDeviceToHost, c.stream));
 		s.download();

@@ -136,23 +136,49 @@ __global__ __launch_bounds__(kBlock) void k_gate_forward(
 // than one value is left, a step adds the lanes of a pair with each keeping half of the values, so
 // that N values take N - 1 exchanges (and log2(64 / N) more for the lanes that then hold the same
 // value) instead of 6 N.  Returns the sum of value `wave_sum_index<N>(lane)`.
+// The exchanges stay in the vector unit: between halves of a wave and of 32 lanes a swap of two
+// registers' halves leaves both lanes' terms in place, inside 16 lanes they are DPP moves (lane ^ 8,
+// ^ 7, ^ 2, ^ 1: the partner's bit S differs and the four reach all 16 lanes).
+template <int S> __device__ __forceinline__ double lane_partner(double v)
+{
+	constexpr int ctrl = (S == 8) ? 0x128 : (S == 4) ? 0x141 : (S == 2) ? 0x4e : 0xb1;
+	const long b = __double_as_longlong(v);
+	const unsigned lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffff), ctrl, 0xf, 0xf, true),
+		hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), ctrl, 0xf, 0xf, true);
+	return __longlong_as_double((long)(((unsigned long)hi << 32) | lo));
+}
+
+// lanes with bit S clear: a's sum over the pair, the others: b's
+template <int S> __device__ __forceinline__ double pair_sum(double a, double b)
+{
+	if constexpr (S >= 16) {
+		const long x = __double_as_longlong(a), y = __double_as_longlong(b);
+		auto swap = [](unsigned p, unsigned q) {
+			if constexpr (S == 32) { return __builtin_amdgcn_permlane32_swap(p, q, false, false); }
+			else { return __builtin_amdgcn_permlane16_swap(p, q, false, false); }
+		};
+		const auto lo = swap((unsigned)x, (unsigned)y), hi = swap((unsigned)(x >> 32), (unsigned)(y >> 32));
+		return __longlong_as_double((long)(((unsigned long)hi[0] << 32) | lo[0])) +
+			__longlong_as_double((long)(((unsigned long)hi[1] << 32) | lo[1]));
+	} else {
+		const bool up = (threadIdx.x & S) != 0;
+		return (up ? b : a) + lane_partner<S>(up ? a : b);
+	}
+}
+
 template <int N, int S = 32>
 __device__ __forceinline__ double wave_sum(double (&v)[N])
 {
 	if constexpr (N > 1) {
 		double h[N / 2];
-		const bool up = (threadIdx.x & S) != 0;
 #pragma unroll
-		for (int i = 0; i < N / 2; i++) {
-			const double keep = up ? v[i + N / 2] : v[i], give = up ? v[i] : v[i + N / 2];
-			h[i] = keep + __shfl_xor(give, S, 64);
-		}
-		return wave_sum<N / 2, S / 2>(h);
+		for (int i = 0; i < N / 2; i++) { h[i] = pair_sum<S>(v[i], v[i + N / 2]); }
+		if constexpr (S > 1) { return wave_sum<N / 2, S / 2>(h); }
+		else { return h[0]; }
 	} else {
-		double s = v[0];
-#pragma unroll
-		for (int o = S; o >= 1; o >>= 1) { s += __shfl_xor(s, o, 64); }
-		return s;
+		double w[1] = {pair_sum<S>(v[0], v[0])};
+		if constexpr (S > 1) { return wave_sum<1, S / 2>(w); }
+		else { return w[0]; }
 	}
 }
 

@@ -1,0 +1,48 @@
+"""HVP of a statevector in passes over tiles (rqc_state_kernels.hpp) against the launches of one gate
+each, and against the oracle where it is small.
+
+2 qubits is less than a wave, 6 to 9 change the threads of a tile, 10 is one whole tile, 11 and more
+have several tiles and bits outside the gates' window; 64 gates fill a pass and 65 begin the next.
+Both paths round FP64 sums of at most 2^13 terms of norm-1 states over at most 130 gates: 130 gates
+times 16 products at 2^-53, 2.3e-13, in norm; within 1e-12.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+import rqcopt_hpc_amd as R
+from helpers import crandn, haar_unitary, reldiff
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+@pytest.fixture(autouse=True)
+def engine():
+    R.require_gpu()
+    yield
+    R.set_sweep_engine(R.ENGINE_TILE_PASS)
+
+
+@pytest.mark.parametrize("L,ngates", [(2, 1), (2, 5), (3, 4), (5, 64), (6, 9), (7, 65), (8, 30), (9, 130), (10, 17), (10, 65),
+                                      (11, 1), (11, 40), (12, 66), (13, 25)])
+def test_passes_match_gate_launches(L, ngates):
+    print("qubits", L, "gates", ngates, flush=True)
+    rng = np.random.default_rng(10 * L + ngates)
+    g = np.stack([haar_unitary(rng) for _ in range(ngates)])
+    z = crandn(rng, (ngates, 4, 4))
+    w = np.array([rng.choice(L, 2, replace=False) for _ in range(ngates)], dtype=np.int32)
+    psi, phi = (v / np.linalg.norm(v) for v in crandn(rng, (2, 1 << L)))
+    a = R.quantum_circuit_gates_hessian_vector_product(g, z, w, psi, phi)
+    R.set_sweep_engine(R.ENGINE_PER_GATE)
+    b = R.quantum_circuit_gates_hessian_vector_product(g, z, w, psi, phi)
+    for x, y in zip(a, b):
+        if np.max(np.abs(y)) > 0:
+            assert reldiff(x, y) < TOL
+        else:
+            assert np.max(np.abs(x)) == 0   # one gate: no second derivative
+    if L <= 6:
+        c = O.quantum_circuit_gates_hvp(g, z, w, psi, phi)
+        for x, y in zip(a, c):
+            assert reldiff(x, y) < TOL or np.max(np.abs(y)) == 0
