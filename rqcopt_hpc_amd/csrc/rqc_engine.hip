@@ -747,7 +747,11 @@ struct TilePlan
 	std::vector<Pass> passes;
 	std::vector<TileArgs> args;
 	std::vector<TileArgs> args_fwd;
-	std::vector<TileGates> gks;
+	// reverse passes whose partial sums are reduced together, highest first: the pass after which
+	// (the lowest), its first execution slot and the gates
+	struct Reduction { int pass, x0, ng; };
+	std::vector<Reduction> reductions;
+	int reduce_gates = 0;           // the most gates of one
 	std::vector<GateTerms> terms;   // per gate, in execution order
 	std::vector<GateTerms> terms_fwd;   // forward tiles' terms (when tsf differs from ts)
 	size_t fterms_off = 0;          // byte offset of the forward terms in the table's terms region
@@ -851,14 +855,10 @@ static std::shared_ptr<TilePlan> plan_tiles(const Context& dev, const Circuit& C
 		tp->args.push_back(make_tile_args(C, p, ts.K, ts.logC, ilog2_or_neg(pl.B >> ts.logC), x, (int)sizeof(cx<T>),
 			tp->terms.data()));
 		if (!own_fwd) { tp->args_fwd.push_back(tp->args.back()); }
-		TileGates tg;
-		std::memset(&tg, 0, sizeof(tg));
-		for (size_t j = 0; j < p.gates.size(); j++) {
-			tg.k[j] = p.gates[j];
-			tp->order.push_back(p.gates[j]);
+		for (int k : p.gates) {
+			tp->order.push_back(k);
 			x++;
 		}
-		tp->gks.push_back(tg);
 		maxng = std::max(maxng, (int)p.gates.size());
 	}
 	const int E = 1 << (ts.K + ts.logC);
@@ -890,7 +890,22 @@ static std::shared_ptr<TilePlan> plan_tiles(const Context& dev, const Circuit& C
 	RQC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_r, reinterpret_cast<const void*>(kr), kTileThreads, tp->lds_rev));
 	tp->gfwd = (unsigned)std::min<long>(tp->ntiles_fwd, (long)std::max(1, occ_f) * dev.cu_count);
 	tp->grev = (unsigned)std::max<long>(1, std::min<long>(ntiles, (long)std::max(1, occ_r) * dev.cu_count));
-	tp->partial_doubles = (pl.mode == Mode::Target) ? 0 : (size_t)tp->grev * kTileWaves * maxng * 256;
+	if (pl.mode != Mode::Target) {
+		// One reduction (two launches) for as many passes as 16 MiB of partial sums allow: few
+		// workgroups have few parts, and then the reductions' launches take as long as the passes
+		// (block encoding of 10 qubits, 7 layers, 32 workgroups, six reductions: 300 us, one: 245).
+		// The largest grids reduce after each pass.
+		const size_t nparts = (size_t)tp->grev * kTileWaves;
+		const int most = std::max(maxng, (int)std::min<size_t>(kReduceGates, 8192 / nparts));
+		for (int p = (int)passes.size() - 1; p >= 0; p--) {
+			const int ng = (int)passes[p].gates.size();
+			if (tp->reductions.empty() || tp->reductions.back().ng + ng > most) { tp->reductions.push_back({p, 0, 0}); }
+			TilePlan::Reduction& r = tp->reductions.back();
+			r = {p, tp->args[p].x0, r.ng + ng};
+			tp->reduce_gates = std::max(tp->reduce_gates, r.ng);
+		}
+		tp->partial_doubles = nparts * tp->reduce_gates * 256;
+	}
 	return tp;
 }
 
@@ -1069,7 +1084,7 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	} else if (pl.tiles) {
 		// outer-product partials, the chunk sums of the first reduction stage, then the trace
 		// partials of a first reverse pass that takes the target's trace
-		npart = std::max(npart, (pl.tp->partial_doubles + (size_t)kReduceChunks * kMaxTileGates * 256 + 1) / 2 +
+		npart = std::max(npart, (pl.tp->partial_doubles + (size_t)kReduceChunks * pl.tp->reduce_gates * 256 + 1) / 2 +
 			(size_t)pl.tp->grev * kTileWaves);
 	}
 	else { npart = std::max(npart, (size_t)pl.grev_pg * kWidth); }
@@ -1273,8 +1288,8 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 	auto* krs = rev_kernel<T>(dual, tp.ts.K + tp.ts.logC, true);
 	const GateTerms* fterms = reinterpret_cast<const GateTerms*>(reinterpret_cast<const char*>(gterms) + tp.fterms_off);
 	const zc* rmats = reinterpret_cast<const zc*>(reinterpret_cast<const char*>(mats) + pl.rmats_off);
-	double* mpart = reinterpret_cast<double*>(d_partial);   // grev * waves * ng * 256 doubles
-	double* cpart = mpart + tp.partial_doubles;             // chunk sums: kReduceChunks * ng * 256 doubles
+	double* mpart = reinterpret_cast<double*>(d_partial);   // grev * waves * gates * 256 doubles
+	double* cpart = mpart + tp.partial_doubles;             // chunk sums: kReduceChunks * gates * 256 doubles
 	zc* tpart = d_partial;                                  // trace partials (reused, sequential)
 	const unsigned gtr = pl.gtr;
 	const int logB = ilog2_or_neg(B);
@@ -1285,7 +1300,7 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 	// FP64), forms the seed -conj(U) in LDS and takes the trace on the way (no separate target
 	// pass over U, psi and the seed)
 	const bool fuse_trace = dual && be == nullptr && !pl.sampled && B == N && P >= 1;
-	double* ttr = cpart + (size_t)kReduceChunks * kMaxTileGates * 256;   // its per-wave trace partials
+	double* ttr = cpart + (size_t)kReduceChunks * tp.reduce_gates * 256;   // its per-wave trace partials
 	// and, with the planned tiles (one tile for both directions), it also runs the circuit's
 	// last forward pass on its tiles first: the circuit's output states never go through HBM
 	const int logEr = tp.ts.K + tp.ts.logC;
@@ -1329,6 +1344,8 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 		}
 		if (mode == Mode::Target) { continue; }
 		int cur = 0;
+		const long nparts = (long)tp.grev * kTileWaves;
+		auto red = tp.reductions.begin();   // the reduction that the pass belongs to
 		for (int p = P - 1; p >= 0; p--) {
 			int flags = 0;
 			if (p == P - 1) { flags |= 4; }
@@ -1356,20 +1373,22 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 				(seed_pass ? krs : kr)<<<tp.grev, kTileThreads, seed_pass ? tp.lds_rev_seed : tp.lds_rev, s.stream>>>(
 					with_fwd ? PS(p) : PS(p + 1), dual ? (with_fwd ? DPS(p) : DPS(p + 1)) : nullptr,
 					seed_pass ? reinterpret_cast<const cx<T>*>(seed) : phi[cur], dual ? dphi[cur] : nullptr, phi[1 - cur],
-					dual ? dphi[1 - cur] : nullptr, tp.args[p], mats, gterms, B, b0, ntiles, flags, mpart, ttr, skip);
+					dual ? dphi[1 - cur] : nullptr, tp.args[p], mats, gterms, B, b0, ntiles, flags,
+					mpart + (tp.args[p].x0 - red->x0) * nparts * 256, ttr, skip);
 			}
 			if (seed_pass) {
 				LaunchTimer lt(s, RQC_KERNEL_OTHER);
 				k_reduce_partials<<<1, kBlock, 0, s.stream>>>(reinterpret_cast<const zc*>(ttr),
 					(int)(tp.grev * kTileWaves), 1, d_acc, skip);
 			}
-			{
+			if (p == red->pass) {
 				LaunchTimer lt(s, RQC_KERNEL_OTHER);
-				const long nparts = (long)tp.grev * kTileWaves;
 				const int nch = (int)std::min<long>(kReduceChunks, nparts);
-				k_tile_reduce_chunks<<<dim3(ng, nch), 256, 0, s.stream>>>(mpart, nparts, ng, nch, cpart, skip);
-				k_tile_reduce<<<ng, 256, 0, s.stream>>>(cpart, nch, ng, tp.gks[p], rmats + 32L * tp.args[p].x0, dual ? 1 : 0,
-					d_acc, skip);
+				TileGates tg;
+				std::copy_n(tp.order.begin() + red->x0, red->ng, tg.k);
+				k_tile_reduce_chunks<<<dim3(red->ng, nch), 256, 0, s.stream>>>(mpart, nparts, nch, cpart, skip);
+				k_tile_reduce<<<red->ng, 256, 0, s.stream>>>(cpart, nch, tg, rmats + 32L * red->x0, dual ? 1 : 0, d_acc, skip);
+				++red;
 			}
 			cur = 1 - cur;
 		}

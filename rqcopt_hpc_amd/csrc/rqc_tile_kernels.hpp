@@ -1005,7 +1005,7 @@ __global__ __launch_bounds__(kTileThreads, (fwd_waves_per_simd<T, DUAL, LOGE>())
 // the seed -conj(U) is formed in LDS and the trace sum(-conj(U) psi) goes to
 // trace[2 (block * waves + wave)] (a separate instantiation, so that the other passes run
 // exactly the kernel without it: the extra loop code measured 8 % slower on every pass).
-// partial[((part * ng + j) * 256) + row * 16 + col], part = block * waves + wave:
+// partial[(j * parts + part) * 256 + row * 16 + col], part = block * waves + wave:
 // the 16 x 16 outer-product sums of gate j (rows: component 4 (2 s + p) + r of
 // the adjoint at the gate input, columns: that of the state before the gate).
 // Reverse-pass buffering.  Dual sweeps hold one buffer of the four tile states
@@ -1586,7 +1586,7 @@ __global__ __launch_bounds__(kTileThreads, (rev_waves_per_simd<T, DUAL>())) void
 #pragma unroll
 	for (int j = 0; j < kMaxTileGates; j++) {
 		if (j < P.ng) {
-			double* d = partial + (part * P.ng + j) * 256;
+			double* d = partial + (j * (long)gridDim.x * kTileWaves + part) * 256;
 			if constexpr (sizeof(T) == 8) {
 				// the four blocks' sums (lane bits 2, 3) into the 16 x 16 layout: A1 and A2 as
 				// the (re, re), (re, im) blocks of phi (x) psi and phi (x) dpsi, zeros elsewhere
@@ -1610,10 +1610,11 @@ __global__ __launch_bounds__(kTileThreads, (rev_waves_per_simd<T, DUAL>())) void
 	}
 }
 
-// gate indices of a pass for the reduction
+// gate indices of a reduction
+constexpr int kReduceGates = 128;
 struct TileGates
 {
-	int k[kMaxTileGates];
+	int k[kReduceGates];
 };
 
 // First stage of the partial-sum reduction: chunk c of nchunks sums the parts
@@ -1621,7 +1622,7 @@ struct TileGates
 // out has the partials' layout with nchunks parts.
 constexpr int kReduceChunks = 16;
 
-__global__ __launch_bounds__(256) void k_tile_reduce_chunks(const double* __restrict__ partial, long nparts, int ng,
+__global__ __launch_bounds__(256) void k_tile_reduce_chunks(const double* __restrict__ partial, long nparts,
 	int nchunks, double* __restrict__ out, const int* skip)
 {
 	if (skipped(skip)) { return; }
@@ -1629,13 +1630,13 @@ __global__ __launch_bounds__(256) void k_tile_reduce_chunks(const double* __rest
 	const long per = (nparts + nchunks - 1) / nchunks;
 	const long p0 = (long)c * per, p1 = min(nparts, p0 + per);
 	double s = 0;
-	for (long p = p0; p < p1; p++) { s += partial[(p * ng + j) * 256 + i]; }
-	out[((long)c * ng + j) * 256 + i] = s;
+	for (long p = p0; p < p1; p++) { s += partial[(j * nparts + p) * 256 + i]; }
+	out[((long)j * nchunks + c) * 256 + i] = s;
 }
 
 // Sum of the outer-product partials over all parts in a fixed order, decoded
 // into 16 gradient and (DUAL) 16 HVP entries per gate and added to
-// acc[1 + 32 * gate + e].  One workgroup of 256 threads per gate of the pass.
+// acc[1 + 32 * gate + e].  One workgroup of 256 threads per gate of the reduction.
 // The partials pair the adjoint at the gate input (phi_in = G^T phi,
 // dphi_in = G^T dphi + Z^T phi) with the state before the gate; component
 // 4 (2 s + p) + r is array s (primary / tangent; plain sweeps: the quad of the
@@ -1643,8 +1644,8 @@ __global__ __launch_bounds__(256) void k_tile_reduce_chunks(const double* __rest
 // A2 = sum phi_in (x) dpsi, A3 = sum dphi_in (x) psi and Q = G^-T, the gate's
 // sums over the adjoint at its output are
 //   grad = Q A1,   hess = Q (A2 + A3) + W^T A1   (W = -G^-1 Z G^-1);
-// rm holds Q and W^T of the pass's gates (FP64, 32 entries per gate).
-__global__ __launch_bounds__(256) void k_tile_reduce(const double* __restrict__ partial, long nparts, int ng,
+// rm holds Q and W^T of the gates (FP64, 32 entries per gate).
+__global__ __launch_bounds__(256) void k_tile_reduce(const double* __restrict__ partial, long nparts,
 	const TileGates gk, const zc* __restrict__ rm, int dual, zc* __restrict__ acc, const int* skip)
 {
 	if (skipped(skip)) { return; }
@@ -1652,7 +1653,7 @@ __global__ __launch_bounds__(256) void k_tile_reduce(const double* __restrict__ 
 	__shared__ zc A[2][16];
 	const int j = blockIdx.x, i = threadIdx.x;
 	double s = 0;
-	for (long p = 0; p < nparts; p++) { s += partial[(p * ng + j) * 256 + i]; }
+	for (long p = 0; p < nparts; p++) { s += partial[(j * nparts + p) * 256 + i]; }
 	Dm[i >> 4][i & 15] = s;
 	__syncthreads();
 	const int which = (i >> 4) & 1, r = (i >> 2) & 3, c = i & 3;
