@@ -759,7 +759,6 @@ struct TilePlan
 	std::vector<int> order;         // circuit gate index of each execution slot
 	unsigned gfwd = 0, grev = 0;
 	size_t lds_fwd = 0, lds_rev = 0;
-	size_t lds_rev_seed = 0;        // the seed pass: also the fused forward pass's G, Z
 	size_t partial_doubles = 0;
 	// cyclic-product sweeps (EvalPlan::cyc): the launches and their grids
 	CycPlan cyc;
@@ -800,19 +799,9 @@ static decltype(&k_tile_forward<T, true, 0>) fwd_kernel(bool dual, int logE)
 }
 
 template <typename T>
-static decltype(&k_tile_reverse<T, true, 0>) rev_kernel(bool dual, int logE, bool seed = false)
+static decltype(&k_tile_reverse<T, true, 0>) rev_kernel(bool dual, int logE)
 {
 	if (!dual) { return k_tile_reverse<T, false, 0>; }
-	if (seed) {
-		if constexpr (sizeof(T) == 8) {
-			if (logE == 10) { return k_tile_reverse<T, true, 10, true>; }
-			if (logE == 9) { return k_tile_reverse<T, true, 9, true>; }
-		} else {
-			if (logE == 11) { return k_tile_reverse<T, true, 11, true>; }
-			if (logE == 10) { return k_tile_reverse<T, true, 10, true>; }
-		}
-		return k_tile_reverse<T, true, 0, true>;
-	}
 	if constexpr (sizeof(T) == 8) {
 		if (logE == 10) { return k_tile_reverse<T, true, 10>; }
 		if (logE == 9) { return k_tile_reverse<T, true, 9>; }
@@ -878,13 +867,11 @@ static std::shared_ptr<TilePlan> plan_tiles(const Context& dev, const Circuit& C
 	tp->lds_fwd = (size_t)(dual ? fwd_buffers<T, true>() : fwd_buffers<T, false>()) * (dual ? 2 : 1) *
 		(Ef * sizeof(cx<T>) + kLdsPadBytes) + fwd_mats + kFwdVoteBytes;
 	tp->lds_rev = (size_t)(dual ? rev_buffers<T, true>() : rev_buffers<T, false>()) * (dual ? 4 : 2) *
-		(E * sizeof(cx<T>) + lds_pad_rev<T>()) + rev_mats + kRevTraceBytes;
+		(E * sizeof(cx<T>) + lds_pad_rev<T>()) + rev_mats;
 	auto* kf = fwd_kernel<T>(dual, tp->tsf.K + tp->tsf.logC);
 	auto* kr = rev_kernel<T>(dual, ts.K + ts.logC);
 	allow_lds(kf, tp->lds_fwd);
 	allow_lds(kr, tp->lds_rev);
-	tp->lds_rev_seed = tp->lds_rev + (size_t)kMaxTileGates * fwd_mat_stride<true>() * sizeof(cx<T>);
-	allow_lds(rev_kernel<T>(dual, ts.K + ts.logC, true), tp->lds_rev_seed);
 	int occ_f = 0, occ_r = 0;
 	RQC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_f, reinterpret_cast<const void*>(kf), kTileThreads, tp->lds_fwd));
 	RQC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_r, reinterpret_cast<const void*>(kr), kTileThreads, tp->lds_rev));
@@ -1082,10 +1069,8 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 		npart = (mode == Mode::Target) ? (size_t)cp.ntrace * (cyc_nthreads(cp.K, false) / 64)
 		                               : (size_t)pl.G * cyc_parts(cp.L, cp.K) * (mode == Mode::Hvp ? 32 : 16);
 	} else if (pl.tiles) {
-		// outer-product partials, the chunk sums of the first reduction stage, then the trace
-		// partials of a first reverse pass that takes the target's trace
-		npart = std::max(npart, (pl.tp->partial_doubles + (size_t)kReduceChunks * pl.tp->reduce_gates * 256 + 1) / 2 +
-			(size_t)pl.tp->grev * kTileWaves);
+		// outer-product partials, then the chunk sums of the first reduction stage
+		npart = std::max(npart, (pl.tp->partial_doubles + (size_t)kReduceChunks * pl.tp->reduce_gates * 256 + 1) / 2);
 	}
 	else { npart = std::max(npart, (size_t)pl.grev_pg * kWidth); }
 	pl.n_part = npart;
@@ -1285,7 +1270,6 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 	const double outer_issued = (sizeof(T) == 8) ? (dual ? 96.0 : 32.0) : (dual ? 128.0 : 64.0);
 	auto* kf = fwd_kernel<T>(dual, tp.tsf.K + tp.tsf.logC);
 	auto* kr = rev_kernel<T>(dual, tp.ts.K + tp.ts.logC);
-	auto* krs = rev_kernel<T>(dual, tp.ts.K + tp.ts.logC, true);
 	const GateTerms* fterms = reinterpret_cast<const GateTerms*>(reinterpret_cast<const char*>(gterms) + tp.fterms_off);
 	const zc* rmats = reinterpret_cast<const zc*>(reinterpret_cast<const char*>(mats) + pl.rmats_off);
 	double* mpart = reinterpret_cast<double*>(d_partial);   // grev * waves * gates * 256 doubles
@@ -1295,25 +1279,13 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 	const int logB = ilog2_or_neg(B);
 	const double ab = (double)sz * sizeof(cx<T>);   // bytes of one state block
 	const int ns = dual ? 2 : 1;                     // state arrays per side
-	// HVP sweeps over the whole of a dense target in one block: the first reverse pass reads
-	// U's block as its output adjoint (FP64: into LDS; FP32: from HBM into registers, U staying
-	// FP64), forms the seed -conj(U) in LDS and takes the trace on the way (no separate target
-	// pass over U, psi and the seed)
-	const bool fuse_trace = dual && be == nullptr && !pl.sampled && B == N && P >= 1;
-	double* ttr = cpart + (size_t)kReduceChunks * tp.reduce_gates * 256;   // its per-wave trace partials
-	// and, with the planned tiles (one tile for both directions), it also runs the circuit's
-	// last forward pass on its tiles first: the circuit's output states never go through HBM
-	const int logEr = tp.ts.K + tp.ts.logC;
-	const bool planned_tile = (sizeof(T) == 8) ? (logEr == 9 || logEr == 10) : (logEr == 10 || logEr == 11);
-	const bool fuse_fwd = fuse_trace && P >= 2 && tp.tsf.K == tp.ts.K && tp.tsf.logC == tp.ts.logC && planned_tile;
-	const int Pf = fuse_fwd ? P - 1 : P;   // forward launches
 
 	for (long blk = 0; blk < pl.nblk; blk++) {
 		const long b0 = blk * B;
 		// the block's input columns and the trace's seed columns: basis columns and U, or samples and U X
 		const zc* seed = (be != nullptr) ? nullptr : pl.sampled ? W + (size_t)blk * sz : dU;
 		const long ldu = pl.sampled ? B : N, u0 = pl.sampled ? 0 : b0;
-		for (int p = 0; p < Pf; p++) {
+		for (int p = 0; p < P; p++) {
 			// pass 0 starts from the identity block (flags 1) or the sample block, with dpsi = 0 (flags 2)
 			const int flags = (p == 0) ? (pl.sampled ? 2 : 3) : 0;
 			const cx<T>* in = (p == 0) ? (pl.sampled ? X + (size_t)blk * sz : nullptr)
@@ -1333,12 +1305,12 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 			k_blockenc_residual<T><<<gtr, kBlock, 0, s.stream>>>(be->H, pl.L / 2, b0, psiG,
 				mode == Mode::Target ? nullptr : phi[0], dual ? DPS(P) : nullptr, dual ? be->J : nullptr, B, logB, N * B,
 				tpart, skip);
-		} else if (!fuse_trace) {
+		} else {
 			LaunchTimer lt(s, RQC_KERNEL_TARGET, (double)sz * sizeof(zc) + (mode == Mode::Target ? 1 : 2) * ab);
 			k_target_trace<T><<<gtr, kBlock, 0, s.stream>>>(seed, ldu, u0, psiG, mode == Mode::Target ? nullptr : phi[0],
 				B, logB, N * B, tpart, skip);
 		}
-		if (!fuse_trace) {
+		{
 			LaunchTimer lt(s, RQC_KERNEL_OTHER);
 			k_reduce_partials<<<1, kBlock, 0, s.stream>>>(tpart, (int)gtr, 1, d_acc, skip);
 		}
@@ -1352,34 +1324,20 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 			if (p == 0) { flags |= 8; }
 			// the first pass from identity columns: only tiles with an identity element contribute
 			if (p == 0 && !pl.sampled) { flags |= 32; }
-			const bool seed_pass = fuse_trace && p == P - 1;
-			const bool with_fwd = seed_pass && fuse_fwd;   // psi, dpsi at the pass input (flags 16)
-			if (with_fwd) { flags |= 16; }
 			const int ng = (int)tp.passes[p].gates.size();
 			{
-				// (the FP32 seed pass reads U in FP64: twice an FP32 array)
-				const int reads = (dual ? 3 + (p < P - 1) : 2) + ((seed_pass && sizeof(T) == 4) ? 1 : 0);
+				const int reads = dual ? 3 + (p < P - 1) : 2;
 				// algorithmic work of the launch: per amplitude and gate of the tiles it processes,
-				// the adjoint update and the outer products (dual 24 complex MACs, plain 8), and a
-				// fused forward pass (12); issued besides: the recovery, in the forms above
+				// the adjoint update and the outer products (dual 24 complex MACs, plain 8); issued
+				// besides: the recovery, in the forms above
 				const double frac = (flags & 32) ? (double)active_tiles(tp.args[p], pl.B) / (double)ntiles : 1.0;
 				const double amps = frac * (double)ntiles * E;
 				const double rflops = (dual ? 192.0 : 64.0) * ng * amps;
 				const double rissued = (2.0 * app_issued + outer_issued) * ng * amps;
-				const double fflops = with_fwd ? 96.0 * ng * (double)ntiles * E : 0.0;
-				const double fissued = with_fwd ? app_issued * ng * (double)ntiles * E : 0.0;
-				LaunchTimer lt(s, RQC_KERNEL_REVERSE, (double)(reads * frac + ns * (p > 0)) * ab, rflops + fflops,
-					rissued + fissued);
-				(seed_pass ? krs : kr)<<<tp.grev, kTileThreads, seed_pass ? tp.lds_rev_seed : tp.lds_rev, s.stream>>>(
-					with_fwd ? PS(p) : PS(p + 1), dual ? (with_fwd ? DPS(p) : DPS(p + 1)) : nullptr,
-					seed_pass ? reinterpret_cast<const cx<T>*>(seed) : phi[cur], dual ? dphi[cur] : nullptr, phi[1 - cur],
-					dual ? dphi[1 - cur] : nullptr, tp.args[p], mats, gterms, B, b0, ntiles, flags,
-					mpart + (tp.args[p].x0 - red->x0) * nparts * 256, ttr, skip);
-			}
-			if (seed_pass) {
-				LaunchTimer lt(s, RQC_KERNEL_OTHER);
-				k_reduce_partials<<<1, kBlock, 0, s.stream>>>(reinterpret_cast<const zc*>(ttr),
-					(int)(tp.grev * kTileWaves), 1, d_acc, skip);
+				LaunchTimer lt(s, RQC_KERNEL_REVERSE, (double)(reads * frac + ns * (p > 0)) * ab, rflops, rissued);
+				kr<<<tp.grev, kTileThreads, tp.lds_rev, s.stream>>>(PS(p + 1), dual ? DPS(p + 1) : nullptr, phi[cur],
+					dual ? dphi[cur] : nullptr, phi[1 - cur], dual ? dphi[1 - cur] : nullptr, tp.args[p], mats, gterms, B, b0,
+					ntiles, flags, mpart + (tp.args[p].x0 - red->x0) * nparts * 256, skip);
 			}
 			if (p == red->pass) {
 				LaunchTimer lt(s, RQC_KERNEL_OTHER);

@@ -115,8 +115,6 @@ enum { kMatG = 0, kMatZ = 1, kMatGinv = 2, kMatW = 3, kMatGT = 4, kMatZT = 5 };
 constexpr int kMatPairOff = 20;
 template <bool DUAL> constexpr int fwd_mat_stride() { return DUAL ? 2 * kMatPairOff : 16; }
 template <bool DUAL> constexpr int rev_mat_stride() { return DUAL ? 4 * kMatPairOff : 2 * kMatPairOff; }
-// after the reverse pass's gate matrices: a running trace sum (two doubles) per wave
-constexpr int kRevTraceBytes = kTileWaves * 16;
 // after the forward pass's gate matrices: one word per wave (pass 0's zero-tile vote)
 constexpr int kFwdVoteBytes = kTileWaves * 4;
 
@@ -997,14 +995,8 @@ __global__ __launch_bounds__(kTileThreads, (fwd_waves_per_simd<T, DUAL, LOGE>())
 // reverse pass.  Inputs: psi (and dpsi) at the pass output (checkpoint), phi
 // (and dphi) at the pass output; outputs phi (and dphi) at the pass input.
 // flags: 4 = dphi at the pass output is zero, 8 = do not write phi at the pass input,
-// 16 (SEED, planned tiles) = psi and dpsi are given at the pass input and the pass's
-// gates are applied to them first (G, Z after the trace sums in LDS), 32 (with 8) = the
-// sweep started from identity columns b0 + j: tiles without an identity element are skipped.
-// SEED (dual sweeps, the circuit's last pass): phi_out is the target U's column block (FP64 in
-// both precisions; FP32 reads it from HBM in the seed step, FP64 loads it as the adjoint tile);
-// the seed -conj(U) is formed in LDS and the trace sum(-conj(U) psi) goes to
-// trace[2 (block * waves + wave)] (a separate instantiation, so that the other passes run
-// exactly the kernel without it: the extra loop code measured 8 % slower on every pass).
+// 32 (with 8) = the sweep started from identity columns b0 + j: tiles without an identity
+// element are skipped.
 // partial[(j * parts + part) * 256 + row * 16 + col], part = block * waves + wave:
 // the 16 x 16 outer-product sums of gate j (rows: component 4 (2 s + p) + r of
 // the adjoint at the gate input, columns: that of the state before the gate).
@@ -1020,13 +1012,13 @@ __global__ __launch_bounds__(kTileThreads, (fwd_waves_per_simd<T, DUAL, LOGE>())
 template <typename T, bool DUAL> constexpr int rev_buffers() { return DUAL ? 1 : 2; }
 template <typename T, bool DUAL> constexpr int rev_waves_per_simd() { return 2; }
 
-template <typename T, bool DUAL, int LOGE = 0, bool SEED = false>
+template <typename T, bool DUAL, int LOGE = 0>
 __global__ __launch_bounds__(kTileThreads, (rev_waves_per_simd<T, DUAL>())) void k_tile_reverse(
 	const cx<T>* __restrict__ psi_out, const cx<T>* __restrict__ dpsi_out,
 	const cx<T>* __restrict__ phi_out, const cx<T>* __restrict__ dphi_out,
 	cx<T>* __restrict__ phi_in, cx<T>* __restrict__ dphi_in,
 	const TileArgs P, const cx<T>* __restrict__ mats, const GateTerms* __restrict__ gterms, long B, long b0, long ntiles,
-	int flags, double* __restrict__ partial, double* __restrict__ trace, const int* skip)
+	int flags, double* __restrict__ partial, const int* skip)
 {
 	if (skipped(skip)) { return; }
 	extern __shared__ __align__(16) char lds_raw[];
@@ -1068,8 +1060,7 @@ __global__ __launch_bounds__(kTileThreads, (rev_waves_per_simd<T, DUAL>())) void
 	auto prefetch = [&](long tile, int b) {
 		const long base = deposit_bits(tile >> P.lognc, P.rmask) * B + ((tile & cmask) << P.logC);
 		tile_issue(state(b, 0), psi_out, base, io);
-		// (the FP32 seed pass reads the FP64 target's tile itself, in its seed step)
-		if constexpr (!(SEED && sizeof(T) == 4)) { tile_issue(state(b, NS / 2), phi_out, base, io); }
+		tile_issue(state(b, NS / 2), phi_out, base, io);
 		if (DUAL) {
 			tile_issue(state(b, 1), dpsi_out, base, io);
 			if (flags & 4) { tile_fill(state(b, 3), io, cx<T>{0, 0}); }
@@ -1409,163 +1400,9 @@ __global__ __launch_bounds__(kTileThreads, (rev_waves_per_simd<T, DUAL>())) void
 			store(prev, b ^ 1);
 		}
 	} else {
-		// SEED: phi_out holds the target U's tile; the adjoint seed is -conj(U), formed in
-		// place, and the target's trace sum(-conj(U) psi) is taken over the tile on the way
-		// (per thread and wave, then added to the wave's running sum)
-		static_assert(!SEED || DUAL, "the seed pass is a dual sweep");
-		// (the running trace sum of a wave sits in LDS after the gate matrices, so that no
-		// register is held across the gates for it)
-		double* tracc = reinterpret_cast<double*>(lds_raw + rev_buffers<T, DUAL>() * NS * sbytes +
-			kMaxTileGates * rev_mat_stride<DUAL>() * (int)sizeof(cx<T>)) + 2 * (threadIdx.x >> 6);
-		if constexpr (SEED) {
-			if (lane == 0) { tracc[0] = 0; tracc[1] = 0; }
-		}
-		// SEED with flags & 16 (planned tiles): psi_out and dpsi_out hold the states at
-		// the pass input, and the pass's gates are applied to them here first, so that the
-		// circuit's output states never go through HBM (its last forward pass, fused)
-		cx<T>* lmf = reinterpret_cast<cx<T>*>(reinterpret_cast<char*>(tracc - 2 * (threadIdx.x >> 6)) + kRevTraceBytes);
-		if constexpr (SEED && FIXED) {
-			if (flags & 16) {
-				const int whichf[2] = {kMatG, kMatZ};
-				load_pass_mats(mats, P.x0, P.ng, whichf, 2, fwd_mat_stride<true>(), lmf);
-			}
-		}
-		auto forward_gates = [&]() {
-			if constexpr (SEED && FIXED) {
-				// the forward pass's steps: FP64 the 4 x 4 blocks, FP32 the real 16 x 16 form with
-				// amplitude-major rows (the forward kernel's gate code, so that the states are the
-				// ones a forward launch would write)
-				constexpr int GSF = 2, gqf = 16;
-				constexpr int NSTF = ((1 << LOGE) / 4 / kTileWaves) / (GSF * gqf);
-				static_assert(NSTF >= 1 && NSTF <= 4, "one to four steps per gate and wave");
-				auto fgate = [&](auto jc) {
-					constexpr int j = decltype(jc)::value;
-					if (j < P.ng) {
-						if (j > 0 && ((P.barrier >> j) & 1)) { __syncthreads(); }
-						Frag44 f;
-						T af[4];
-						if constexpr (F44) {
-							f = frag44(reinterpret_cast<const cx<double>*>(lmf + j * fwd_mat_stride<true>()));
-						} else {
-							const AOperandMap<T, true> amf = a_operand_map<T, true, true>();
-							const T* mjf = reinterpret_cast<const T*>(lmf + j * fwd_mat_stride<true>());
-#pragma unroll
-							for (int kk = 0; kk < 4; kk++) { af[kk] = mjf[amf.aoff[kk]] * amf.afac[kk]; }
-						}
-						int ea = eabj[j];
-						asm volatile("" : "+v"(ea));
-						if constexpr (F44) { __builtin_assume((ea & 15) == 0); }
-						GateOperands<T, GSF> o[NSTF];
-						unsigned la[NSTF][GSF];
-						auto load_step = [&](auto sc) {
-							constexpr int SI = decltype(sc)::value;
-#pragma unroll
-							for (int n = 0; n < GSF; n++) {
-								const int gi = (SI * GSF * gqf + n * gqf) >> 4;
-								const int gb = sgj[j][0] ^ ((gi & 1) ? sgj[j][1] : 0) ^ ((gi & 2) ? sgj[j][2] : 0) ^
-								               ((gi & 4) ? sgj[j][3] : 0);
-								la[SI][n] = (unsigned)(ea ^ gb);
-								if constexpr (F44) {
-									o[SI].x[n] = lds_load_cxd(la[SI][n]);
-									o[SI].y[n] = lds_load_cxd(la[SI][n] + sbytes);
-								} else {
-									o[SI].x[n] = *reinterpret_cast<const cx<T>*>(lds_raw + la[SI][n]);
-									o[SI].y[n] = *reinterpret_cast<const cx<T>*>(lds_raw + la[SI][n] + sbytes);
-								}
-							}
-						};
-						auto step = [&](auto sc) {
-							constexpr int SI = decltype(sc)::value;
-							if constexpr (SI + 1 < NSTF) { load_step(std::integral_constant<int, SI + 1>{}); }
-							__builtin_amdgcn_sched_barrier(0);
-							__builtin_amdgcn_s_setprio(1);
-							if constexpr (F44) { gate_mfma44<GSF>(f, o[SI]); }
-							else { gate_mfma<T, GSF>(af, o[SI]); }
-							__builtin_amdgcn_s_setprio(0);
-#pragma unroll
-							for (int n = 0; n < GSF; n++) {
-								if constexpr (F44) {
-									lds_store_cxd(la[SI][n], cx<double>{o[SI].acc[n][0], o[SI].acc[n][1]});
-									lds_store_cxd(la[SI][n] + sbytes, cx<double>{o[SI].acc[n][2], o[SI].acc[n][3]});
-								} else {
-									*reinterpret_cast<cx<T>*>(lds_raw + la[SI][n]) = cx<T>{o[SI].acc[n][0], o[SI].acc[n][1]};
-									*reinterpret_cast<cx<T>*>(lds_raw + la[SI][n] + sbytes) =
-										cx<T>{o[SI].acc[n][2], o[SI].acc[n][3]};
-								}
-							}
-						};
-						load_step(std::integral_constant<int, 0>{});
-						step(std::integral_constant<int, 0>{});
-						if constexpr (NSTF > 1) { step(std::integral_constant<int, 1>{}); }
-						if constexpr (NSTF > 2) { step(std::integral_constant<int, 2>{}); }
-						if constexpr (NSTF > 3) { step(std::integral_constant<int, 3>{}); }
-					}
-				};
-				fgate(std::integral_constant<int, 0>{});
-				fgate(std::integral_constant<int, 1>{});
-				fgate(std::integral_constant<int, 2>{});
-				fgate(std::integral_constant<int, 3>{});
-				fgate(std::integral_constant<int, 4>{});
-				fgate(std::integral_constant<int, 5>{});
-				fgate(std::integral_constant<int, 6>{});
-				fgate(std::integral_constant<int, 7>{});
-			}
-		};
 		while (tile < ntiles) {
 			__builtin_amdgcn_s_waitcnt(0);
 			__syncthreads();
-			if constexpr (SEED && FIXED) {
-				if (flags & 16) {
-					forward_gates();
-					__syncthreads();
-				}
-			}
-			// FP32 seed pass: the target's FP64 elements of the thread's slots, from HBM (held
-			// across the forward gates they would take registers the gates need)
-			constexpr int EPL = TileIO<T>::epl;
-			cx<double> useed[(SEED && sizeof(T) == 4) ? kMaxSlots * EPL : 1];
-			if constexpr (SEED && sizeof(T) == 4) {
-				const cx<double>* Ud = reinterpret_cast<const cx<double>*>(phi_out);
-				const long base = deposit_bits(tile >> P.lognc, P.rmask) * B + ((tile & cmask) << P.logC);
-#pragma unroll
-				for (int k = 0; k < kMaxSlots; k++) {
-					if (k < io.nk) {
-#pragma unroll
-						for (int i = 0; i < EPL; i++) { useed[k * EPL + i] = Ud[base + io.goff[k] + i]; }
-					}
-				}
-			}
-			if constexpr (SEED) {
-				double tr_re = 0, tr_im = 0;
-#pragma unroll
-				for (int k = 0; k < kMaxSlots; k++) {
-					if (k < io.nk) {
-#pragma unroll
-						for (int i = 0; i < EPL; i++) {
-							const int e = (threadIdx.x + k * kTileThreads) * EPL + i;   // the slot's elements
-							cx<T>* ph = state(0, NS / 2) + e;
-							cx<double> u;
-							if constexpr (sizeof(T) == 4) { u = useed[k * EPL + i]; }
-							else { u = cx<double>{(double)ph->x, (double)ph->y}; }
-							const cx<double> ps = {(double)state(0, 0)[e].x, (double)state(0, 0)[e].y};
-							const cx<double> sd = {-u.x, u.y};
-							*ph = cx<T>{(T)sd.x, (T)sd.y};
-							tr_re += sd.x * ps.x - sd.y * ps.y;
-							tr_im += sd.x * ps.y + sd.y * ps.x;
-						}
-					}
-				}
-#pragma unroll
-				for (int o = 32; o > 0; o >>= 1) {
-					tr_re += __shfl_xor(tr_re, o);
-					tr_im += __shfl_xor(tr_im, o);
-				}
-				if (lane == 0) {
-					tracc[0] += tr_re;
-					tracc[1] += tr_im;
-				}
-				__syncthreads();
-			}
 			run_tile(0);
 			__syncthreads();
 			// each thread stores the slots that it then refills
@@ -1573,13 +1410,6 @@ __global__ __launch_bounds__(kTileThreads, (rev_waves_per_simd<T, DUAL>())) void
 			const long next = next_tile(tile + gridDim.x);
 			if (next < ntiles) { prefetch(next, 0); }
 			tile = next;
-		}
-		if constexpr (SEED) {
-			if (lane == 0) {
-				const long w = (long)blockIdx.x * kTileWaves + (threadIdx.x >> 6);
-				trace[2 * w] = tracc[0];
-				trace[2 * w + 1] = tracc[1];
-			}
 		}
 	}
 	const long part = (long)blockIdx.x * kTileWaves + (threadIdx.x >> 6);
