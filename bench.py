@@ -41,14 +41,13 @@ METRIC = "grad+HVP evals/s, L=14 brickwall d9, FP64 vs mixed; served p99 latency
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 REVERSE_KERNEL = {
-    "tile_pass": "k_tile_reverse<double,dual> (reverse tile pass: up to 8 gates per HBM pass; state recovery, "
-                 "adjoint update and gradient/HVP outer products on the FP64 matrix cores as 4x4x4 block "
-                 "products, the gate applications in the three-real-product complex form; the launch of the circuit's last pass also runs that pass's forward gates, and "
-                 "the circuit's first pass skips the tiles that hold no identity element)",
+    "tile_pass": "k_cyc_sweep<6,dual,double> (conjugations M <- G M G^-1 of the cyclic product and its derivative, "
+                 "up to 8 gates per HBM pass, each gate's partial trace recorded; FP64 matrix cores as 4x4x4 block "
+                 "products in the three-real-product complex form)",
     "per_gate": "k_gate_reverse<double,dual> (per-gate reverse sweep with gradient/HVP sums)",
 }
 # measured HBM traffic of the reverse kernel (rocprofv3 FETCH_SIZE / WRITE_SIZE, copy-kernel calibrated)
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_k_tile_reverse_L14_d9.json")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_k_cyc_sweep_L14_d9.json")
 
 
 def reverse_alg_flops(L, d):
@@ -189,10 +188,9 @@ def run(args):
     # arrays read + written once, summed by the library per launch) is reported beside it
     rev_ms, rev_n, rev_bytes = r64["prof"][R.KERNEL_REVERSE]
     engine_used, passes = R.last_sweep()
-    # the library's count per launch: 192 flops (issued on the matrix cores: 240, recovery
-    # included, gate applications in the three-product form) per amplitude and gate of the tiles
-    # a launch processes (the first pass skips the tiles without an identity element, whose
-    # terms vanish), plus the forward pass the last launch carries (96; issued 72)
+    # the library's count per launch: 72 flops per element and side of each gate of the tiles a
+    # launch processes, both algorithmic and issued (a conjugation in the three-product form; it
+    # stands for the adjoint update and the outer products of the count below)
     rev_flops, rev_issued = r64["flops"][R.KERNEL_REVERSE] if engine == "tile_pass" else (None, None)
     achieved_tf = rev_flops / (rev_ms * 1e-3) / 1e12 if rev_flops else None
     issued_tf = rev_issued / (rev_ms * 1e-3) / 1e12 if rev_flops else None
@@ -200,7 +198,7 @@ def run(args):
     traffic = None
     if engine == "tile_pass" and os.path.exists(TRAFFIC_FILE) and (L, d) == (14, 9):
         with open(TRAFFIC_FILE) as fh:
-            traffic = json.load(fh)["k_tile_reverse_fp64"]["hbm_bytes_per_launch"]
+            traffic = json.load(fh)["k_cyc_sweep_reverse_fp64"]["hbm_bytes_per_launch"]
     f64, g64, h64 = r64["out"]
     f32, g32, h32 = r32["out"]
     mixed_err = {"f_abs": float(abs(f32 - f64)), "f_abs_over_N": float(abs(f32 - f64) / N),
