@@ -75,6 +75,27 @@ void DeviceBuffer::release()
 	}
 }
 
+void HostBuffer::reserve(size_t n)
+{
+	if (n <= bytes) { return; }
+	if (ptr != nullptr) {
+		RQC_HIP(hipDeviceSynchronize());
+		release();
+	}
+	const size_t r = (n + 65535) & ~(size_t)65535;
+	RQC_HIP(hipHostMalloc(&ptr, r, hipHostMallocDefault));
+	bytes = r;
+}
+
+void HostBuffer::release()
+{
+	if (ptr != nullptr) {
+		(void)hipHostFree(ptr);
+		ptr = nullptr;
+		bytes = 0;
+	}
+}
+
 Context& ctx()
 {
 	static Context* c = nullptr;
@@ -1551,6 +1572,21 @@ void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit
 		pl.fp32 ? (be != nullptr ? 2 : 1) : 0, cps.stride, cps.res_stride, skip);
 }
 
+// A copy kernel is queued like any other launch, where a copy call of some 30 KB takes the host 15 us
+// more and its engine has to hand over to the compute queue; beyond 256 KiB (some 128 gates) the
+// copy engine's bandwidth counts for more.
+void upload_pinned(Slot& s, void* dst, const void* src, size_t bytes)
+{
+	const size_t n = (bytes + 15) & ~(size_t)15;
+	if (n > ((size_t)1 << 18)) {
+		RQC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, s.stream));
+		return;
+	}
+	LaunchTimer lt(s, RQC_KERNEL_OTHER);
+	k_copy16<<<nblocks((long)(n / sizeof(zc))), kBlock, 0, s.stream>>>(static_cast<const zc*>(src), static_cast<zc*>(dst),
+		(long)(n / sizeof(zc)));
+}
+
 void unpack_result(const EvalPlan& pl, const char* res, EvalResult& R)
 {
 	const size_t n = 16 * (size_t)pl.ng;
@@ -1628,7 +1664,29 @@ static TileChoice tune_eval(Context& c, const Circuit& C, Mode mode, int per, bo
 	return best;
 }
 
-// one evaluation on the main slot (the reference ABI's target functions)
+// One evaluation on the main slot.  Its tables go up from pinned memory and k_finalize writes its
+// results there, so that a call has no copy but the one kernel (6 qubits, 3 layers: 103 us with a
+// copy call each way, 66 us without; 10 qubits, 5 layers: 239 and 197 us).
+static EvalResult run_eval(Context& c, const EvalPlan& pl, const Circuit& C, const zc* dU, const void* X, const zc* W,
+	const BlockEnc* be)
+{
+	const size_t off = align256(pl.tab_bytes), nres = pl.res_bytes();
+	c.io.reserve(off + nres);
+	char* io = c.io.as<char>();
+	std::memset(io, 0, off + nres);
+	fill_eval_tables(pl, C, io);
+	c.work.reserve(pl.bytes);
+	char* work = c.work.as<char>();
+	upload_pinned(c, work + pl.off_tab, io, pl.tab_bytes);
+	enqueue_eval(c, c, pl, C, dU, work, nullptr, io + off, nullptr, nullptr, X, W, be);
+	RQC_HIP(hipStreamSynchronize(c.stream));
+	RQC_HIP(hipGetLastError());
+	EvalResult R;
+	unpack_result(pl, io + off, R);
+	return R;
+}
+
+// one evaluation of a dense target (the reference ABI's target functions)
 static EvalResult eval_targets(const Circuit& C, linear_func ufunc, void* udata, Mode mode, int per, bool project)
 {
 	Context& c = ctx();
@@ -1639,19 +1697,7 @@ static EvalResult eval_targets(const Circuit& C, linear_func ufunc, void* udata,
 	if (c.eval_autotune && c.engine == RQC_ENGINE_TILE_PASS) { tc = tune_eval(c, C, mode, per, project, unitary, dU); }
 	const EvalPlan pl = plan_eval(c, C, mode, per, c.precision == RQC_PRECISION_MIXED, project, unitary, c.ws_limit,
 		c.work.bytes, tc.logE > 0 ? &tc : nullptr);
-	std::vector<char> tab(pl.tab_bytes);
-	fill_eval_tables(pl, C, tab.data());
-	c.work.reserve(pl.bytes);
-	char* work = c.work.as<char>();
-	enqueue_eval(c, c, pl, C, dU, work, nullptr, nullptr, tab.data(), nullptr, nullptr, nullptr);
-	std::vector<char> res(pl.res_bytes());
-	const size_t nres = (mode == Mode::Target) ? sizeof(zc) : res.size();
-	RQC_HIP(hipMemcpyAsync(res.data(), work + pl.off_res, nres, hipMemcpyDeviceToHost, c.stream));
-	RQC_HIP(hipStreamSynchronize(c.stream));
-	RQC_HIP(hipGetLastError());
-	EvalResult R;
-	unpack_result(pl, res.data(), R);
-	return R;
+	return run_eval(c, pl, C, dU, nullptr, nullptr, nullptr);
 }
 
 // ============================================================== device targets
@@ -1834,11 +1880,12 @@ struct StateSums
 		part = acc + n;
 	}
 	zc* part_of(int k) const { return part + (size_t)k * grid * kWidth; }
-	void reduce(Context& c) const
+	// into acc, or into pinned memory
+	void reduce(Context& c, zc* out = nullptr) const
 	{
 		if (ngates == 0) { return; }
 		LaunchTimer lt(c, RQC_KERNEL_OTHER);
-		k_reduce_gates<<<dim3(ngates, kWidth), kBlock, 0, c.stream>>>(part, (int)grid, acc);
+		k_reduce_gates<<<dim3(ngates, kWidth), kBlock, 0, c.stream>>>(part, (int)grid, out != nullptr ? out : acc);
 	}
 };
 
@@ -1876,18 +1923,19 @@ static std::vector<StatePass> plan_state(const Circuit& C)
 }
 
 // the HVP of a statevector in passes: psi_out, and every gate's sums into sums.part; S holds the
-// states between the passes and the tangents after them, then the adjoint and its tangent.  ops is
-// read by a copy on the stream.
+// states between the passes and the tangents after them, then the adjoint and its tangent; ops:
+// pinned memory for the gates' operands
 static void state_passes(Context& c, const Circuit& C, const std::vector<StatePass>& plan, const StateSums& sums, const zc* psi,
-	const zc* phi, zc* psi_out, zc* S, std::vector<StateOp>& ops, StateOp* dev_ops)
+	const zc* phi, zc* psi_out, zc* S, StateOp* ops, StateOp* dev_ops)
 {
 	const int L = C.L, P = (int)plan.size(), K = plan[0].tile.K;
 	const size_t n = (size_t)1 << L;
 	std::vector<int> first;
+	int x = 0;
 	for (const StatePass& p : plan) {
 		int pos[32];
 		for (int t = 0; t < K; t++) { pos[p.tile.bit[t]] = t; }
-		first.push_back((int)ops.size());
+		first.push_back(x);
 		for (int k : p.gates) {
 			StateOp o;
 			std::memcpy(o.g, &C.gates[16 * (size_t)k], sizeof(o.g));
@@ -1899,11 +1947,11 @@ static void state_passes(Context& c, const Circuit& C, const std::vector<StatePa
 			o.gate.pi = pos[L - 1 - C.wi[k]];
 			o.gate.pj = pos[L - 1 - C.wj[k]];
 			o.gate.index = k;
-			o.gate.first = ops.empty();
-			ops.push_back(o);
+			o.gate.first = x == 0;
+			ops[x++] = o;
 		}
 	}
-	RQC_HIP(hipMemcpyAsync(dev_ops, ops.data(), ops.size() * sizeof(StateOp), hipMemcpyHostToDevice, c.stream));
+	upload_pinned(c, dev_ops, ops, x * sizeof(StateOp));
 	const int nt = std::max(128, 1 << (K - 1));
 	const size_t lds_f = state_lds_bytes(false), lds_r = state_lds_bytes(true);
 	allow_lds(k_state_pass<false>, lds_f);
@@ -2388,7 +2436,6 @@ extern "C" int quantum_circuit_gates_hessian_vector_product(const struct mat4x4 
 		const bool passes = c.engine == RQC_ENGINE_TILE_PASS && ngates > 1 && L <= 30 && gates_near_unitary(C);
 		const std::vector<StatePass> plan = passes ? plan_state(C) : std::vector<StatePass>();
 		const StateSums sums(c, ngates, L, passes ? 1u << (L - plan[0].tile.K) : 0);
-		zc* acc = sums.acc;
 		Staging s(c);
 		const int a = s.add(psi->data, bytes, true, false);
 		const int f = s.add(phi->data, bytes, true, false);
@@ -2397,9 +2444,12 @@ extern "C" int quantum_circuit_gates_hessian_vector_product(const struct mat4x4 
 		const int tab = s.scratch(passes ? ngates * sizeof(StateOp) : 0);
 		s.upload();
 		zc* S = s.dev<zc>(st);
-		std::vector<StateOp> ops;
+		// the gates' operands, then the sums
+		const size_t opbytes = passes ? ngates * sizeof(StateOp) : 0;
+		c.io.reserve(std::max<size_t>(opbytes + ngates * kWidth * sizeof(zc), 16));
+		zc* hacc = reinterpret_cast<zc*>(c.io.as<char>() + opbytes);
 		if (passes) {
-			state_passes(c, C, plan, sums, s.dev<zc>(a), s.dev<zc>(f), s.dev<zc>(o), S, ops, s.dev<StateOp>(tab));
+			state_passes(c, C, plan, sums, s.dev<zc>(a), s.dev<zc>(f), s.dev<zc>(o), S, c.io.as<StateOp>(), s.dev<StateOp>(tab));
 		} else {
 			auto P = [&](int k) { return k == 0 ? s.dev<zc>(a) : S + k * n; };   // psi_k, k = 0 .. G
 			auto D = [&](int k) { return S + (ngates + k) * n; };                // dpsi_k, k = 1 .. G
@@ -2420,9 +2470,7 @@ extern "C" int quantum_circuit_gates_hessian_vector_product(const struct mat4x4 
 			}
 			dcopy(c, s.dev<zc>(o), P(ngates), bytes);   // last: psi and psi_out may be one array
 		}
-		sums.reduce(c);
-		std::vector<zc> hacc(32 * (size_t)ngates);
-		RQC_HIP(hipMemcpyAsync(hacc.data(), acc, hacc.size() * sizeof(zc), hipMemcpyDeviceToHost, c.stream));
+		sums.reduce(c, hacc);
 		s.download();
 		for (int k = 0; k < ngates; k++) {
 			std::memcpy(dgates[k].data, &hacc[32 * (size_t)k], 16 * sizeof(zc));
@@ -3146,19 +3194,8 @@ static EvalResult eval_blockenc(const Circuit& C, linear_func hfunc, void* hdata
 	const EvalPlan pl = plan_eval(c, C, mode, C.L / 2, c.precision == RQC_PRECISION_MIXED, project, unitary, c.ws_limit,
 		c.work.bytes, nullptr, 1L << (C.L / 2));
 	const BlockEncInputs bi = prepare_blockenc(c, pl, hfunc, hdata, 0);
-	std::vector<char> tab(pl.tab_bytes);
-	fill_eval_tables(pl, C, tab.data());
-	c.work.reserve(pl.bytes);
-	char* work = c.work.as<char>();
 	const BlockEnc be{bi.H, nullptr};
-	enqueue_eval(c, c, pl, C, nullptr, work, nullptr, nullptr, tab.data(), nullptr, bi.X, nullptr, &be);
-	std::vector<char> res(pl.res_bytes());
-	RQC_HIP(hipMemcpyAsync(res.data(), work + pl.off_res, res.size(), hipMemcpyDeviceToHost, c.stream));
-	RQC_HIP(hipStreamSynchronize(c.stream));
-	RQC_HIP(hipGetLastError());
-	EvalResult R;
-	unpack_result(pl, res.data(), R);
-	return R;
+	return run_eval(c, pl, C, nullptr, bi.X, nullptr, &be);
 }
 
 // HVP columns of a Hessian on a cyclic-product plan: several evaluations per launch, their tables
@@ -3166,7 +3203,7 @@ static EvalResult eval_blockenc(const Circuit& C, linear_func hfunc, void* hdata
 // 2.55 ms, launch after launch of 64 small tiles; together 0.33 ms (both with the host side).
 static void hessian_columns(Context& c, const EvalPlan& pl, const Circuit& C, const zc* dU, int m, char* hres, size_t rs)
 {
-	const size_t stride = align256(pl.bytes), res_off = align256(pl.tab_bytes), base = res_off + (size_t)m * rs;
+	const size_t stride = align256(pl.bytes), base = align256(pl.tab_bytes), nres = (size_t)m * rs;
 	// enough tiles to fill the device 16 times over and no more (2 GiB of arrays in FP64)
 	const long tiles = 1L << (2 * (pl.L - pl.tile_K));
 	int chunk = (int)std::max<long>(1, std::min<long>(m, 4096 / tiles));
@@ -3181,9 +3218,11 @@ static void hessian_columns(Context& c, const EvalPlan& pl, const Circuit& C, co
 	}
 	c.work.reserve(base + (size_t)chunk * stride);
 	char* work = c.work.as<char>();
-	std::vector<char> tab(pl.tab_bytes);
-	fill_eval_tables(pl, C, tab.data());
-	RQC_HIP(hipMemcpyAsync(work, tab.data(), pl.tab_bytes, hipMemcpyHostToDevice, c.stream));
+	c.io.reserve(base + nres);
+	char* io = c.io.as<char>();
+	std::memset(io, 0, base + nres);
+	fill_eval_tables(pl, C, io);
+	upload_pinned(c, work, io, pl.tab_bytes);
 	for (int c0 = 0; c0 < m; c0 += chunk) {
 		const int n = std::min(chunk, m - c0);
 		char* w = work + base;
@@ -3193,12 +3232,12 @@ static void hessian_columns(Context& c, const EvalPlan& pl, const Circuit& C, co
 			k_cyc_unit_tables<<<dim3(g, n), kBlock, 0, c.stream>>>(work, w + pl.off_tab, (long)stride, (long)pl.tab_bytes,
 				(long)pl.rmats_off, (long)pl.mats_bytes, pl.G, pl.per, c0);
 		}
-		enqueue_eval(c, c, pl, C, dU, w, nullptr, work + res_off + (size_t)c0 * rs, nullptr, nullptr, nullptr, nullptr, nullptr,
+		enqueue_eval(c, c, pl, C, dU, w, nullptr, io + base + (size_t)c0 * rs, nullptr, nullptr, nullptr, nullptr, nullptr,
 			EvalCopies{n, (long)stride, (long)rs});
 	}
-	RQC_HIP(hipMemcpyAsync(hres, work + res_off, (size_t)m * rs, hipMemcpyDeviceToHost, c.stream));
 	RQC_HIP(hipStreamSynchronize(c.stream));
 	RQC_HIP(hipGetLastError());
+	std::memcpy(hres, io + base, nres);
 }
 
 // Complex Hessian of the brickwall target (reference src/target.c:687-797).  Column
@@ -3314,17 +3353,7 @@ static EvalResult eval_sampled(const Circuit& C, linear_func ufunc, void* udata,
 	const EvalPlan pl = plan_eval(c, C, mode, per, c.precision == RQC_PRECISION_MIXED, project, unitary, c.ws_limit,
 		c.work.bytes, nullptr, nsamples);
 	const SampleBlocks sb = prepare_samples(c, pl, ufunc, udata, rng);
-	std::vector<char> tab(pl.tab_bytes);
-	fill_eval_tables(pl, C, tab.data());
-	c.work.reserve(pl.bytes);
-	char* work = c.work.as<char>();
-	enqueue_eval(c, c, pl, C, nullptr, work, nullptr, nullptr, tab.data(), nullptr, sb.X, sb.W);
-	std::vector<char> res(pl.res_bytes());
-	RQC_HIP(hipMemcpyAsync(res.data(), work + pl.off_res, res.size(), hipMemcpyDeviceToHost, c.stream));
-	RQC_HIP(hipStreamSynchronize(c.stream));
-	RQC_HIP(hipGetLastError());
-	EvalResult R;
-	unpack_result(pl, res.data(), R);
+	EvalResult R = run_eval(c, pl, C, nullptr, sb.X, sb.W, nullptr);
 	scale_result(R, (double)pl.N / (double)nsamples);
 	return R;
 }
@@ -3591,6 +3620,7 @@ extern "C" void rqc_release_workspace(void)
 		c.small.release();
 		c.vecs.release();
 		c.ubuf.release();
+		c.io.release();
 	} catch (...) {}
 }
 

@@ -157,6 +157,10 @@ struct EvalResult
 	std::vector<zc> dv, hz;          // ngroups * 16
 	std::vector<double> grad, hvp;   // ngroups * 16
 };
+// table bytes (rounded up to 16) from pinned host memory to the device, in stream order; the source
+// stays as it is until then
+void upload_pinned(Slot& s, void* dst, const void* src, size_t bytes);
+
 // decode the result region (pl.res_bytes() bytes copied from work + pl.off_res)
 void unpack_result(const EvalPlan& pl, const char* res, EvalResult& R);
 

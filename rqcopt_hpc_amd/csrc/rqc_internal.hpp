@@ -43,6 +43,16 @@ struct DeviceBuffer
 	template <typename T> T* as() const { return static_cast<T*>(ptr); }
 };
 
+// grow-only pinned host allocation, read and written by kernels
+struct HostBuffer
+{
+	void* ptr = nullptr;
+	size_t bytes = 0;
+	void reserve(size_t n);
+	void release();
+	template <typename T> T* as() const { return static_cast<T*>(ptr); }
+};
+
 // An execution slot: one HIP stream and the bookkeeping of the evaluations
 // enqueued on it.  Evaluations on different slots share nothing on the device
 // and may run concurrently.
@@ -80,6 +90,7 @@ struct Context : Slot
 	DeviceBuffer vecs;     // uploaded statevectors of the statevector-level API
 	DeviceBuffer ubuf;     // U assembled from a host callback
 	DeviceBuffer samples;  // sample states and trace seeds of stochastic-trace evaluations
+	HostBuffer io;         // tables and results of one call (held until its stream is synchronised)
 	char* scratch = nullptr;   // device address of the static no-allocation scratch array (kScratchBytes)
 
 	double prof_ms[RQC_KERNEL_KINDS] = {0, 0, 0, 0};

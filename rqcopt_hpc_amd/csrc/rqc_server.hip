@@ -159,13 +159,13 @@ static void ensure_pinned(char** p, size_t* cap, size_t n)
 static void run_request(Server& S, Worker& w, Req& r)
 {
 	const EvalPlan& pl = *r.plan;
-	ensure_pinned(&w.h_tab, &w.tab_cap, pl.tab_bytes);
+	ensure_pinned(&w.h_tab, &w.tab_cap, pl.tab_bytes + 16);
 	ensure_pinned(&w.h_res, &w.res_cap, pl.res_bytes());
 	fill_eval_tables(pl, r.C, w.h_tab);
 	char* work = S.arena + r.off;
-	enqueue_eval(*S.dev, w.slot, pl, r.C, r.s->dU, work, nullptr, nullptr, w.h_tab, nullptr);
-	const size_t nres = (r.kind == RQC_EVAL_TARGET) ? sizeof(zc) : pl.res_bytes();
-	RQC_HIP(hipMemcpyAsync(w.h_res, work + pl.off_res, nres, hipMemcpyDeviceToHost, w.slot.stream));
+	// (the results go to pinned memory straight from the last kernel)
+	upload_pinned(w.slot, work + pl.off_tab, w.h_tab, pl.tab_bytes);
+	enqueue_eval(*S.dev, w.slot, pl, r.C, r.s->dU, work, nullptr, w.h_res, nullptr, nullptr);
 	RQC_HIP(hipStreamSynchronize(w.slot.stream));
 	EvalResult R;
 	unpack_result(pl, w.h_res, R);
