@@ -3,11 +3,13 @@
 //
 // A gate alone moves its arrays once (an HVP at 18 qubits: 16 MB forward, 24 MB reverse, 5 and 11 us
 // per launch from the last-level cache, 51 gates 0.89 ms); a pass moves them once for up to 18 gates
-// (4 passes, 0.34 ms; 6 qubits, 15 gates: 0.19 to 0.09 ms, 20 qubits 1.0 ms).  The reverse pass starts
-// at the pass's last state and takes the gates back with G^-1, so that a state is kept per pass
-// instead of per gate.  Two threads own a quad of amplitudes per gate, two rows of every product
-// each: vector FMAs have the rate of the FP64 matrix products here, and the quad needs no operand
-// layout; the outer products go through lane exchanges (wave_sum).
+// (4 passes; 0.34 ms, with host copies taken out 0.31 and the outer products on the matrix cores 0.29).
+// The reverse pass starts at the pass's last state and takes the gates back with G^-1, so that a
+// state is kept per pass instead of per gate.  Two threads of a wave own a quad of amplitudes per
+// gate, two rows of every product each: vector FMAs have the rate of the FP64 matrix products here,
+// and the quad needs no operand layout.  The outer products are matrix products over 16 quads, their
+// operands read again from LDS: as vector products and lane exchanges they took 255 of 563 vector
+// instructions per wave and gate (20 qubits: 930 us against 890, 10 qubits 139 against 130).
 #pragma once
 
 #include "rqc_tile_kernels.hpp"
@@ -33,7 +35,7 @@ constexpr int kStateMats = 64;     // matrix entries of an op
 // LDS: the arrays, two gates' matrices and (reverse) two gates' sums of each wave, both in turn
 constexpr int state_lds_bytes(bool rev)
 {
-	return (rev ? 4 : 2) * kStateArray + 2 * kStateMats * 16 + (rev ? kStateThreads * 8 : 0);
+	return (rev ? 4 : 2) * kStateArray + 2 * kStateMats * 16 + (rev ? 2 * kStateThreads * 8 : 0);
 }
 
 // index bits of the tile bits 0 .. K - 1, then those of the tile number's bits
@@ -56,6 +58,14 @@ __device__ __forceinline__ long state_deposit(const int* bit, int n, unsigned x)
 template <int N> __device__ __forceinline__ double row_value(double v)
 {
 	return __longlong_as_double(__builtin_amdgcn_mov_dpp(__double_as_longlong(v), 0x150 + N, 0xf, 0xf, true));
+}
+// the value of lane + N (mod 16) of each 16 lanes
+template <int N> __device__ __forceinline__ double row_rotate(double v)
+{
+	const long b = __double_as_longlong(v);
+	const unsigned lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffff), 0x120 + N, 0xf, 0xf, true),
+		hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0x120 + N, 0xf, 0xf, true);
+	return __longlong_as_double((long)(((unsigned long)hi << 32) | lo));
 }
 __device__ __forceinline__ zc of_lane(zc v, int n)
 {
@@ -81,12 +91,11 @@ __device__ __forceinline__ void mac_first(zc& s, zc a, zc b, bool first)
 // pass, replaced by those before it in (of, odf) unless null; sums of gate `index` and tile t at
 // part[(index gridDim.x + t) kWidth].
 //
-// At 18 qubits a CU has one tile, two waves per SIMD, and a gate takes 1.4 us forward and 3.4 us
-// reverse: bound by the chain of LDS reads, products, wave sums and two barriers, with the vector
-// units (reverse: 576 FMAs per quad and as many other instructions) busy about half of the time.
-// The gates' matrices come through LDS, loaded a gate ahead, an entry per lane and broadcast inside
-// 16 lanes: from scalar loads, each waiting for the cache, a gate took 2.8 and 5.7 us, and with one
-// thread per quad 2.0 and 4.4.
+// At 18 qubits a CU has one tile, two waves per SIMD, and a gate takes 1.4 us forward and 3.1 us
+// reverse: bound by the chain of LDS reads, products and the barrier.  The gates' matrices come
+// through LDS, loaded a gate ahead, an entry per lane and broadcast inside 16 lanes: from scalar
+// loads, each waiting for the cache, a gate took 2.8 and 5.7 us, and with one thread per quad 2.0
+// and 4.4; four threads per quad (16 waves) gave nothing at 18 qubits and lost 20 % at 20.
 template <bool REV>
 __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* __restrict__ ops, int nops, StateTile T,
 	const zc* a, const zc* da, const zc* f, const zc* df, zc* oa, zc* oda, zc* __restrict__ part)
@@ -94,8 +103,9 @@ __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* 
 	extern __shared__ __align__(16) char lds_raw[];
 	constexpr int A = kStateArray;
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = blockDim.x;
-	// the thread's half of the rows (uniform in a wave) and its quad
-	const int h = __builtin_amdgcn_readfirstlane(2 * wave >= nt / 64 ? 1 : 0), quad = tid & (nt / 2 - 1);
+	// the thread's half of the rows and its quad: a wave owns 32 quads, so that its reads of a quad
+	// precede its writes without a barrier
+	const int h = lane >> 5, quad = 32 * wave + (lane & 31);
 	// (tiles of fewer than 8 qubits: zeros up to a quad per lane)
 	const unsigned ne = 1u << T.K, nz = max(ne, 256u);
 	const long base = state_deposit(T.bit + T.K, T.L - T.K, blockIdx.x), mine = base | state_deposit(T.bit, T.K, tid);
@@ -121,10 +131,10 @@ __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* 
 	int stored = -1;
 	auto store = [&](int j) {
 		if (stored >= 0 && tid < 2 * kWidth) {
-			// double tid of the sums: matrix, row, column, part; the waves of the column's half
-			const int i = (tid & 32) / 2 + 4 * ((tid >> 3) & 3) + 2 * ((tid >> 1) & 1) + (tid & 1), w0 = ((tid >> 2) & 1) * (nt / 128);
+			// double tid of the sums: matrix, row, column, part (lane 16 row + 8 matrix + 4 part + column)
+			const int i = 16 * ((tid >> 3) & 3) + 8 * (tid >> 5) + 4 * (tid & 1) + ((tid >> 1) & 3);
 			double s = 0;
-			for (int w = 0; w < nt / 128; w++) { s += sums[(j & 1) * (kStateThreads / 2) + (w0 + w) * kWidth + i]; }
+			for (int w = 0; w < nt / 64; w++) { s += sums[(j & 1) * kStateThreads + w * 64 + i]; }
 			reinterpret_cast<double*>(part + ((long)stored * gridDim.x + blockIdx.x) * kWidth)[tid] = s;
 		}
 	};
@@ -153,6 +163,13 @@ __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* 
 			x[k] = lds_load_cxd(at[k]);
 			dx[k] = lds_load_cxd(at[k] + A);
 		}
+		auto put_before = [&]() {
+#pragma unroll
+			for (int k = 0; k < 2; k++) {
+				lds_store_cxd(to[k], y[k]);
+				lds_store_cxd(to[k] + A, dy[k]);
+			}
+		};
 		if constexpr (!REV) {
 #pragma unroll
 			for (int r = 0; r < 2; r++) {
@@ -164,7 +181,7 @@ __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* 
 					cmac(dy[r], of_lane(mz, 4 * r + c), x[c]);
 				}
 			}
-			__syncthreads();
+			put_before();
 		} else {
 			const zc mi = lds_load_cxd(by_row + 512), mw = lds_load_cxd(by_row + 768);
 			zc fx[4], dfx[4], u[2], du[2];
@@ -173,6 +190,18 @@ __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* 
 				fx[k] = lds_load_cxd(at[k] + 2 * A);
 				dfx[k] = lds_load_cxd(at[k] + 3 * A);
 			}
+			// the outer products' operands (4 x 4 x 4 matrix products over 16 quads): amplitude lane & 3 of quad
+			// 4 ((lane >> 2) & 3) + (lane >> 4)
+			const int lo = min(o.pi, o.pj), hi = max(o.pi, o.pj);
+			const unsigned mb = state_slot((unsigned)quad_base(32 * wave + (lane & 12) + (lane >> 4), lo, hi)) ^
+				(sj & -(unsigned)(lane & 1)) ^ (si & -(unsigned)((lane >> 1) & 1));
+			const unsigned mo[2] = {mb, mb ^ state_slot((unsigned)quad_base(16, lo, hi))};
+			GateOperands<double, 2> oa, os;
+			auto operand = [&](unsigned at) {
+				const zc v = lds_load_cxd(at), d = lds_load_cxd(at + A);
+				return double4_t{v.x, v.y, d.x, d.y};
+			};
+			for (int n = 0; n < 2; n++) { oa.acc[n] = operand(mo[n] + 2 * A); }
 			// before the gate: G^-1 x and its tangent G^-1 dx - G^-1 Z G^-1 x
 			const bool dzero = o.first != 0;
 #pragma unroll
@@ -187,6 +216,9 @@ __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* 
 				}
 				dy[r] = dzero ? zc{0, 0} : dy[r] - t;
 			}
+			put_before();
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			for (int n = 0; n < 2; n++) { os.acc[n] = operand(mo[n]); }
 			// the adjoint before the gate: G^T f, its tangent G^T df + Z^T f
 #pragma unroll
 			for (int c = 0; c < 2; c++) {
@@ -198,36 +230,19 @@ __global__ __launch_bounds__(kStateThreads, 2) void k_state_pass(const StateOp* 
 					cmac(du[c], of_lane(mz, 4 * r + c), fx[r]);
 				}
 			}
-			__syncthreads();
 #pragma unroll
 			for (int k = 0; k < 2; k++) {
 				lds_store_cxd(to[k] + 2 * A, u[k]);
 				lds_store_cxd(to[k] + 3 * A, du[k]);
 			}
-			// columns 2 h, 2 h + 1 of the outer products
-			double v[kWidth];
-#pragma unroll
-			for (int r = 0; r < 4; r++) {
-#pragma unroll
-				for (int c = 0; c < 2; c++) {
-					zc g, d;
-					mac_first(g, fx[r], y[c], true);
-					mac_first(d, fx[r], dy[c], true);
-					cmac(d, dfx[r], y[c]);
-					v[2 * (2 * r + c)] = g.x;
-					v[2 * (2 * r + c) + 1] = g.y;
-					v[16 + 2 * (2 * r + c)] = d.x;
-					v[16 + 2 * (2 * r + c) + 1] = d.y;
-				}
+			double4_t c = {0, 0, 0, 0};
+			outer44<2>(os, oa, c);
+			for (int n = 0; n < 4; n++) {
+				c[n] += row_rotate<8>(c[n]);
+				c[n] += row_rotate<4>(c[n]);
 			}
-			const double s = wave_sum<kWidth>(v);
-			if ((lane & 1) == 0) { sums[(j & 1) * (kStateThreads / 2) + wave * kWidth + wave_sum_index<kWidth>(lane)] = s; }
+			sums[(j & 1) * kStateThreads + tid] = (lane & 8) ? ((lane & 4) ? c[3] : c[2]) : ((lane & 4) ? c[1] : c[0]);
 			stored = o.index;
-		}
-#pragma unroll
-		for (int k = 0; k < 2; k++) {
-			lds_store_cxd(to[k], y[k]);
-			lds_store_cxd(to[k] + A, dy[k]);
 		}
 		if (tid < kStateMats) { put(j + 1, ahead); }
 	}
