@@ -1885,7 +1885,7 @@ struct StateSums
 	{
 		if (ngates == 0) { return; }
 		LaunchTimer lt(c, RQC_KERNEL_OTHER);
-		k_reduce_gates<<<dim3(ngates, kWidth), kBlock, 0, c.stream>>>(part, (int)grid, out != nullptr ? out : acc);
+		k_reduce_gates<<<dim3(ngates, kWidth / 8), kBlock, 0, c.stream>>>(part, (int)grid, out != nullptr ? out : acc);
 	}
 };
 

@@ -479,19 +479,24 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(const zc* __restrict
 	if (threadIdx.x == 0) { acc[e] += res[0]; }
 }
 
-// out[x * kWidth + y] = sum over the parts p of partial[(x * nparts + p) * kWidth + y] in a fixed
-// order: the sums of gate x of a sweep over one statevector, all gates in one launch
+// out[x * kWidth + e] = sum over the parts p of partial[(x * nparts + p) * kWidth + e] in a fixed
+// order: the sums of gate x of a sweep over one statevector, all gates in one launch; eight entries
+// (128 bytes of a part) and 32 slices of the parts per workgroup
 __global__ __launch_bounds__(kBlock) void k_reduce_gates(const zc* __restrict__ partial, int nparts, zc* __restrict__ out)
 {
-	const int e = blockIdx.y;
-	const zc* p = partial + (long)blockIdx.x * nparts * kWidth;
+	__shared__ zc red[32][8];
+	const int q = threadIdx.x >> 3, e = threadIdx.x & 7;
+	const zc* p = partial + (long)blockIdx.x * nparts * kWidth + 8 * blockIdx.y + e;
 	zc s = {0, 0};
-	for (int i = threadIdx.x; i < nparts; i += kBlock) { s += p[(long)i * kWidth + e]; }
-	zc r[1] = {s};
-	__shared__ zc res[1];
-	block_sum_store<1>(r, res);
+#pragma unroll 4
+	for (int i = q; i < nparts; i += 32) { s += p[(long)i * kWidth]; }
+	red[q][e] = s;
 	__syncthreads();
-	if (threadIdx.x == 0) { out[(long)blockIdx.x * kWidth + e] = res[0]; }
+	if (threadIdx.x < 8) {
+		zc r = red[0][e];
+		for (int i = 1; i < 32; i++) { r += red[i][e]; }
+		out[(long)blockIdx.x * kWidth + 8 * blockIdx.y + e] = r;
+	}
 }
 
 // X[a * B + c] = (a == b0 + c)
