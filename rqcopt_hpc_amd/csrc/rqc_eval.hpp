@@ -161,7 +161,7 @@ struct EvalResult
 // stays as it is until then
 void upload_pinned(Slot& s, void* dst, const void* src, size_t bytes);
 
-// decode the result region (pl.res_bytes() bytes copied from work + pl.off_res)
+// decode the result region (pl.res_bytes() bytes, as k_finalize wrote them)
 void unpack_result(const EvalPlan& pl, const char* res, EvalResult& R);
 
 // the device-resident dense target of rqc_device_ufunc (checked; L < 0 skips the qubit check)
