@@ -1333,7 +1333,7 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 		}
 		{
 			LaunchTimer lt(s, RQC_KERNEL_OTHER);
-			k_reduce_partials<<<1, kBlock, 0, s.stream>>>(tpart, (int)gtr, 1, d_acc, skip);
+			k_reduce_partials<<<1, kBlock, 0, s.stream>>>(tpart, (int)gtr, 1, d_acc, skip, blk > 0 ? 1 : 0);
 		}
 		if (mode == Mode::Target) { continue; }
 		int cur = 0;
@@ -1362,11 +1362,14 @@ static void run_tiles(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* 
 			}
 			if (p == red->pass) {
 				LaunchTimer lt(s, RQC_KERNEL_OTHER);
+				// (few parts: in one stage)
+				const bool chunks = nparts > kReduceDirect;
 				const int nch = (int)std::min<long>(kReduceChunks, nparts);
 				TileGates tg;
 				std::copy_n(tp.order.begin() + red->x0, red->ng, tg.k);
-				k_tile_reduce_chunks<<<dim3(red->ng, nch), 256, 0, s.stream>>>(mpart, nparts, nch, cpart, skip);
-				k_tile_reduce<<<red->ng, 256, 0, s.stream>>>(cpart, nch, tg, rmats + 32L * red->x0, dual ? 1 : 0, d_acc, skip);
+				if (chunks) { k_tile_reduce_chunks<<<dim3(red->ng, nch), 256, 0, s.stream>>>(mpart, nparts, nch, cpart, skip); }
+				k_tile_reduce<<<red->ng, 256, 0, s.stream>>>(chunks ? cpart : mpart, chunks ? nch : nparts, tg, rmats + 32L * red->x0,
+					dual ? 1 : 0, d_acc, blk > 0 ? 1 : 0, skip);
 				++red;
 			}
 			cur = 1 - cur;
@@ -1548,7 +1551,7 @@ void enqueue_eval(const Context& dev, Slot& s, const EvalPlan& pl, const Circuit
 	s.last_logC = pl.tiles ? pl.tile_logC : 0;
 	s.last_gmax = pl.tiles ? pl.gmax : 0;
 	s.last_passes = pl.passes;
-	if (!pl.cyc) {
+	if (!pl.tiles) {   // (the sweeps of the first column block store their sums)
 		LaunchTimer lt(s, RQC_KERNEL_OTHER);
 		k_fill_zero<<<nblocks((long)pl.n_acc), kBlock, 0, s.stream>>>(acc, (long)pl.n_acc, skip);
 	}

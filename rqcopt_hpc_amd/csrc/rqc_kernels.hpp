@@ -464,9 +464,9 @@ __global__ __launch_bounds__(kBlock) void k_gram_hermitian(const zc* __restrict_
 	}
 }
 
-// acc[e] += sum_p partial[p * width + e] in a fixed order; one workgroup per e
+// acc[e] += (or, without add, =) sum_p partial[p * width + e] in a fixed order; one workgroup per e
 __global__ __launch_bounds__(kBlock) void k_reduce_partials(const zc* __restrict__ partial, int nparts, int width,
-	zc* __restrict__ acc, const int* skip)
+	zc* __restrict__ acc, const int* skip, int add = 1)
 {
 	if (skipped(skip)) { return; }
 	const int e = blockIdx.x;
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(const zc* __restrict
 	__shared__ zc res[1];
 	block_sum_store<1>(r, res);
 	__syncthreads();
-	if (threadIdx.x == 0) { acc[e] += res[0]; }
+	if (threadIdx.x == 0) { acc[e] = add ? acc[e] + res[0] : res[0]; }
 }
 
 // out[x * kWidth + e] = sum over the parts p of partial[(x * nparts + p) * kWidth + e] in a fixed

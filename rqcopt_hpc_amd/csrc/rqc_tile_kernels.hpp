@@ -1451,6 +1451,9 @@ struct TileGates
 // [c * ceil(nparts / nchunks), ...) in order, for every gate j (grid ng x nchunks);
 // out has the partials' layout with nchunks parts.
 constexpr int kReduceChunks = 16;
+// parts that k_tile_reduce sums by itself (128 parts, block encoding of 10 qubits and 7 layers: 211 us,
+// in two stages 220)
+constexpr int kReduceDirect = 128;
 
 __global__ __launch_bounds__(256) void k_tile_reduce_chunks(const double* __restrict__ partial, long nparts,
 	int nchunks, double* __restrict__ out, const int* skip)
@@ -1465,8 +1468,8 @@ __global__ __launch_bounds__(256) void k_tile_reduce_chunks(const double* __rest
 }
 
 // Sum of the outer-product partials over all parts in a fixed order, decoded
-// into 16 gradient and (DUAL) 16 HVP entries per gate and added to
-// acc[1 + 32 * gate + e].  One workgroup of 256 threads per gate of the reduction.
+// into 16 gradient and (DUAL) 16 HVP entries per gate and added to (or, without
+// add, stored in) acc[1 + 32 * gate + e].  One workgroup of 256 threads per gate of the reduction.
 // The partials pair the adjoint at the gate input (phi_in = G^T phi,
 // dphi_in = G^T dphi + Z^T phi) with the state before the gate; component
 // 4 (2 s + p) + r is array s (primary / tangent; plain sweeps: the quad of the
@@ -1476,13 +1479,14 @@ __global__ __launch_bounds__(256) void k_tile_reduce_chunks(const double* __rest
 //   grad = Q A1,   hess = Q (A2 + A3) + W^T A1   (W = -G^-1 Z G^-1);
 // rm holds Q and W^T of the gates (FP64, 32 entries per gate).
 __global__ __launch_bounds__(256) void k_tile_reduce(const double* __restrict__ partial, long nparts,
-	const TileGates gk, const zc* __restrict__ rm, int dual, zc* __restrict__ acc, const int* skip)
+	const TileGates gk, const zc* __restrict__ rm, int dual, zc* __restrict__ acc, int add, const int* skip)
 {
 	if (skipped(skip)) { return; }
 	__shared__ double Dm[16][16];
 	__shared__ zc A[2][16];
 	const int j = blockIdx.x, i = threadIdx.x;
 	double s = 0;
+#pragma unroll 8
 	for (long p = 0; p < nparts; p++) { s += partial[(j * nparts + p) * 256 + i]; }
 	Dm[i >> 4][i & 15] = s;
 	__syncthreads();
@@ -1505,17 +1509,16 @@ __global__ __launch_bounds__(256) void k_tile_reduce(const double* __restrict__ 
 		A[which][4 * r + c] = zc{re, im};
 	}
 	__syncthreads();
-	if (i < 32 && (dual || !which)) {
+	if (i < 32) {
 		const zc* Q = rm + 32L * j;
 		const zc* WT = Q + 16;
 		zc v = {0, 0};
 		for (int k = 0; k < 4; k++) { cmac(v, Q[4 * r + k], A[which][4 * k + c]); }
-		if (which) {
+		if (which && dual) {
 			for (int k = 0; k < 4; k++) { cmac(v, WT[4 * r + k], A[0][4 * k + c]); }
 		}
 		zc* a = acc + 1 + 32L * gk.k[j] + 16 * which + 4 * r + c;
-		a->x += v.x;
-		a->y += v.y;
+		*a = add ? *a + v : v;
 	}
 }
 
