@@ -24,7 +24,8 @@ struct rqc_target;  /* opaque: a dense 2^L x 2^L complex128 U in device memory *
 enum rqc_precision
 {
 	RQC_PRECISION_FP64  = 0,  /* complex FP64 sweeps and reductions */
-	RQC_PRECISION_MIXED = 1,  /* complex FP32 sweeps, FP64 reductions, FP64 projection */
+	RQC_PRECISION_MIXED = 1,  /* complex FP32 arrays and gates; products in FP64 (dense targets) or FP32
+	                             (column blocks); FP64 reductions and projection */
 };
 
 enum rqc_sweep_engine
