@@ -19,7 +19,6 @@
 #include <algorithm>
 #include <cstring>
 #include <functional>
-#include <list>
 #include <map>
 #include <string>
 #include <set>
@@ -31,6 +30,7 @@
 #include "rqc_tile_kernels.hpp"
 #include "rqc_cyc_kernels.hpp"
 #include "rqc_state_kernels.hpp"
+#include "rqc_plan_cache.hpp"
 #include "mat4.hpp"
 #include "rqcopt/gate.h"
 #include "rqcopt/statevector.h"
@@ -528,33 +528,6 @@ static std::vector<Pass> plan_passes(const Circuit& C, int K, int gmax)
 	}
 	return out;
 }
-
-// Plans by circuit structure.  A program evaluates one structure many times with new gates; the
-// search costs up to a few milliseconds, as much as an evaluation of 10 qubits.  The last kMost
-// plans are kept (host memory only); the key holds the whole structure, nothing of the gates.
-template <typename P>
-class PlanCache
-{
-public:
-	std::shared_ptr<const P> get(const std::vector<int>& key, const std::function<std::shared_ptr<const P>()>& make)
-	{
-		std::lock_guard<std::mutex> lk(mu_);
-		for (auto it = plans_.begin(); it != plans_.end(); ++it) {
-			if (it->first == key) {
-				plans_.splice(plans_.begin(), plans_, it);
-				return it->second;
-			}
-		}
-		plans_.emplace_front(key, make());
-		if (plans_.size() > kMost) { plans_.pop_back(); }
-		return plans_.front().second;
-	}
-
-private:
-	static constexpr size_t kMost = 64;
-	std::mutex mu_;
-	std::list<std::pair<std::vector<int>, std::shared_ptr<const P>>> plans_;
-};
 
 static std::vector<int> structure_ints(const Circuit& C, std::initializer_list<int> head)
 {

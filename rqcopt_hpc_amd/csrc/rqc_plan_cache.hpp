@@ -1,0 +1,55 @@
+// Plans by circuit structure (host).  A program evaluates one structure many times with new gates; the
+// search costs up to a few milliseconds, as much as an evaluation of 10 qubits.  The last kMost plans
+// are kept (host memory only); the key holds the whole structure, nothing of the gates.
+#pragma once
+
+#include <cstddef>
+#include <functional>
+#include <list>
+#include <memory>
+#include <mutex>
+#include <utility>
+#include <vector>
+
+namespace rqc {
+
+template <typename P>
+class PlanCache
+{
+public:
+	// Plans are made outside the lock, so that a thread with a new structure does not keep others from
+	// theirs; of two threads that make the same plan the first one's is kept.
+	std::shared_ptr<const P> get(const std::vector<int>& key, const std::function<std::shared_ptr<const P>()>& make)
+	{
+		if (auto p = find(key)) { return p; }
+		auto made = make();
+		std::lock_guard<std::mutex> lk(mu_);
+		if (auto p = find_locked(key)) { return p; }
+		plans_.emplace_front(key, made);
+		if (plans_.size() > kMost) { plans_.pop_back(); }
+		return made;
+	}
+
+private:
+	static constexpr size_t kMost = 64;
+	std::mutex mu_;
+	std::list<std::pair<std::vector<int>, std::shared_ptr<const P>>> plans_;
+
+	std::shared_ptr<const P> find(const std::vector<int>& key)
+	{
+		std::lock_guard<std::mutex> lk(mu_);
+		return find_locked(key);
+	}
+	std::shared_ptr<const P> find_locked(const std::vector<int>& key)
+	{
+		for (auto it = plans_.begin(); it != plans_.end(); ++it) {
+			if (it->first == key) {
+				plans_.splice(plans_.begin(), plans_, it);
+				return it->second;
+			}
+		}
+		return nullptr;
+	}
+};
+
+}  // namespace rqc
