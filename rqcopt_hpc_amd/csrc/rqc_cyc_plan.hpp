@@ -29,6 +29,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "rqc_pass_search.hpp"
+
 namespace rqc {
 
 constexpr int kCycOps = 8;     // most two-sided gate products of a launch's job
@@ -97,10 +99,18 @@ struct SideOp
 	int a = -1, ma = 0, b = -1, mb = 0, rec = -1;   // slots and table matrices of the two factors
 };
 
+// colours of a step's row and column bits by qubit bit
+struct Colouring
+{
+	std::vector<int> r, c;   // indexed by qubit bit, 0 outside the tile
+	int beta(int id, int L) const { return id >= L ? r[id - L] : c[id] << 2; }
+};
+
 struct Step
 {
-	std::vector<int> rows, cols;   // qubit bits of the tile
+	std::vector<int> rows, cols;   // qubit bits of the tile, ascending
 	std::vector<SideOp> ops;
+	Colouring col;
 	unsigned fout = 0;             // free qubits of its output
 	bool conj = false;
 	int flags = 0;
@@ -134,27 +144,25 @@ inline std::vector<int> colours(const std::vector<int>& q, const std::vector<std
 	return col;
 }
 
-// rank of n <= 4 vectors of GF(2)^4
-inline int rank4(std::array<int, 4> v, int n)
+// The span of vectors of GF(2)^4 as a bit set of its 16 elements (1: the zero vector alone)
+inline unsigned span_add(unsigned span, int v)
 {
-	int r = 0;
-	for (int bit = 0; bit < 4 && r < n; bit++) {
-		int p = r;
-		while (p < n && !((v[p] >> bit) & 1)) { p++; }
-		if (p == n) { continue; }
-		std::swap(v[r], v[p]);
-		for (int i = r + 1; i < n; i++) { if ((v[i] >> bit) & 1) { v[i] ^= v[r]; } }
-		r++;
-	}
-	return r;
+	if ((span >> v) & 1) { return span; }
+	unsigned t = span;
+	if (v & 1) { t = ((t & 0x5555) << 1) | ((t >> 1) & 0x5555); }
+	if (v & 2) { t = ((t & 0x3333) << 2) | ((t >> 2) & 0x3333); }
+	if (v & 4) { t = ((t & 0x0f0f) << 4) | ((t >> 4) & 0x0f0f); }
+	if (v & 8) { t = ((t & 0x00ff) << 8) | ((t >> 8) & 0x00ff); }
+	return span | t;
 }
+inline int span_rank(unsigned span) { return __builtin_ctz((unsigned)__builtin_popcount(span)); }
 
 // Bank conflicts of 16-byte LDS accesses by the XOR-linear slots d0 .. d5 of the lane index bits
 // (measured): a read's 16-lane phases are the lanes with one parity of bits 2, 3, 4 (lane bit 5
-// apart), free of conflicts iff d0, d1, d2 + d3, d2 + d4 are independent mod 16 slots; a write takes
-// 8 consecutive lanes at half the rate, at full speed iff d0, d1, d2 have rank 2 mod 8 slots.
-inline int cyc_read_rank(int d0, int d1, int d2, int d3, int d4) { return rank4({d0, d1, d2 ^ d3, d2 ^ d4}, 4); }
-inline int cyc_write_rank(int d0, int d1, int d2) { return std::min(2, rank4({d0 & 7, d1 & 7, d2 & 7, 0}, 3)); }
+// apart), free of conflicts iff d0, d1, d2 + d3, d2 + d4 are independent mod 16 slots (the read's
+// rank, 4); a write takes 8 consecutive lanes at half the rate, at full speed iff d0, d1, d2 have
+// rank 2 mod 8 slots.
+inline int cyc_write_rank(int d0, int d1, int d2) { return std::min(2, span_rank(span_add(span_add(span_add(1, d0 & 7), d1 & 7), d2 & 7))); }
 
 // the combination of four independent vectors of GF(2)^4 that gives v
 inline int cyc_combination(const int* basis, int v)
@@ -167,124 +175,30 @@ inline int cyc_combination(const int* basis, int v)
 	return 0;
 }
 
-// colours of a step's row and column bits by qubit bit
-struct Colouring
-{
-	std::vector<int> r, c;   // indexed by qubit bit, 0 outside the tile
-	int beta(int id, int L) const { return id >= L ? r[id - L] : c[id] << 2; }
-};
-
 }  // namespace cyc_detail
 
-// Passes of the circuit (gate k on qubit bits bi[k], bj[k]): a beam search like the tile passes'
-// (plan_passes), every pass a set of K qubits and the ready gates inside it, at most gmax.  Among
-// the plans with the fewest passes found it takes the one whose successive passes share qubits
-// best (two shared qubits are the four index bits of a 256-byte run that both launches move
-// whole) and whose first pass holds the lowest qubit bits (runs of U's rows).  Qubits that a pass
-// does not need are filled up with its neighbours'.
+// Passes of the circuit (gate k on qubit bits bi[k], bj[k]), at most gmax gates each.  Among the plans
+// with the fewest passes found the search takes the one whose successive passes share qubits best (two
+// shared qubits are the four index bits of a 256-byte run that both launches move whole) and whose first
+// pass holds the lowest qubit bits (runs of U's rows).  Qubits that a pass does not need are filled up
+// with its neighbours'.
 inline std::vector<CycPass> plan_cyc_passes(int L, const std::vector<int>& bi, const std::vector<int>& bj, int K, int gmax)
 {
-	const int G = (int)bi.size();
-	std::vector<unsigned> gm(G);
-	std::vector<int> prev_i(G, -1), prev_j(G, -1), last(L, -1);
-	for (int k = 0; k < G; k++) {
-		gm[k] = (1u << bi[k]) | (1u << bj[k]);
-		prev_i[k] = last[bi[k]];
-		prev_j[k] = last[bj[k]];
-		last[bi[k]] = last[bj[k]] = k;
-	}
-	const size_t width = (G <= 256) ? 32 : (G <= 2048) ? 4 : 1;
-	struct State
-	{
-		std::vector<char> done;
-		int ndone = 0, from = 0, pen = 0;   // gates before `from` are done
-		std::vector<std::vector<int>> passes;
-		std::vector<unsigned> used;
-	};
-	auto penalty = [&](const State& st, unsigned u) {
-		if (st.used.empty()) {
+	PassSearch S{L, K, gmax, {}, false, true};
+	for (size_t k = 0; k < bi.size(); k++) { S.gm.push_back((1u << bi[k]) | (1u << bj[k])); }
+	const std::vector<FoundPass> plan = search_passes(S, [&](unsigned last, unsigned u) {
+		if (last == 0) {
 			int run = 0;
 			while (run < 3 && ((u >> run) & 1)) { run++; }
 			return std::max(0, 3 - run - (K - __builtin_popcount(u)));
 		}
-		const unsigned p = st.used.back();
-		const int ov = __builtin_popcount(p & u) + 2 * K - __builtin_popcount(p) - __builtin_popcount(u);
+		const int ov = __builtin_popcount(last & u) + 2 * K - __builtin_popcount(last) - __builtin_popcount(u);
 		return ov >= 2 ? 0 : ov == 1 ? 2 : 5;
-	};
-	std::vector<State> beam(1);
-	beam[0].done.assign(G, 0);
-	State plan;
-	bool finished = false;
-	std::vector<char> taken(G);
-	while (!beam.empty() && !finished) {
-		std::vector<State> next;
-		for (const State& st : beam) {
-			std::vector<unsigned> cands;
-			if (K >= L) { cands.push_back((1u << L) - 1); }
-			else {
-				for (int s = 0; s < L; s++) {
-					unsigned m = 0;
-					for (int t = 0; t < K; t++) { m |= 1u << (s + t) % L; }
-					cands.push_back(m);
-				}
-				unsigned m = 0;
-				for (int k = st.from; k < G; k++) {
-					if (st.done[k] || (prev_i[k] >= 0 && !st.done[prev_i[k]]) || (prev_j[k] >= 0 && !st.done[prev_j[k]])) { continue; }
-					if (__builtin_popcount(m | gm[k]) <= K) { m |= gm[k]; }
-				}
-				cands.push_back(m);
-			}
-			for (unsigned m : cands) {
-				std::vector<int> lst;
-				unsigned u = 0;
-				std::fill(taken.begin() + st.from, taken.end(), 0);
-				for (int k = st.from; k < G && (int)lst.size() < gmax; k++) {
-					if (st.done[k] || (gm[k] & ~m) != 0) { continue; }
-					auto ok = [&](int p) { return p < 0 || st.done[p] || taken[p]; };
-					if (!ok(prev_i[k]) || !ok(prev_j[k])) { continue; }
-					taken[k] = 1;
-					lst.push_back(k);
-					u |= gm[k];
-				}
-				if (lst.empty()) { continue; }
-				State t;
-				t.done = st.done;
-				for (int k : lst) { t.done[k] = 1; }
-				t.ndone = st.ndone + (int)lst.size();
-				t.pen = st.pen + penalty(st, u);
-				for (t.from = st.from; t.from < G && t.done[t.from]; ) { t.from++; }
-				if (t.ndone == G) {
-					if (!finished || t.pen < plan.pen) {
-						t.passes = st.passes;
-						t.used = st.used;
-						t.passes.push_back(lst);
-						t.used.push_back(u);
-						plan = std::move(t);
-						finished = true;
-					}
-					continue;
-				}
-				bool dup = false;
-				for (size_t i = 0; i < next.size() && !dup; i++) {
-					dup = next[i].ndone == t.ndone && next[i].used.back() == u && next[i].pen <= t.pen && next[i].done == t.done;
-				}
-				if (dup) { continue; }
-				t.passes = st.passes;
-				t.used = st.used;
-				t.passes.push_back(std::move(lst));
-				t.used.push_back(u);
-				next.push_back(std::move(t));
-			}
-		}
-		std::stable_sort(next.begin(), next.end(), [](const State& a, const State& b) {
-			return a.ndone != b.ndone ? a.ndone > b.ndone : a.pen < b.pen;
-		});
-		if (next.size() > width) { next.resize(width); }
-		beam = std::move(next);
-	}
+	});
 	// fill the passes' sets up to K qubits: the neighbours' first (and the lowest bits for the first)
-	const int P = (int)plan.passes.size();
-	std::vector<unsigned> q = plan.used;
+	const int P = (int)plan.size();
+	std::vector<unsigned> q;
+	for (const FoundPass& p : plan) { q.push_back(p.used); }
 	for (int p = 0; p < P; p++) {
 		auto fill = [&](unsigned from) {
 			for (int b = 0; b < L && __builtin_popcount(q[p]) < K; b++) { if ((from >> b) & 1) { q[p] |= 1u << b; } }
@@ -299,16 +213,54 @@ inline std::vector<CycPass> plan_cyc_passes(int L, const std::vector<int>& bi, c
 	std::vector<CycPass> out;
 	for (int p = 0; p < P; p++) {
 		CycPass c;
-		c.slots = plan.passes[p];
+		c.slots = plan[p].gates;
 		for (int b = 0; b < L; b++) { if ((q[p] >> b) & 1) { c.q.push_back(b); } }
 		out.push_back(c);
 	}
 	return out;
 }
 
-// bi, bj: qubit bits of slot x's wires (the more significant gate index first); with target only,
-// the forward launches run to the end and the last one sums the trace
-inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, const std::vector<int>& bi,
+inline unsigned cyc_qubits(const std::vector<int>& q)
+{
+	unsigned m = 0;
+	for (int b : q) { m |= 1u << b; }
+	return m;
+}
+
+// passes multiplied from the left: the split with the least work, by the conjugation work that the
+// shrinking free sets leave
+inline int cyc_split(int L, int K, const std::vector<CycPass>& passes, bool target_only)
+{
+	const int P = (int)passes.size();
+	if (target_only) { return (P + 1) / 2; }
+	// the work of every pass on either side: log2 of its tiles counts the bits outside the tile, and
+	// a qubit that is not free and outside the tile's rows and columns once
+	std::vector<double> left(P + 1, 0), right(P + 1, 0);   // of the first n, of the last n passes
+	for (int side = 0; side < 2; side++) {
+		unsigned f = 0;
+		for (int i = 0; i < P; i++) {
+			const CycPass& p = passes[side == 0 ? i : P - 1 - i];
+			const unsigned q = cyc_qubits(p.q);
+			const int gens = (L - __builtin_popcount(q)) + __builtin_popcount(f & ~q);
+			(side == 0 ? left : right)[i + 1] = (side == 0 ? left : right)[i] +
+				((double)p.slots.size() + 4.0) * (double)(1UL << gens);
+			f |= q;
+		}
+	}
+	int m = 0;
+	double best = -1;
+	for (int s = 0; s <= P; s++) {
+		double w = left[s];
+		w += right[P - s];
+		w += std::max(s, P - s) * 2.0 * (double)(1UL << (2 * (L - K)));
+		if (best < 0 || w < best) { best = w; m = s; }
+	}
+	return m;
+}
+
+// bi, bj: qubit bits of slot x's wires (the more significant gate index first); m: cyc_split's; with
+// target only, the forward launches run to the end and the last one sums the trace
+inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, int m, const std::vector<int>& bi,
 	const std::vector<int>& bj, bool target_only, bool dual, int matG, int matGinv)
 {
 	using namespace cyc_detail;
@@ -317,39 +269,7 @@ inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, c
 	plan.L = L;
 	plan.K = K;
 	plan.up.assign(bi.size(), 0);
-	auto qmask = [](const std::vector<int>& q) { unsigned m = 0; for (int b : q) { m |= 1u << b; } return m; };
-	// log2 of a step's tiles: bits outside the tile; a qubit that is not free and outside the
-	// tile's rows and columns counts once
-	auto gens = [&](unsigned r, unsigned c, unsigned fout) {
-		int n = 0;
-		for (int b = 0; b < L; b++) {
-			const unsigned m = 1u << b;
-			const bool ir = r & m, ic = c & m;
-			if (ir && ic) { continue; }
-			n += (ir || ic) ? 1 : (fout & m) ? 2 : 1;
-		}
-		return n;
-	};
-	// split: the conjugation work left by the shrinking free sets
-	int m = (P + 1) / 2;
-	if (!target_only) {
-		double best = -1;
-		for (int s = 0; s <= P; s++) {
-			double w = 0;
-			for (int side = 0; side < 2; side++) {
-				const int n = side == 0 ? s : P - s;
-				unsigned f = 0;
-				for (int i = 0; i < n; i++) {
-					const CycPass& p = passes[side == 0 ? i : P - 1 - i];
-					const unsigned q = qmask(p.q);
-					w += ((double)p.slots.size() + 4.0) * (double)(1UL << gens(q, q, f));
-					f |= q;
-				}
-			}
-			w += std::max(s, P - s) * 2.0 * (double)(1UL << (2 * (L - K)));
-			if (best < 0 || w < best) { best = w; m = s; }
-		}
-	}
+	auto qmask = [](const std::vector<int>& q) { return cyc_qubits(q); };
 	// steps
 	std::vector<Step> fwd, down, up;
 	const int F = std::max(m, P - m);
@@ -429,21 +349,21 @@ inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, c
 		for (int b : s.cols) { t[b] = 1; }
 		return t;
 	};
-	auto colour = [&](const Step& s) {
-		Colouring c;
-		c.r.assign(L, 0);
-		c.c.assign(L, 0);
-		std::vector<std::pair<int, int>> er, ec;
-		for (const SideOp& o : s.ops) {
-			const int ra = o.a >= 0 ? o.a : s.conj ? o.rec : -1, cb = o.b >= 0 ? o.b : s.conj ? o.rec : -1;
-			if (ra >= 0) { er.emplace_back(bi[ra], bj[ra]); }
-			if (cb >= 0) { ec.emplace_back(bi[cb], bj[cb]); }
+	for (auto* steps : {&fwd, &down, &up}) {
+		for (Step& s : *steps) {
+			s.col.r.assign(L, 0);
+			s.col.c.assign(L, 0);
+			std::vector<std::pair<int, int>> er, ec;
+			for (const SideOp& o : s.ops) {
+				const int ra = o.a >= 0 ? o.a : s.conj ? o.rec : -1, cb = o.b >= 0 ? o.b : s.conj ? o.rec : -1;
+				if (ra >= 0) { er.emplace_back(bi[ra], bj[ra]); }
+				if (cb >= 0) { ec.emplace_back(bi[cb], bj[cb]); }
+			}
+			const auto cr = colours(s.rows, er), cc = colours(s.cols, ec);
+			for (size_t i = 0; i < s.rows.size(); i++) { s.col.r[s.rows[i]] = cr[i]; }
+			for (size_t i = 0; i < s.cols.size(); i++) { s.col.c[s.cols[i]] = cc[i]; }
 		}
-		const auto cr = colours(s.rows, er), cc = colours(s.cols, ec);
-		for (size_t i = 0; i < s.rows.size(); i++) { c.r[s.rows[i]] = cr[i]; }
-		for (size_t i = 0; i < s.cols.size(); i++) { c.c[s.cols[i]] = cc[i]; }
-		return c;
-	};
+	}
 	// memory bit order (id -> position) that step s leaves for its successors (the first primary)
 	auto next_layout = [&](const Step& s, const std::vector<const Step*>& succ, const std::vector<int>& pin) {
 		const auto ts = tile_ids(s);
@@ -459,25 +379,38 @@ inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, c
 		for (auto* v : {&common, &mid, &rest}) { std::sort(v->begin(), v->end(), by_pin); }
 		// the lowest five: stores of s read LDS, and loads of its successors write it, by these bits
 		if (common.size() >= 4) {
-			const Colouring cs = colour(s);
-			std::vector<Colouring> cn;
-			for (auto* n : succ) { cn.push_back(colour(*n)); }
 			const std::vector<int>& five = common.size() >= 5 ? common : mid;
 			int best = -1;
 			std::array<int, 5> pick = {};
-			const int n = std::min<int>((int)common.size(), 8);
-			for (int a = 0; a < n && best < 100; a++) for (int b = 0; b < n && best < 100; b++) for (int c = 0; c < n && best < 100; c++) {
-				for (int d = 0; d < n && best < 100; d++) {
-					if (a == b || a == c || a == d || b == c || b == d || c == d) { continue; }
-					for (int e = 0; e < (int)std::min<size_t>(five.size(), 8); e++) {
-						if (&five == &common && (e == a || e == b || e == c || e == d)) { continue; }
-						const int id[5] = {common[a], common[b], common[c], common[d], five[e]};
-						// (bit five may lie outside the tile of s: no LDS term)
-						int sc = 8 * cyc_read_rank(cs.beta(id[0], L), cs.beta(id[1], L), cs.beta(id[2], L), cs.beta(id[3], L), cs.beta(id[4], L));
-						int w = 2;
-						for (auto& k : cn) { w = std::min(w, cyc_write_rank(k.beta(id[0], L), k.beta(id[1], L), k.beta(id[2], L))); }
-						sc = sc + 2 * w + (sc == 32 && w == 2 ? 100 : 0);
-						if (sc > best) { best = sc; for (int i = 0; i < 5; i++) { pick[i] = id[i]; } }
+			const int n = std::min<int>((int)common.size(), 8), n5 = (int)std::min<size_t>(five.size(), 8);
+			// bank terms of the candidates in the tile of s (a fifth bit outside it has none) and in its successors'
+			int cs[8], c5[8], cn[2][8];
+			for (int i = 0; i < n; i++) {
+				cs[i] = s.col.beta(common[i], L);
+				for (size_t k = 0; k < succ.size(); k++) { cn[k][i] = succ[k]->col.beta(common[i], L); }
+			}
+			for (int i = 0; i < n5; i++) { c5[i] = s.col.beta(five[i], L); }
+			// score: 8 times the stores' read rank and 2 times the loads' write rank, 100 more if both are full
+			// (the search ends there); a branch that cannot gain is left out
+			auto most = [](int rank, int w) { return rank >= 4 ? 32 + 2 * w + (w == 2 ? 100 : 0) : 8 * rank + 2 * w; };
+			for (int a = 0; a < n && best < 100; a++) for (int b = 0; b < n && best < 100; b++) {
+				if (a == b) { continue; }
+				const unsigned ab = span_add(span_add(1, cs[a]), cs[b]);
+				if (most(span_rank(ab) + 2, 2) <= best) { continue; }
+				for (int c = 0; c < n && best < 100; c++) {
+					if (c == a || c == b) { continue; }
+					int w = 2;
+					for (size_t k = 0; k < succ.size(); k++) { w = std::min(w, cyc_write_rank(cn[k][a], cn[k][b], cn[k][c])); }
+					if (most(span_rank(ab) + 2, w) <= best) { continue; }
+					for (int d = 0; d < n && best < 100; d++) {
+						if (d == a || d == b || d == c) { continue; }
+						const unsigned abd = span_add(ab, cs[c] ^ cs[d]);
+						if (most(span_rank(abd) + 1, w) <= best) { continue; }
+						for (int e = 0; e < n5; e++) {
+							if (&five == &common && (e == a || e == b || e == c || e == d)) { continue; }
+							const int sc = most(span_rank(span_add(abd, cs[c] ^ c5[e])), w);
+							if (sc > best) { best = sc; pick = {common[a], common[b], common[c], common[d], five[e]}; }
+						}
 					}
 				}
 			}
@@ -497,7 +430,7 @@ inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, c
 	const int nb = 2 * K;
 	auto build_job = [&](const Step& s, const std::vector<int>& pin, const std::vector<int>& pout, double* sides) {
 		CycJob J = {};
-		const Colouring col = colour(s);
+		const Colouring& col = s.col;
 		J.flags = s.flags;
 		J.nops = (int)s.ops.size();
 		// tile positions: the four lowest from bits with independent bank terms (the map is then
@@ -549,104 +482,121 @@ inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, c
 			}
 		}
 		// products
-		struct Choice { std::vector<int> w; int cl, ch, rl, rh; std::array<int, 2> ur, uc; int x, y, score; std::array<int, 2> g; bool good; };
-		auto others = [](const std::vector<int>& q, const std::vector<int>& without) {
-			std::vector<int> o;
-			for (int b : q) { if (std::find(without.begin(), without.end(), b) == without.end()) { o.push_back(b); } }
-			return o;
-		};
-		// the op's layout with wave bits (rows wr, columns wc), if they avoid its gates
-		auto fit = [&](const SideOp& o, const std::vector<int>& wr, const std::vector<int>& wc, Choice& out) {
-			const int ra = o.a >= 0 ? o.a : s.conj ? o.rec : -1, cb = o.b >= 0 ? o.b : s.conj ? o.rec : -1;
-			auto side = [&](int x, const std::vector<int>& q, const std::vector<int>& c, const std::vector<int>& w, int& lo, int& hi,
-				std::array<int, 2>& u) {
-				std::vector<int> left = others(q, w);   // four bits: the gate's two and the block's two
-				if (left.size() != 4) { return false; }
-				if (x >= 0) {
-					lo = bj[x];
-					hi = bi[x];
-					const auto r = others(left, {lo, hi});
-					if (r.size() != 2) { return false; }
-					u = {r[0], r[1]};
-				} else {
-					// no gate on this side: any two bits, the colours differing in both pairs
-					bool found = false;
-					for (int a = 1; a < 4 && !found; a++) {
-						const auto r = others(left, {left[0], left[a]});
-						found = c[left[0]] != c[left[a]] && c[r[0]] != c[r[1]];
-						if (found || a == 3) { lo = left[0]; hi = left[a]; u = {r[0], r[1]}; }
-					}
-				}
-				return true;
-			};
-			if (!side(ra, s.rows, col.r, wr, out.rl, out.rh, out.ur)) { return false; }
-			if (!side(cb, s.cols, col.c, wc, out.cl, out.ch, out.uc)) { return false; }
-			out.w.clear();
-			for (size_t i = 0; i < wr.size(); i++) { out.w.push_back(L + wr[i]); out.w.push_back(wc[i]); }
-			// block directions x, y and group bits: among the four bits left (row and column bits of
-			// two qubits each) the pair whose reads and writes have the fewest bank conflicts
-			const int bits[4] = {L + out.ur[0], out.uc[0], L + out.ur[1], out.uc[1]};
-			auto beta = [&](int mask) {
-				int v = 0;
-				for (int t = 0; t < 4; t++) { if ((mask >> t) & 1) { v ^= col.beta(bits[t], L); } }
-				return v;
-			};
-			const int rl = col.beta(L + out.rl, L), rh = col.beta(L + out.rh, L), cl = col.beta(out.cl, L), ch = col.beta(out.ch, L);
-			const bool right = o.b >= 0 || (o.a < 0 && o.rec >= 0);
-			out.score = -1;
-			for (int x = 1; x < 16 && out.score < 36; x++) {
-				for (int y = 1; y < 16 && out.score < 36; y++) {
+		struct Choice { int cl, ch, rl, rh; int ur[2], uc[2]; int x, y, score; int g[2]; };
+		// the block directions x, y among four bits (row and column bits of two qubits, bank terms b[0 .. 3])
+		// whose reads and writes have the fewest bank conflicts: read s0, s1, x + y, x + t, write w0, w1, x;
+		// kept by the terms, since few sets of them occur
+		struct Blocks { uint64_t key; int x, y, score; };
+		std::array<Blocks, 128> known;
+		for (Blocks& k : known) { k.key = 0; }
+		auto blocks = [&](const int* b, int s0, int s1, int t, int w0, int w1) {
+			const uint64_t key = 1ull << 40 | (uint64_t)s0 << 36 | (uint64_t)s1 << 32 | (uint64_t)t << 28 | (uint64_t)w0 << 24 |
+				(uint64_t)w1 << 20 | (uint64_t)(b[0] | b[1] << 4 | b[2] << 8 | b[3] << 12);
+			Blocks& r = known[(key * 0x9e3779b97f4a7c15ull) >> 57];
+			if (r.key == key) { return r; }
+			r = Blocks{key, 0, 0, -1};
+			int v[16];
+			for (int m = 0; m < 16; m++) { v[m] = (m & 1 ? b[0] : 0) ^ (m & 2 ? b[1] : 0) ^ (m & 4 ? b[2] : 0) ^ (m & 8 ? b[3] : 0); }
+			const unsigned base = span_add(span_add(1, s0), s1);
+			for (int x = 1; x < 16 && r.score < 36; x++) {
+				const int w = 2 * cyc_write_rank(w0, w1, v[x]);
+				const unsigned sx = span_add(base, v[x] ^ t);
+				if (8 * std::min(4, span_rank(sx) + 1) + w <= r.score) { continue; }
+				for (int y = 1; y < 16 && r.score < 36; y++) {
 					if (y == x) { continue; }
-					const int bx = beta(x), by = beta(y);
-					const int rd = right ? cyc_read_rank(rl, rh, bx, by, cl) : cyc_read_rank(cl, ch, bx, by, rl);
-					const int sc = 8 * rd + 2 * cyc_write_rank(cl, ch, bx);
-					if (sc > out.score) { out.score = sc; out.x = x; out.y = y; }
+					const int sc = 8 * span_rank(span_add(sx, v[x] ^ v[y])) + w;
+					if (sc > r.score) { r.score = sc; r.x = x; r.y = y; }
 				}
-			}
-			// the group bits complete x and y (mod the span): the first two single bits that do
-			{
-				std::array<int, 4> v = {out.x, out.y, 0, 0};
-				int n = 0;
-				for (int t : {1, 3, 0, 2}) {
-					if (n == 2) { break; }
-					v[2 + n] = 1 << t;
-					if (rank4(v, 3 + n) == 3 + n) { out.g[n++] = t; }
-				}
-			}
-			out.good = out.score == 36;
-			return true;
-		};
-		auto subsets = [&](const std::vector<int>& q, int n) {
-			std::vector<std::vector<int>> r;
-			if (n == 0) { r.push_back({}); return r; }
-			for (size_t a = 0; a < q.size(); a++) {
-				if (n == 1) { r.push_back({q[a]}); continue; }
-				for (size_t b = a + 1; b < q.size(); b++) { r.push_back({q[a], q[b]}); }
 			}
 			return r;
 		};
-		const auto wrs = subsets(s.rows, K - 4), wcs = subsets(s.cols, K - 4);
-		std::vector<int> wr, wc;
+		const int half = K - 4;   // row bits (and column bits) that number the waves
+		auto row_slot = [&](const SideOp& o) { return o.a >= 0 ? o.a : s.conj ? o.rec : -1; };
+		auto col_slot = [&](const SideOp& o) { return o.b >= 0 ? o.b : s.conj ? o.rec : -1; };
+		auto gate = [&](int x) { return x >= 0 ? (1u << bi[x]) | (1u << bj[x]) : 0u; };
+		// the bits of one side with the wave bits w taken out, a gate's (x) first: lo, hi, then the block's
+		auto side = [&](int x, unsigned q, const std::vector<int>& c, unsigned w, int& lo, int& hi, int* u) {
+			int left[4], n = 0;
+			for (unsigned m = q & ~w; m != 0; m &= m - 1) { left[n++] = __builtin_ctz(m); }
+			if (x >= 0) {
+				lo = bj[x];
+				hi = bi[x];
+			} else {
+				// no gate on this side: any two bits, the colours differing in both pairs
+				lo = left[0];
+				for (int a = 1; a < 4; a++) {
+					hi = left[a];
+					const int r0 = left[a == 1 ? 2 : 1], r1 = left[a == 3 ? 2 : 3];
+					if (c[lo] != c[hi] && c[r0] != c[r1]) { break; }
+				}
+			}
+			int k = 0;
+			for (int i = 0; i < 4; i++) { if (left[i] != lo && left[i] != hi) { u[k++] = left[i]; } }
+		};
+		// the op's layout with wave bits (rows wr, columns wc) that avoid its gates
+		auto fit = [&](const SideOp& o, unsigned wr, unsigned wc, Choice& out) {
+			side(row_slot(o), rm, col.r, wr, out.rl, out.rh, out.ur);
+			side(col_slot(o), cm, col.c, wc, out.cl, out.ch, out.uc);
+			const int b[4] = {col.r[out.ur[0]], col.c[out.uc[0]] << 2, col.r[out.ur[1]], col.c[out.uc[1]] << 2};
+			const int rl = col.r[out.rl], rh = col.r[out.rh], cl = col.c[out.cl] << 2, ch = col.c[out.ch] << 2;
+			const bool right = o.b >= 0 || (o.a < 0 && o.rec >= 0);
+			const Blocks k = right ? blocks(b, rl, rh, cl, cl, ch) : blocks(b, cl, ch, rl, cl, ch);
+			out.x = k.x;
+			out.y = k.y;
+			out.score = k.score;
+			return k.score == 36;
+		};
+		// sets of wave bits, and from product j on the products that they avoid the gates of
+		auto subsets = [&](const std::vector<int>& q) {
+			std::vector<unsigned> r;
+			for (size_t a = 0; a < q.size(); a++) {
+				if (half == 1) { r.push_back(1u << q[a]); }
+				else { for (size_t b = a + 1; b < q.size(); b++) { r.push_back((1u << q[a]) | (1u << q[b])); } }
+			}
+			return r;
+		};
+		const auto wrs = subsets(s.rows), wcs = subsets(s.cols);
+		unsigned wr = 0, wc = 0;
 		bool have = false;
 		for (size_t j = 0; j < s.ops.size(); j++) {
 			const SideOp& o = s.ops[j];
 			Choice ch;
-			bool keep = have && fit(o, wr, wc, ch) && ch.good;
+			const bool keep = have && !(gate(row_slot(o)) & wr) && !(gate(col_slot(o)) & wc) && fit(o, wr, wc, ch);
 			if (!keep) {
 				// the wave bits that serve the most products from here on
+				const int left = (int)(s.ops.size() - j);
+				auto reach = [&](const std::vector<unsigned>& ws, auto slot) {
+					std::vector<int> n(ws.size(), 0);
+					for (size_t i = 0; i < ws.size(); i++) {
+						while (n[i] < left && !(gate(slot(s.ops[j + n[i]])) & ws[i])) { n[i]++; }
+					}
+					return n;
+				};
+				const std::vector<int> nr = reach(wrs, row_slot), nc = reach(wcs, col_slot);
 				int best = -1000;
-				for (auto& a : wrs) {
-					for (auto& b : wcs) {
-						if (s.conj && a != b) { continue; }
-						int run = 0;
+				for (size_t a = 0; a < wrs.size() && best < left; a++) {
+					for (size_t b = s.conj ? a : 0; b < (s.conj ? a + 1 : wcs.size()) && best < left; b++) {
+						const int most = std::min(nr[a], nc[b]);
+						if (most == 0 || most <= best) { continue; }
 						Choice t;
-						if (!fit(o, a, b, t)) { continue; }
-						run = t.score - 36;
-						if (t.good) { for (run = 1; j + run < s.ops.size() && fit(s.ops[j + run], a, b, t) && t.good; run++) { } }
-						if (run > best) { best = run; wr = a; wc = b; }
+						int run = 1;
+						if (!fit(o, wrs[a], wcs[b], t)) { run = t.score - 36; }
+						else { while (run < most && fit(s.ops[j + run], wrs[a], wcs[b], t)) { run++; } }
+						if (run > best) { best = run; wr = wrs[a]; wc = wcs[b]; }
 					}
 				}
 				fit(o, wr, wc, ch);
+			}
+			// the group bits complete x and y (mod the span): the first two single bits that do
+			{
+				unsigned span = span_add(span_add(1, ch.x), ch.y);
+				int n = 0;
+				for (int t : {1, 3, 0, 2}) {
+					if (n < 2 && !((span >> (1 << t)) & 1)) {
+						span = span_add(span, 1 << t);
+						ch.g[n++] = t;
+					}
+				}
 			}
 			CycOp& q = J.op[j];
 			q.barrier = (j > 0 && !keep) ? 1 : 0;
@@ -663,7 +613,11 @@ inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, c
 			const int d[8] = {byte[L + ch.rl], byte[L + ch.rh], byte[ch.cl], byte[ch.ch], at(ch.x), at(ch.y), byte[bits[ch.g[0]]],
 				byte[bits[ch.g[1]]]};
 			for (int i = 0; i < 8; i++) { q.dir[i] = d[i]; }
-			for (size_t i = 0; i < ch.w.size(); i++) { q.dir[8 + i] = byte[ch.w[i]]; }
+			unsigned r = wr, c = wc;
+			for (int i = 0; i < half; i++, r &= r - 1, c &= c - 1) {
+				q.dir[8 + 2 * i] = byte[L + __builtin_ctz(r)];
+				q.dir[9 + 2 * i] = byte[__builtin_ctz(c)];
+			}
 			// the blocks with equal row and column bits, as combinations of the block and group
 			// directions (x, y, g0, g1: four bits each)
 			if (o.rec >= 0) {

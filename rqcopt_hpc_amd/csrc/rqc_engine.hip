@@ -21,7 +21,6 @@
 #include <functional>
 #include <map>
 #include <string>
-#include <set>
 #include <vector>
 
 #include "rqc_internal.hpp"
@@ -402,121 +401,23 @@ struct Pass
 	std::vector<int> rb;     // tile row bits, ascending
 };
 
-// Pass planning over the circuit's dependency order: gates on disjoint wires
-// commute, so a pass may take any gate whose predecessors on its two wires are
-// done, as long as its wires lie in the pass's K tile qubits.  Candidate tile
-// sets for a pass: every window of K consecutive wires (cyclic) and the wires of
-// the ready gates in circuit order; a candidate takes its ready gates in circuit
-// order, at most gmax.  A beam search over these choices keeps, after each pass,
-// the kPlanBeam states with the most gates done (ties to the earlier state and
-// candidate), and the first plan to finish has the fewest passes found; width 1
-// is the greedy plan (the candidate that takes the most gates).  At L = 14,
-// depth 9, K = 6 and 8 gates the beam finds 9 passes where the greedy plan
-// needs 10 (its last passes take 3 and 1 gates).  Tiles are padded with the
-// lowest unused row bits.  Any topological order of the gates gives the same
-// states at each gate up to rounding, so the sweeps of the passes compute the
-// reference's per-gate quantities.
+// Passes of the tile sweeps (rqc_pass_search.hpp: the fewest passes found).  At L = 14, depth 9, K = 6
+// and 8 gates the search finds 9 passes where the greedy plan (the candidate that takes the most gates)
+// needs 10: its last passes take 3 and 1 gates.  Tiles are padded with the lowest unused row bits.  Any
+// topological order of the gates gives the same states at each gate up to rounding, so the sweeps of the
+// passes compute the reference's per-gate quantities.
 static std::vector<Pass> plan_passes(const Circuit& C, int K, int gmax)
 {
 	const int L = C.L, G = C.ngates;
-	auto bitmask = [&](int k) { return (1u << (L - 1 - C.wi[k])) | (1u << (L - 1 - C.wj[k])); };
-	std::vector<int> prev_i(G, -1), prev_j(G, -1), last(L, -1);
-	for (int k = 0; k < G; k++) {
-		prev_i[k] = last[C.wi[k]];
-		prev_j[k] = last[C.wj[k]];
-		last[C.wi[k]] = k;
-		last[C.wj[k]] = k;
-	}
-	const int beam_width = (G <= 256) ? 32 : (G <= 2048) ? 4 : 1;
-	std::vector<char> taken(G, 0);
-	auto ok = [&](const std::vector<char>& done, int k) {
-		return (prev_i[k] < 0 || done[prev_i[k]] || taken[prev_i[k]]) &&
-		       (prev_j[k] < 0 || done[prev_j[k]] || taken[prev_j[k]]);
-	};
-	// the ready gates of the tile set `mask`, in circuit order, at most gmax
-	auto take = [&](const std::vector<char>& done, unsigned mask, std::vector<int>& out) {
-		std::fill(taken.begin(), taken.end(), 0);
-		out.clear();
-		for (int k = 0; k < G && (int)out.size() < gmax; k++) {
-			if (done[k] || (bitmask(k) & ~mask) != 0 || !ok(done, k)) { continue; }
-			taken[k] = 1;
-			out.push_back(k);
-		}
-		std::fill(taken.begin(), taken.end(), 0);
-	};
-	auto candidates = [&](const std::vector<char>& done) {
-		std::vector<unsigned> cands;
-		if (K >= L) {
-			cands.push_back((L >= 32) ? ~0u : ((1u << L) - 1));
-			return cands;
-		}
-		for (int s = 0; s < L; s++) {
-			unsigned m = 0;
-			for (int t = 0; t < K; t++) { m |= 1u << (L - 1 - (s + t) % L); }
-			cands.push_back(m);
-		}
-		unsigned m = 0;
-		for (int k = 0; k < G; k++) {
-			if (done[k] || !ok(done, k)) { continue; }
-			const unsigned m2 = m | bitmask(k);
-			if (__builtin_popcount(m2) <= K) { m = m2; }
-		}
-		cands.push_back(m);
-		return cands;
-	};
-	struct State
-	{
-		std::vector<char> done;
-		int ndone;
-		std::vector<std::vector<int>> passes;
-	};
-	std::vector<State> beam(1);
-	beam[0].done.assign(G, 0);
-	beam[0].ndone = 0;
-	std::vector<std::vector<int>> plan;
-	if (G == 0) { beam.clear(); }
-	std::vector<int> lst;
-	while (!beam.empty()) {
-		std::vector<State> next;
-		std::set<std::vector<char>> seen;
-		bool finished = false;
-		for (const State& st : beam) {
-			// expansions in candidate order, the one taking the most gates first
-			std::vector<std::pair<int, std::vector<int>>> exps;
-			for (unsigned m : candidates(st.done)) {
-				take(st.done, m, lst);
-				if (!lst.empty()) { exps.emplace_back((int)lst.size(), lst); }
-			}
-			std::stable_sort(exps.begin(), exps.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
-			for (auto& e : exps) {
-				State t;
-				t.done = st.done;
-				for (int k : e.second) { t.done[k] = 1; }
-				if (!seen.insert(t.done).second) { continue; }
-				t.ndone = st.ndone + e.first;
-				t.passes = st.passes;
-				t.passes.push_back(std::move(e.second));
-				if (t.ndone == G) {
-					plan = std::move(t.passes);
-					finished = true;
-					break;
-				}
-				next.push_back(std::move(t));
-			}
-			if (finished) { break; }
-		}
-		if (finished) { break; }
-		if (next.empty()) { throw Error(-4, "pass planning made no progress"); }
-		std::stable_sort(next.begin(), next.end(), [](const State& a, const State& b) { return a.ndone > b.ndone; });
-		if ((int)next.size() > beam_width) { next.resize(beam_width); }
-		beam = std::move(next);
-	}
+	PassSearch S{L, K, gmax, {}, true, false};
+	for (int k = 0; k < G; k++) { S.gm.push_back((1u << (L - 1 - C.wi[k])) | (1u << (L - 1 - C.wj[k]))); }
+	const std::vector<FoundPass> plan = search_passes(S, [](unsigned, unsigned) { return 0; });
+	if (plan.empty() && G > 0) { throw Error(-4, "pass planning made no progress"); }
 	std::vector<Pass> out;
-	for (auto& gl : plan) {
+	for (const FoundPass& f : plan) {
 		Pass p;
-		p.gates = gl;
-		unsigned used = 0;
-		for (int k : p.gates) { used |= bitmask(k); }
+		p.gates = f.gates;
+		const unsigned used = f.used;
 		for (int b = 0; b < L; b++) {
 			if (used & (1u << b)) { p.rb.push_back(b); }
 		}
@@ -927,26 +828,45 @@ static size_t cyc_lds(int K, bool dual)
 // evaluations share a launch.
 static int cyc_tile_qubits(int L, int copies) { return (L >= 10 || (L >= 6 && copies >= 1 << (20 - 2 * L))) ? 6 : 5; }
 
-static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const Circuit& C, bool dual, bool fp32, bool target_only, int K)
+// A circuit's passes for tiles of K qubits, shared by the kinds of evaluations and the precisions: the
+// execution order (gate of each slot, its wires' qubit bits) and the passes' slots
+struct CycCircuit
+{
+	std::vector<int> order, bi, bj;
+	std::vector<CycPass> passes;
+};
+
+static std::shared_ptr<const CycCircuit> cyc_circuit(const Circuit& C, int K)
+{
+	static PlanCache<CycCircuit> cache;
+	return cache.get(structure_ints(C, {K}), [&] {
+		auto cc = std::make_shared<CycCircuit>();
+		std::vector<int> gi(C.ngates), gj(C.ngates);
+		for (int k = 0; k < C.ngates; k++) {
+			gi[k] = C.L - 1 - C.wi[k];
+			gj[k] = C.L - 1 - C.wj[k];
+		}
+		// a circuit inside one tile: two passes of at most kCycOps gates suit the two directions
+		const int gmax = (C.L <= K) ? std::min(kCycOps, std::max(1, (C.ngates + 1) / 2)) : kCycOps;
+		cc->passes = plan_cyc_passes(C.L, gi, gj, K, gmax);
+		for (CycPass& p : cc->passes) {
+			for (int& k : p.slots) {
+				cc->order.push_back(k);
+				cc->bi.push_back(gi[k]);
+				cc->bj.push_back(gj[k]);
+				k = (int)cc->order.size() - 1;
+			}
+		}
+		return cc;
+	});
+}
+
+static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const Circuit& C, const CycCircuit& cc, int split, bool dual,
+	bool fp32, bool target_only, int K)
 {
 	auto tp = std::make_shared<TilePlan>();
-	std::vector<int> gi(C.ngates), gj(C.ngates), bi, bj;
-	for (int k = 0; k < C.ngates; k++) {
-		gi[k] = C.L - 1 - C.wi[k];
-		gj[k] = C.L - 1 - C.wj[k];
-	}
-	// a circuit inside one tile: two passes of at most kCycOps gates suit the two directions
-	const int gmax = (C.L <= K) ? std::min(kCycOps, std::max(1, (C.ngates + 1) / 2)) : kCycOps;
-	std::vector<CycPass> passes = plan_cyc_passes(C.L, gi, gj, K, gmax);
-	for (CycPass& p : passes) {
-		for (int& k : p.slots) {
-			tp->order.push_back(k);
-			bi.push_back(gi[k]);
-			bj.push_back(gj[k]);
-			k = (int)tp->order.size() - 1;
-		}
-	}
-	tp->cyc = make_cyc_plan(C.L, K, passes, bi, bj, target_only, dual, kMatG, kMatGinv);
+	tp->order = cc.order;
+	tp->cyc = make_cyc_plan(C.L, K, cc.passes, split, cc.bi, cc.bj, target_only, dual, kMatG, kMatGinv);
 	const size_t lds = cyc_lds(K, dual);
 	int occ = 0;
 	for (bool out : {false, true}) {
@@ -962,15 +882,16 @@ static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const 
 		while (2 * g <= std::min<long>(n, (long)std::max(1, occ) * dev.cu_count)) { g *= 2; }
 		tp->cyc_grid.push_back((unsigned)g);
 	}
-	tp->passes.resize(passes.size());
+	tp->passes.resize(cc.passes.size());
 	return tp;
 }
 
-static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circuit& C, bool dual, bool fp32, bool target_only, int K)
+static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circuit& C, const CycCircuit& cc, int split, bool dual, bool fp32,
+	bool target_only, int K)
 {
 	static PlanCache<TilePlan> cache;
 	return cache.get(structure_ints(C, {K, dual, fp32, target_only, dev.device}),
-		[&] { return make_cyc_tiles(dev, C, dual, fp32, target_only, K); });
+		[&] { return make_cyc_tiles(dev, C, cc, split, dual, fp32, target_only, K); });
 }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1005,7 +926,10 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	if (tiles && !pl.sampled && C.L >= 5 && 2 * (C.L - 6) <= kCycGens) {
 		const int K = cyc_tile_qubits(C.L, copies);
 		const bool dual = (mode == Mode::Hvp);
-		auto tp = plan_cyc(dev, C, dual, fp32, mode == Mode::Target, K);
+		const bool target_only = (mode == Mode::Target);
+		const auto cc = cyc_circuit(C, K);
+		const int split = cyc_split(C.L, K, cc->passes, target_only);
+		auto tp = plan_cyc(dev, C, *cc, split, dual, fp32, target_only, K);
 		const int nst = tp->cyc.nbuf * (dual ? 2 : 1);
 		// (arrays that fit the held workspace need no look at the free memory)
 		const size_t need = (size_t)nst * pl.N * pl.N * elem;

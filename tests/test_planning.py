@@ -1,15 +1,22 @@
-"""Host planning (headers without device code, compiled here with g++): the cache of plans."""
+"""Host planning (headers without device code, compiled here with g++): the cache of plans, the search of a
+circuit's passes and the plans of the cyclic-product sweeps."""
 import os
 import subprocess
+
+import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rqcopt_hpc_amd", "csrc")
 
 
-def _run(tmp_path, source):
-    src, exe = tmp_path / "check.cpp", tmp_path / "check"
+def _build(folder, source):
+    src, exe = folder / "check.cpp", folder / "check"
     src.write_text(source)
     subprocess.check_call(["g++", "-std=c++17", "-O3", "-Wall", "-Werror", "-pthread", "-I", CSRC, str(src), "-o", str(exe)])
-    return subprocess.run([str(exe)], text=True, capture_output=True, timeout=120)
+    return str(exe)
+
+
+def _run(exe, *args):
+    return subprocess.run([exe] + [str(a) for a in args], text=True, capture_output=True, timeout=120)
 
 
 CACHE = r"""
@@ -53,6 +60,82 @@ int main()
 
 
 def test_a_thread_that_plans_does_not_keep_others_from_their_plans(tmp_path):
-    r = _run(tmp_path, CACHE)
+    r = _run(_build(tmp_path, CACHE))
     assert r.returncode == 0, r.stderr
     assert r.stdout.split("\n")[:2] == ["1 10 1 21", "21 -2"]
+
+
+PLAN = r"""
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include "rqc_cyc_plan.hpp"
+using namespace rqc;
+int main(int argc, char** argv)
+{
+	// L layers: a periodic brickwall; L 0 gates: a random circuit
+	const int L = atoi(argv[1]), layers = atoi(argv[2]), ngates = atoi(argv[3]), K = L >= 10 ? 6 : 5;
+	std::vector<int> bi, bj;
+	for (int i = 0; i < layers; i++) {
+		for (int q = 0; q + 1 < L; q += 2) {
+			bi.push_back((q + i % 2) % L);
+			bj.push_back((q + 1 + i % 2) % L);
+		}
+	}
+	srand(L + ngates);
+	for (int k = 0; k < ngates; k++) {
+		bi.push_back(rand() % L);
+		bj.push_back((bi.back() + 1 + rand() % (L - 1)) % L);
+	}
+	const int G = (int)bi.size();
+	double best = 1e9;
+	for (int rep = 0; rep < (G > 500 ? 3 : 20); rep++) {
+		const auto t0 = std::chrono::steady_clock::now();
+		std::vector<CycPass> passes = plan_cyc_passes(L, bi, bj, K, kCycOps);
+		// every gate once, after the gates before it on its wires, in a pass that holds its wires
+		std::vector<int> last(L, -1), si, sj;
+		std::vector<char> seen(G, 0);
+		for (CycPass& p : passes) {
+			if ((int)p.q.size() != K || p.slots.empty() || (int)p.slots.size() > kCycOps) { return 1; }
+			for (int& k : p.slots) {
+				unsigned q = 0;
+				for (int b : p.q) { q |= 1u << b; }
+				if (seen[k]++ || !((q >> bi[k]) & 1) || !((q >> bj[k]) & 1)) { return 2; }
+				for (int b : {bi[k], bj[k]}) {
+					if (last[b] > k) { return 3; }
+					last[b] = k;
+				}
+				si.push_back(bi[k]);
+				sj.push_back(bj[k]);
+				k = (int)si.size() - 1;
+			}
+		}
+		if ((int)si.size() != G) { return 4; }
+		for (int kind = 0; kind < 3; kind++) {
+			const int split = cyc_split(L, K, passes, kind == 0);
+			const CycPlan p = make_cyc_plan(L, K, passes, split, si, sj, kind == 0, kind == 2, 0, 2);
+			if (p.nbuf > 4) { return 5; }
+		}
+		best = std::min(best, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count());
+	}
+	printf("%.0f\n", best);
+	return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    return _build(tmp_path_factory.mktemp("plan"), PLAN)
+
+
+# Bounds: a first evaluation's planning (passes once, then the target's, the gradient's and the HVP's plan)
+# has to stay below what an evaluation of the sizes takes with its planning, 0.13 ms at 6 qubits and 9
+# layers to 2.3 ms at 12 and 9; the bound is that of one target evaluation, three times the 0.1 to 0.7 ms
+# measured here.
+@pytest.mark.parametrize("L,layers,ngates,us", [(6, 3, 0, 130), (6, 9, 0, 400), (8, 7, 0, 600), (10, 5, 0, 600), (10, 9, 0, 1900),
+                                                (12, 9, 0, 2100), (14, 0, 200, 16000), (10, 0, 1000, 30000)])
+def test_plans_hold_every_gate_in_order_and_are_quick(plan, L, layers, ngates, us):
+    r = _run(plan, L, layers, ngates)
+    assert r.returncode == 0, r.returncode
+    assert float(r.stdout) < us
