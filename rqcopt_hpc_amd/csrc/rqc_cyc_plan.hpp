@@ -258,6 +258,22 @@ inline int cyc_split(int L, int K, const std::vector<CycPass>& passes, bool targ
 	return m;
 }
 
+// array pairs (one array without directions) of P passes split at m: the forward launches use two in
+// turn, and see the jobs' arrays in make_cyc_plan
+inline int cyc_arrays(int P, int m, bool target_only)
+{
+	const int F = std::max(m, P - m), longer = F, shorter = P - F;
+	if (target_only) { return std::min(F - 1, 2); }
+	return shorter >= 2 ? 4 : longer >= 3 ? 3 : longer == 2 ? 2 : 1;
+}
+
+// least arrays of any circuit of G gates (before its passes are known)
+inline int cyc_least_arrays(int G, bool target_only)
+{
+	const int P = (G + kCycOps - 1) / kCycOps;
+	return target_only ? cyc_arrays(P, (P + 1) / 2, true) : P <= 2 ? 1 : P == 3 ? 2 : 3;
+}
+
 // bi, bj: qubit bits of slot x's wires (the more significant gate index first); m: cyc_split's; with
 // target only, the forward launches run to the end and the last one sums the trace
 inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, int m, const std::vector<int>& bi,

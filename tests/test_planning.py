@@ -114,7 +114,9 @@ int main(int argc, char** argv)
 		for (int kind = 0; kind < 3; kind++) {
 			const int split = cyc_split(L, K, passes, kind == 0);
 			const CycPlan p = make_cyc_plan(L, K, passes, split, si, sj, kind == 0, kind == 2, 0, 2);
-			if (p.nbuf > 4) { return 5; }
+			// the arrays are known before the plan is made, and the least of them before the search
+			if (p.nbuf != cyc_arrays((int)passes.size(), split, kind == 0)) { return 5; }
+			if (p.nbuf < cyc_least_arrays(G, kind == 0)) { return 6; }
 		}
 		best = std::min(best, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count());
 	}
