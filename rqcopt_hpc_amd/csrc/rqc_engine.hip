@@ -776,9 +776,11 @@ static std::shared_ptr<TilePlan> plan_tiles(const Context& dev, const Circuit& C
 		// One reduction (two launches) for as many passes as 16 MiB of partial sums allow: few
 		// workgroups have few parts, and then the reductions' launches take as long as the passes
 		// (block encoding of 10 qubits, 7 layers, 32 workgroups, six reductions: 300 us, one: 245).
-		// The largest grids reduce after each pass.
+		// The largest grids reduce after each pass, and so do plans that have to be small: for 10 qubits,
+		// 5 layers in blocks of 16 columns the sums of all gates take 3.3 MB next to 2 MB of states, those
+		// of a pass 1 MB.
 		const size_t nparts = (size_t)tp->grev * kTileWaves;
-		const int most = std::max(maxng, (int)std::min<size_t>(kReduceGates, 8192 / nparts));
+		const int most = pl.lean ? maxng : std::max(maxng, (int)std::min<size_t>(kReduceGates, 8192 / nparts));
 		for (int p = (int)passes.size() - 1; p >= 0; p--) {
 			const int ng = (int)passes[p].gates.size();
 			if (tp->reductions.empty() || tp->reductions.back().ng + ng > most) { tp->reductions.push_back({p, 0, 0}); }
@@ -897,7 +899,7 @@ static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circui
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, bool fp32, bool project, bool unitary,
-	size_t budget, size_t held, const TileChoice* choice, long ncols, int copies)
+	size_t budget, size_t held, const TileChoice* choice, long ncols, int copies, bool lean)
 {
 	const int logE_c = (choice != nullptr) ? choice->logE : 0;
 	const int gmax = (choice != nullptr && choice->gmax > 0) ? std::min(choice->gmax, (int)kMaxTileGates) : tile_gmax();
@@ -908,6 +910,7 @@ EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, boo
 	pl.mode = mode;
 	pl.fp32 = fp32;
 	pl.project = project;
+	pl.lean = lean;
 	pl.L = C.L;
 	pl.G = C.ngates;
 	pl.per = per;
@@ -2686,6 +2689,7 @@ static EvalPlan plan_in_scratch(const Context& c, const Circuit& C, Mode mode, i
 		EvalPlan pl;
 		try {
 			pl = plan_eval(c, C, mode, per, fp32, project, unitary, budget, 0);
+			if (pl.bytes > kScratchBytes) { pl = plan_eval(c, C, mode, per, fp32, project, unitary, budget, 0, nullptr, 0, 1, true); }
 		} catch (const Error&) {
 			break;   // not even one column's state arrays fit
 		}

@@ -62,6 +62,7 @@ struct EvalPlan
 	bool project = false;  // Riemannian projection of gradient and HVP
 	bool tiles = false;    // tile-pass engine (else one gate per pass)
 	bool cyc = false;      // cyclic-product sweeps (with tiles; rqc_cyc_plan.hpp)
+	bool lean = false;     // see plan_eval
 	int L = 0, G = 0, per = 1, ng = 0;
 	long N = 0, B = 0;     // 2^L and the column-block width
 	bool sampled = false;  // columns are given states (stochastic trace), not the basis
@@ -92,9 +93,11 @@ struct EvalPlan
 // (0 = automatic, 85% of the free device memory plus `held`); `ncols` > 0: the
 // sweep's columns are that many given states instead of the 2^L basis columns
 // (the column block is then at most the power of two covering them); `copies`: evaluations of the
-// plan that will share launches (EvalCopies; it only sizes the tiles)
+// plan that will share launches (EvalCopies; it only sizes the tiles); `lean`: the least workspace
+// besides the state arrays (column sweeps then reduce their sums after every pass), for callers whose
+// whole workspace is limited
 EvalPlan plan_eval(const Context& dev, const Circuit& C, Mode mode, int per, bool fp32, bool project, bool unitary,
-	size_t budget, size_t held, const TileChoice* choice = nullptr, long ncols = 0, int copies = 1);
+	size_t budget, size_t held, const TileChoice* choice = nullptr, long ncols = 0, int copies = 1, bool lean = false);
 // host image of the evaluation's table region (pl.tab_bytes bytes at `host`)
 void fill_eval_tables(const EvalPlan& pl, const Circuit& C, char* host);
 

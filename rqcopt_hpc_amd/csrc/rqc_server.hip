@@ -239,7 +239,13 @@ static std::shared_ptr<const EvalPlan> session_plan(Session& s, int kind, bool u
 			const Mode m = kind == RQC_EVAL_TARGET ? Mode::Target : (kind == RQC_EVAL_GRADIENT ? Mode::Grad : Mode::Hvp);
 			Circuit C = s.C;
 			C.dirs.assign(C.gates.size(), zc{0, 0});
-			auto np = std::make_shared<EvalPlan>(plan_eval(*S.dev, C, m, s.per, s.fp32, true, unitary, S.max_req, 0));
+			auto plan = [&](bool lean) {
+				return std::make_shared<EvalPlan>(plan_eval(*S.dev, C, m, s.per, s.fp32, true, unitary, S.max_req, 0, nullptr, 0, 1, lean));
+			};
+			// (sums of several passes only where the request stays below the cap with them: they would
+			// otherwise keep other requests out of the arena, or this one)
+			auto np = plan(false);
+			if (np->bytes > S.max_req) { np = plan(true); }
 			if (np->bytes > S.alloc.size) {
 				throw Error(-1, "request workspace (" + std::to_string(np->bytes) + " bytes) exceeds the server arena");
 			}
