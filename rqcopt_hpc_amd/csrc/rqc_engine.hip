@@ -2684,8 +2684,10 @@ extern "C" int brickwall_unitary_target_projected_hessian_vector_product(linear_
 static EvalPlan plan_in_scratch(const Context& c, const Circuit& C, Mode mode, int per, bool fp32, bool project,
 	bool unitary)
 {
+	// (the budget falls below the arrays of a plan that does not fit, so that the next one is narrower:
+	// lowered by the excess alone, it left the same block in place, and 12 qubits, 5 layers were refused)
 	size_t budget = kScratchBytes;
-	for (int it = 0; it < 64 && budget > 0; it++) {
+	while (budget > 0) {
 		EvalPlan pl;
 		try {
 			pl = plan_eval(c, C, mode, per, fp32, project, unitary, budget, 0);
@@ -2694,8 +2696,8 @@ static EvalPlan plan_in_scratch(const Context& c, const Circuit& C, Mode mode, i
 			break;   // not even one column's state arrays fit
 		}
 		if (pl.bytes <= kScratchBytes) { return pl; }
-		const size_t over = pl.bytes - kScratchBytes;
-		budget = (over < budget) ? budget - over : 0;
+		const size_t st = (size_t)pl.state_bytes();
+		budget = (st > 0 && pl.B > 1) ? std::min(budget, st) - 1 : 0;
 	}
 	throw Error(-3, "a " + std::to_string(C.L) + "-qubit circuit of " + std::to_string(C.ngates) +
 		" gates does not fit the no-allocation scratch of " + std::to_string(kScratchBytes >> 20) + " MiB");

@@ -1,4 +1,4 @@
-"""Batches and servers with little memory: the limits that column sweeps which reduce their sums after
+"""Batches, servers and the no-allocation call with little memory: the limits that column sweeps which reduce their sums after
 every pass need are accepted, with column blocks as wide, whatever the sweeps share when there is room.
 
 The limits (bytes) and blocks are those of such plans: 2 P + 4 arrays of 2^L x block amplitudes for P
@@ -67,3 +67,16 @@ def test_requests_fit_their_arena(L, depth, arena, block):
         _check((f, g, h), want)
     finally:
         srv.close()
+
+
+@pytest.mark.parametrize("L,depth", [(10, 6), (12, 4), (12, 5), (12, 20)])
+def test_the_scratch_takes_the_widest_block_that_fits(L, depth):
+    """A column block narrower than the first that is tried: the evaluation runs in half of it, and so on
+    (it is refused only where one column does not fit).  Half of the scratch holds the states at least."""
+    print("qubits", L, "layers", depth, flush=True)
+    P, T, V, D = _problem(L, depth)
+    want = R.brickwall_unitary_target_projected_hessian_vector_product(T, V, D, P)
+    got = R.brickwall_unitary_target_projected_hvp_noalloc(T, V, D, P)
+    B, passes = R.last_column_block(), R.last_sweep()[1]
+    assert B == 1 << L or (2 * passes + 4) * B * 16 << L > R.noalloc_scratch_bytes() // 4
+    _check(got, want)
