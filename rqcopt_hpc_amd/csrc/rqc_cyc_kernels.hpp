@@ -333,10 +333,12 @@ __global__ __launch_bounds__(64 << LW, LW >= 2 * (K - 4) ? 4 : 2) void k_cyc_swe
 // workgroup per execution slot), decoded to its gradient and HVP sums.  Recorded after the gate
 // (M = G E): Tr_rest E = G^-1 R and its derivative G^-1 dR + W R, W = -G^-1 Z G^-1; before it
 // (M = E G): R G^-1 and dR G^-1 + R W.  The gradient of f = -Tr(G E) by G[r][c] is -E[c][r].
-// order: circuit gate of the slot and its side.  Slot 0 writes f = -Tr M.
+// order: circuit gate of the slot and its side.  Slot fslot writes f = -Tr M: the slot recorded first,
+// whose M has seen the forward products alone (the first gate's has been conjugated all the way back:
+// 6 qubits, 9 layers, |f| about 1: root mean square error of f 1.15e-15 there, 0.61e-15 here).
 template <bool DUAL>
 __global__ __launch_bounds__(256) void k_cyc_reduce(const zc* __restrict__ part, long nparts, const int* __restrict__ order,
-	const zc* __restrict__ rmats, zc* __restrict__ acc, long stride, const int* skip)
+	const zc* __restrict__ rmats, zc* __restrict__ acc, int fslot, long stride, const int* skip)
 {
 	if (skipped(skip)) { return; }
 	part = copy_of(part, stride, blockIdx.y);
@@ -357,7 +359,7 @@ __global__ __launch_bounds__(256) void k_cyc_reduce(const zc* __restrict__ part,
 	}
 	__syncthreads();
 	const zc* R = red[0];
-	if (x == 0 && threadIdx.x == 0) {
+	if (x == fslot && threadIdx.x == 0) {
 		const zc t = R[0] + R[5] + R[10] + R[15];
 		acc[0] = zc{-t.x, -t.y};
 	}

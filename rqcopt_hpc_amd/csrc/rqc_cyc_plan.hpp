@@ -80,6 +80,7 @@ struct CycPlan
 	int L = 0, K = 0, nbuf = 0;
 	std::vector<CycLaunch> launches;
 	std::vector<int> up;      // per slot: recorded before (1, upward) or after (0, downward) its gate
+	int fslot = 0;            // the slot recorded first, from M_m itself, whose trace gives f
 	long ntrace = 0;          // tiles of the tracing launch (target evaluations)
 };
 
@@ -341,6 +342,7 @@ inline CycPlan make_cyc_plan(int L, int K, const std::vector<CycPass>& passes, i
 	if (!target_only) {
 		for (int p = m - 1; p >= 0; p--) { down.push_back(conj_step(passes[p], false, p == 0)); }
 		for (int p = m; p < P; p++) { up.push_back(conj_step(passes[p], true, p == P - 1)); }
+		plan.fslot = (!down.empty() ? down : up)[0].ops[0].rec;
 		for (auto* side : {&down, &up}) {
 			unsigned f = 0;
 			for (int i = (int)side->size() - 1; i >= 0; i--) {

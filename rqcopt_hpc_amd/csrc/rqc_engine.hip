@@ -1327,9 +1327,9 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 	if (pl.mode == Mode::Target) {
 		k_cyc_trace<<<1, kBlock, 0, s.stream>>>(d_partial, cp.ntrace * (cyc_nthreads(cp.K, false) / 64), d_acc, skip);
 	} else if (dual) {
-		k_cyc_reduce<true><<<dim3(pl.G, cps.n), 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, cps.stride, skip);
+		k_cyc_reduce<true><<<dim3(pl.G, cps.n), 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, cp.fslot, cps.stride, skip);
 	} else {
-		k_cyc_reduce<false><<<dim3(pl.G, cps.n), 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, cps.stride, skip);
+		k_cyc_reduce<false><<<dim3(pl.G, cps.n), 256, 0, s.stream>>>(d_partial, nparts, order, rmats, d_acc, cp.fslot, cps.stride, skip);
 	}
 }
 

@@ -123,3 +123,33 @@ def test_mixed_precision_rounds_between_launches_only(L, ngates):
     for f in (m[0], m[1][0], m[2][0]):
         assert abs(f - a[0]) < 2e-6 * 2 ** (L / 2)
     assert reldiff(m[1][1], a[1][1]) < 2e-6 and reldiff(m[2][1], a[2][1]) < 2e-6 and reldiff(m[2][2], a[2][2]) < 2e-6
+
+
+def test_f_of_every_kind_is_as_accurate():
+    """f of a gradient or HVP comes from the product before any conjugation, after as many gate products
+    as a target evaluation's: their rounding errors (against 80-bit arithmetic) have one distribution.
+    The root mean squares of 60 complex errors differ by 9 % (120 values each, 1 / sqrt(240) twice);
+    1.35 is four times that above one."""
+    L, depth, n = 6, 9, 60
+    print("qubits", L, "layers", depth, flush=True)
+    N, P = 1 << L, brickwall_perms(L, depth)
+    wires = [(int(p[2 * k]), int(p[2 * k + 1])) for p in P for k in range(L // 2)]
+    err = []
+    for seed in range(n):
+        rng = np.random.default_rng([L, depth, seed])
+        V = np.stack([haar_unitary(rng) for _ in range(depth)])
+        U = np.linalg.qr(crandn(rng, (N, N)))[0]
+        W = np.eye(N, dtype=np.clongdouble)
+        for g, (a, b) in zip(np.repeat(V, L // 2, 0), wires):
+            t = np.moveaxis(W.reshape([2] * L + [N]), (a, b), (0, 1))
+            y = np.tensordot(g.astype(np.clongdouble).reshape(2, 2, 2, 2), t, ((2, 3), (0, 1)))
+            W = np.moveaxis(y, (0, 1), (a, b)).reshape(N, N)
+        f = -(U.astype(np.clongdouble).conj() * W).sum()
+        T = R.DeviceTarget.dense(U)
+        err.append([abs(np.clongdouble(v) - f) for v in (
+            R.brickwall_unitary_target(T, V, P), R.brickwall_unitary_target_and_gradient(T, V, P)[0],
+            R.brickwall_unitary_target_hessian_vector_product(T, V, crandn(rng, V.shape), P)[0])])
+        T.close()
+    target, gradient, hvp = np.sqrt(np.mean(np.array(err, float) ** 2, axis=0))
+    print(target, gradient, hvp, flush=True)
+    assert gradient < 1.35 * target and hvp < 1.35 * target
