@@ -1602,10 +1602,14 @@ static EvalResult eval_targets(const Circuit& C, linear_func ufunc, void* udata,
 	std::lock_guard<std::recursive_mutex> lk(c.mu);
 	const zc* dU = resolve_target(c, ufunc, udata, C.L);
 	const bool unitary = sweep_unitary(C, mode, c.precision == RQC_PRECISION_MIXED);
-	TileChoice tc{0, 0};
-	if (c.eval_autotune && c.engine == RQC_ENGINE_TILE_PASS) { tc = tune_eval(c, C, mode, per, project, unitary, dU); }
-	const EvalPlan pl = plan_eval(c, C, mode, per, c.precision == RQC_PRECISION_MIXED, project, unitary, c.ws_limit,
-		c.work.bytes, tc.logE > 0 ? &tc : nullptr);
+	const bool fp32 = c.precision == RQC_PRECISION_MIXED;
+	EvalPlan pl = plan_eval(c, C, mode, per, fp32, project, unitary, c.ws_limit, c.work.bytes);
+	// (only column sweeps have a tile shape to choose; whether a structure takes them depends on the
+	// workspace limit, so that an evaluation of the other kind decides nothing for it)
+	if (c.eval_autotune && pl.tiles && !pl.cyc) {
+		const TileChoice tc = tune_eval(c, C, mode, per, project, unitary, dU);
+		if (tc.logE > 0) { pl = plan_eval(c, C, mode, per, fp32, project, unitary, c.ws_limit, c.work.bytes, &tc); }
+	}
 	return run_eval(c, pl, C, dU, nullptr, nullptr, nullptr);
 }
 

@@ -1,0 +1,86 @@
+"""Tile shapes and tile autotuning of the column sweeps, which dense targets take when the cyclic-product
+sweeps' arrays do not fit (a workspace limit here), and samples and block encodings always.
+
+Every shape is forced through the environment overrides and has to be the one that ran (last_tiles); its
+FP64 results match the oracle within 1e-12, mixed precision within its stated bounds: |df| / N <= 1e-6,
+gradient and HVP within 1e-4.
+"""
+import os
+
+import numpy as np
+import pytest
+
+import oracle as O
+import rqcopt_hpc_amd as R
+from helpers import brickwall_perms, crandn, haar_unitary, reldiff
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+KEYS = ("RQC_TILE_LOGE_FP64", "RQC_TILE_LOGC_FP64", "RQC_TILE_LOGE_FP32", "RQC_TILE_LOGC_FP32", "RQC_FWD_TILE")
+L, DEPTH = 10, 5
+
+
+@pytest.fixture(autouse=True)
+def clean():
+    R.require_gpu()
+    saved = {k: os.environ.pop(k, None) for k in KEYS}
+    R.set_precision(R.PRECISION_FP64)
+    yield
+    for k, v in saved.items():
+        os.environ.pop(k, None)
+        if v is not None:
+            os.environ[k] = v
+    R.set_precision(R.PRECISION_FP64)
+    R.set_eval_autotune(False)
+    R.set_workspace_limit(0)
+
+
+@pytest.fixture(scope="module")
+def problem():
+    rng = np.random.default_rng(41)
+    U = np.linalg.qr(crandn(rng, (1 << L, 1 << L)))[0]
+    V = np.stack([haar_unitary(rng) for _ in range(DEPTH)])
+    Z, P = crandn(rng, (DEPTH, 4, 4)), brickwall_perms(L, DEPTH)
+    T = R.DeviceTarget.dense(U)
+    yield V, Z, P, T, O.brickwall_unitary_target_hvp(O.Ufunc.dense(U), V, Z, P, L)
+    T.close()
+
+
+def _limit():
+    """Three quarters of the array that one evaluation sweeps: no cyclic-product sweep, several blocks."""
+    R.set_workspace_limit((16 if R.get_precision() == R.PRECISION_FP64 else 8) * 3 << (2 * L - 2))
+
+
+def _launches():
+    return R.profile_query(R.KERNEL_FORWARD)[1]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_tuning_follows_the_sweeps_that_run(problem, prec):
+    """An evaluation on the cyclic-product sweeps has no tile to choose and leaves none behind: under a
+    limit the same structure is then tuned (4 candidates, 3 runs each, before the evaluation) once."""
+    V, Z, P, T, (f_o, dv_o, hz_o) = problem
+    R.set_precision(R.PRECISION_FP64 if prec == "fp64" else R.PRECISION_MIXED)
+    R.set_eval_autotune(True, forget=True)
+    hvp = lambda: R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)   # noqa: E731
+    R.profile_enable(True)
+    try:
+        counts = []
+        for limited in (False, False, True, True):
+            if limited:
+                _limit()
+            R.profile_reset()
+            f, dv, hz = hvp()
+            assert (R.last_column_block() < 1 << L) == limited
+            counts.append(_launches())
+    finally:
+        R.profile_enable(False)
+        R.profile_reset()
+    print(counts, R.last_tiles(), flush=True)
+    assert counts[0] == counts[1] and counts[2] >= 5 * counts[3]
+    K, logC, gmax = R.last_tiles()
+    base = 10 if prec == "fp64" else 11
+    assert K + logC in (base, base - 1) and gmax in (8, 6)
+    tol = TOL if prec == "fp64" else 1e-4
+    assert abs(f - f_o) < (TOL if prec == "fp64" else 1e-6 * (1 << L)) and reldiff(dv, dv_o) < tol and reldiff(hz, hz_o) < tol
