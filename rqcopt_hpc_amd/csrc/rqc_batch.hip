@@ -129,8 +129,8 @@ static void batch_release(Batch& bt)
 	for (auto& e : bt.ev_join) { (void)hipEventDestroy(e); }
 }
 
-static void batch_init(Batch& bt, int n, const rqc_batch_problem* pr, int precision, int nstreams, size_t limit,
-	const TileChoice& tc)
+// the problems' plans and the layout of the arena; no GPU memory is allocated
+static void batch_plan(Batch& bt, int n, const rqc_batch_problem* pr, int precision, size_t limit, const TileChoice& tc)
 {
 	if (n < 1) { throw Error(-3, "a batch needs at least one problem"); }
 	if (precision != RQC_PRECISION_FP64 && precision != RQC_PRECISION_MIXED) { throw Error(-3, "unknown precision"); }
@@ -205,6 +205,12 @@ static void batch_init(Batch& bt, int n, const rqc_batch_problem* pr, int precis
 	bt.up_bytes = bt.off_res;
 	bt.down_bytes = ress;
 	bt.arena_bytes = bt.off_work + works;
+}
+
+static void batch_init(Batch& bt, int n, const rqc_batch_problem* pr, int precision, int nstreams, size_t limit,
+	const TileChoice& tc)
+{
+	batch_plan(bt, n, pr, precision, limit, tc);
 	RQC_HIP(hipMalloc(&bt.arena, bt.arena_bytes));
 	RQC_HIP(hipHostMalloc(reinterpret_cast<void**>(&bt.h_up), bt.up_bytes, hipHostMallocDefault));
 	RQC_HIP(hipHostMalloc(reinterpret_cast<void**>(&bt.h_down), std::max<size_t>(bt.down_bytes, 256), hipHostMallocDefault));
@@ -924,6 +930,22 @@ static TileChoice tune_batch(int n, const rqc_batch_problem* pr, int precision, 
 	return best;
 }
 
+// Whether any of the batch's plans has a tile to choose (or the default plans do not fit and another
+// candidate's may).  Cyclic-product sweeps have none: a batch of them alone is not timed, which took
+// 16 ms for 2 problems and 72 ms for 8, of four candidates that are the same.
+static bool has_tiles(int n, const rqc_batch_problem* pr, int precision, size_t limit)
+{
+	Batch tmp;
+	try {
+		batch_plan(tmp, n, pr, precision, limit, TileChoice{0, 0});
+	} catch (const Error&) {
+		return true;
+	}
+	return std::any_of(tmp.probs.begin(), tmp.probs.end(), [](const BatchProblem& b) {
+		return std::any_of(b.plan, b.plan + kKinds, [](const EvalPlan& pl) { return !pl.cyc; });
+	});
+}
+
 extern "C" int rqc_batch_create(int nproblems, const struct rqc_batch_problem problems[], int precision, int nstreams,
 	size_t workspace_limit, struct rqc_batch** batch)
 {
@@ -931,7 +953,9 @@ extern "C" int rqc_batch_create(int nproblems, const struct rqc_batch_problem pr
 	try {
 		h = new rqc_batch();
 		TileChoice tc{0, 0};
-		if (ctx().autotune && nproblems > 0) { tc = tune_batch(nproblems, problems, precision, nstreams, workspace_limit); }
+		if (ctx().autotune && nproblems > 0 && has_tiles(nproblems, problems, precision, workspace_limit)) {
+			tc = tune_batch(nproblems, problems, precision, nstreams, workspace_limit);
+		}
 		batch_init(h->b, nproblems, problems, precision, nstreams, workspace_limit, tc);
 		*batch = h;
 		return 0;

@@ -6,6 +6,7 @@ FP64 results match the oracle within 1e-12, mixed precision within its stated bo
 gradient and HVP within 1e-4.
 """
 import os
+import time
 
 import numpy as np
 import pytest
@@ -84,3 +85,30 @@ def test_tuning_follows_the_sweeps_that_run(problem, prec):
     assert K + logC in (base, base - 1) and gmax in (8, 6)
     tol = TOL if prec == "fp64" else 1e-4
     assert abs(f - f_o) < (TOL if prec == "fp64" else 1e-6 * (1 << L)) and reldiff(dv, dv_o) < tol and reldiff(hz, hz_o) < tol
+
+
+def test_batches_without_a_tile_to_choose_are_not_timed():
+    """Creating a batch that runs cyclic-product sweeps alone takes about as long with autotuning as
+    without it: twice at most, where timing four candidates took ten times.  Least of five, each
+    another structure."""
+    rng = np.random.default_rng(43)
+    targets = {n: R.DeviceTarget.brickwall(np.stack([haar_unitary(rng)]), brickwall_perms(n, 1)) for n in (8, 10)}
+
+    def create(on):
+        R.set_autotune(on)
+        best = 1e9
+        for _ in range(5):
+            pr = [(np.stack([rng.permutation(n).astype(np.int32) for _ in range(3)]), targets[n]) for n in (8, 10, 8, 10, 8, 10)]
+            t0 = time.perf_counter()
+            B = R.Batch(pr)
+            best = min(best, time.perf_counter() - t0)
+            B.close()
+        return best
+
+    try:
+        create(False)
+        off, on = create(False), create(True)
+    finally:
+        R.set_autotune(True)
+    print(f"without {1e3 * off:.2f} ms, with {1e3 * on:.2f} ms", flush=True)
+    assert on < 2 * off
