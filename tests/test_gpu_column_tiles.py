@@ -112,3 +112,74 @@ def test_batches_without_a_tile_to_choose_are_not_timed():
         R.set_autotune(True)
     print(f"without {1e3 * off:.2f} ms, with {1e3 * on:.2f} ms", flush=True)
     assert on < 2 * off
+
+
+# overrides and the reverse tile (K, logC) that has to run; the forward tile follows RQC_FWD_TILE (twice the
+# columns by default, one more row bit "k", the reverse pass's own "0")
+FP64_SHAPES = {
+    "64x16": ({}, (6, 4)),
+    "64x8_fwd_64x16": ({"RQC_TILE_LOGE_FP64": "9"}, (6, 3)),
+    "64x8_fwd_128x8": ({"RQC_TILE_LOGE_FP64": "9", "RQC_FWD_TILE": "k"}, (6, 3)),
+    "64x8_fwd_same": ({"RQC_TILE_LOGE_FP64": "9", "RQC_FWD_TILE": "0"}, (6, 3)),
+    "128x8": ({"RQC_TILE_LOGE_FP64": "10", "RQC_TILE_LOGC_FP64": "3"}, (7, 3)),
+}
+FP32_SHAPES = {
+    "64x32": ({}, (6, 5)),
+    "64x16_fwd_64x32": ({"RQC_TILE_LOGE_FP32": "10"}, (6, 4)),
+    "64x16_fwd_128x16": ({"RQC_TILE_LOGE_FP32": "10", "RQC_FWD_TILE": "k"}, (6, 4)),
+    "64x16_fwd_same": ({"RQC_TILE_LOGE_FP32": "10", "RQC_FWD_TILE": "0"}, (6, 4)),
+}
+
+
+@pytest.mark.parametrize("name", list(FP64_SHAPES))
+def test_fp64_column_tiles_match_the_oracle(problem, name):
+    V, Z, P, T, (f_o, dv_o, hz_o) = problem
+    env, shape = FP64_SHAPES[name]
+    os.environ.update(env)
+    _limit()
+    print("tile", name, flush=True)
+    for out in (R.brickwall_unitary_target(T, V, P), R.brickwall_unitary_target_and_gradient(T, V, P),
+                R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)):
+        assert R.last_sweep()[0] == R.ENGINE_TILE_PASS and R.last_tiles()[:2] == shape and R.last_column_block() < 1 << L
+        out = out if isinstance(out, tuple) else (out,)
+        assert abs(out[0] - f_o) < TOL * max(1, abs(f_o))
+        for a, b in zip(out[1:], (dv_o, hz_o)):
+            assert reldiff(a, b) < TOL
+
+
+@pytest.mark.parametrize("name", list(FP32_SHAPES))
+def test_mixed_column_tiles_within_bounds(problem, name):
+    V, Z, P, T, (f_o, dv_o, hz_o) = problem
+    env, shape = FP32_SHAPES[name]
+    os.environ.update(env)
+    R.set_precision(R.PRECISION_MIXED)
+    _limit()
+    print("tile", name, flush=True)
+    f, dv, hz = R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+    assert R.last_sweep()[0] == R.ENGINE_TILE_PASS and R.last_tiles()[:2] == shape and R.last_column_block() < 1 << L
+    assert abs(f - f_o) / (1 << L) < 1e-6 and reldiff(dv, dv_o) < 1e-4 and reldiff(hz, hz_o) < 1e-4
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_issued_flops_of_a_column_sweep(problem, prec):
+    """The counters' formula per amplitude and gate, in column blocks (64 x 16 or 64 x 32 tiles): forward
+    96 algorithmic, 72 (FP64) or 128 (FP32) issued; reverse 192, with the recovery and both outer products
+    240 or 384 issued.  The first pass leaves out tiles without an identity element: of the 25 gates in at
+    least 4 passes, all but 8 count in full."""
+    V, Z, P, T, _ = problem
+    R.set_precision(R.PRECISION_FP64 if prec == "fp64" else R.PRECISION_MIXED)
+    _limit()
+    R.profile_enable(True)
+    try:
+        R.profile_reset()
+        R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+        fwd, rev = R.profile_query_flops(R.KERNEL_FORWARD), R.profile_query_flops(R.KERNEL_REVERSE)
+    finally:
+        R.profile_enable(False)
+        R.profile_reset()
+    assert R.last_column_block() < 1 << L
+    work = float(DEPTH * (L // 2)) * (1 << (2 * L))
+    issued = (72, 240) if prec == "fp64" else (128, 384)
+    for (alg, done), per, i in zip((fwd, rev), (96, 192), issued):
+        assert (1 - 8 / 25) * per * work < alg <= per * work * (1 + 1e-12)
+        assert abs(done / alg - i / per) < 1e-12
