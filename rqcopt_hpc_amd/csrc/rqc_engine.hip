@@ -2346,7 +2346,10 @@ extern "C" int quantum_circuit_gates_hessian_vector_product(const struct mat4x4 
 		std::lock_guard<std::recursive_mutex> lk(c.mu);
 		const size_t bytes = ((size_t)1 << L) * sizeof(zc);
 		const size_t n = (size_t)1 << L;
-		const bool passes = c.engine == RQC_ENGINE_TILE_PASS && ngates > 1 && L <= 30 && gates_near_unitary(C);
+		// (the passes take gates back with G^-1, also from the tangent: after a direction with a NaN or an
+		// infinity the tangents before it would not be finite either)
+		const bool passes = c.engine == RQC_ENGINE_TILE_PASS && ngates > 1 && L <= 30 && gates_near_unitary(C) &&
+			std::all_of(C.dirs.begin(), C.dirs.end(), [](const zc& z) { return std::isfinite(z.x) && std::isfinite(z.y); });
 		const std::vector<StatePass> plan = passes ? plan_state(C) : std::vector<StatePass>();
 		const StateSums sums(c, ngates, L, passes ? 1u << (L - plan[0].tile.K) : 0);
 		Staging s(c);

@@ -46,3 +46,23 @@ def test_passes_match_gate_launches(L, ngates):
         c = O.quantum_circuit_gates_hvp(g, z, w, psi, phi)
         for x, y in zip(a, c):
             assert reldiff(x, y) < TOL or np.max(np.abs(y)) == 0
+
+
+@pytest.mark.parametrize("L,ngates,bad", [(4, 5, np.nan), (10, 25, np.inf), (12, 30, np.nan)])
+def test_a_direction_that_is_not_finite_spoils_what_depends_on_it_alone(L, ngates, bad):
+    """The gradients, and the HVP's entries of gates that no path connects with the direction, stay
+    finite: those of the launches of one gate each."""
+    print("qubits", L, "gates", ngates, bad, flush=True)
+    rng = np.random.default_rng(20 * L + ngates)
+    g = np.stack([haar_unitary(rng) for _ in range(ngates)])
+    z = crandn(rng, (ngates, 4, 4))
+    z[ngates // 2, 1, 2] = bad
+    w = np.array([rng.choice(L, 2, replace=False) for _ in range(ngates)], dtype=np.int32)
+    psi, phi = (v / np.linalg.norm(v) for v in crandn(rng, (2, 1 << L)))
+    a = R.quantum_circuit_gates_hessian_vector_product(g, z, w, psi, phi)
+    R.set_sweep_engine(R.ENGINE_PER_GATE)
+    b = R.quantum_circuit_gates_hessian_vector_product(g, z, w, psi, phi)
+    assert np.isfinite(a[0]).all() and np.isfinite(a[1]).all() and np.isfinite(b[2]).any()
+    assert np.array_equal(np.isfinite(a[2]), np.isfinite(b[2]))
+    on = np.isfinite(b[2])
+    assert reldiff(a[1], b[1]) < TOL and np.max(np.abs(a[2][on] - b[2][on])) < TOL * np.max(np.abs(b[2][on]))
