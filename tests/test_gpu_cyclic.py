@@ -153,3 +153,44 @@ def test_f_of_every_kind_is_as_accurate():
     target, gradient, hvp = np.sqrt(np.mean(np.array(err, float) ** 2, axis=0))
     print(target, gradient, hvp, flush=True)
     assert gradient < 1.35 * target and hvp < 1.35 * target
+
+
+@pytest.mark.parametrize("prec", [R.PRECISION_FP64, R.PRECISION_MIXED])
+@pytest.mark.parametrize("L,ngates", [(5, 9), (9, 30), (10, 30), (11, 50)])
+def test_f_of_gates_that_are_not_unitary(L, ngates, prec):
+    """A target evaluation takes any gates onto the cyclic-product sweeps in FP64 (gradients and mixed
+    precision go gate by gate), at the change of the tile size too; within 1e-12 (mixed: 2e-6 of the
+    norm) of the per-gate engine."""
+    print("qubits", L, "gates", ngates, "precision", prec, flush=True)
+    rng = np.random.default_rng(11 * L + ngates)
+    g = crandn(rng, (ngates, 4, 4)) / 2
+    w = np.array([rng.choice(L, 2, replace=False) for _ in range(ngates)], dtype=np.int32)
+    T = R.DeviceTarget.dense(crandn(rng, (1 << L, 1 << L)))
+    R.set_precision(prec)
+    f = R.circuit_unitary_target(T, g, w, L)
+    assert R.last_sweep()[0] == (R.ENGINE_TILE_PASS if prec == R.PRECISION_FP64 else R.ENGINE_PER_GATE)
+    R.set_precision(R.PRECISION_FP64)
+    f64, dg = R.circuit_unitary_target_and_gradient(T, g, w, L)
+    assert R.last_sweep()[0] == R.ENGINE_PER_GATE
+    R.set_sweep_engine(R.ENGINE_PER_GATE)
+    f_o, dg_o = R.circuit_unitary_target_and_gradient(T, g, w, L)
+    assert f64 == f_o and np.array_equal(dg, dg_o)
+    # (f is a sum of 4^L products that cancel: its terms' norm is that of the gradient with its gate)
+    norm = np.linalg.norm(dg_o[0]) * np.linalg.norm(g[0])
+    assert abs(f - f_o) < (TOL if prec == R.PRECISION_FP64 else 2e-6) * max(norm, abs(f_o))
+
+
+def test_six_qubits_one_layer_in_column_blocks():
+    """A limit below the arrays at 6 qubits: the column blocks of one pass against the whole array."""
+    L, depth = 6, 1
+    rng = np.random.default_rng(61)
+    V, Z = np.stack([haar_unitary(rng) for _ in range(depth)]), crandn(rng, (depth, 4, 4))
+    P = brickwall_perms(L, depth)
+    T = R.DeviceTarget.brickwall(np.stack([haar_unitary(rng) for _ in range(3)]), brickwall_perms(L, 3))
+    a = R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+    assert R.last_column_block() == 1 << L
+    R.set_workspace_limit(6 * (16 << (2 * L)) // 4)   # a pass's 6 arrays of 16 columns; the cyclic sweeps need 2 of 64
+    c = R.brickwall_unitary_target_hessian_vector_product(T, V, Z, P)
+    assert R.last_column_block() < 1 << L and R.last_sweep()[0] == R.ENGINE_TILE_PASS
+    for x, y in zip(a, c):
+        assert reldiff(x, y) < TOL or np.max(np.abs(y)) == 0
