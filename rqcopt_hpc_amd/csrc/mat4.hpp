@@ -185,21 +185,4 @@ RQC_HD void m4_retract(const zc* u, const double* eta, zc* v)
 	m4_polar(w, v);
 }
 
-// Riemannian gradient and Hessian-vector product of one gate as real 16-vectors
-// (reference src/target.c:650-671): dv, hz are the Euclidean (holomorphic)
-// gradient and directional second derivative, v the gate, z the direction.
-RQC_HD void m4_project_grad_hvp(const zc* v, const zc* z, const zc* dv, const zc* hz, double* grad, double* hvp)
-{
-	zc g[16], h[16], gh[16], pd[16];
-	for (int e = 0; e < 16; e++) { g[e] = conj(dv[e]); }
-	m4_tangent_to_real(v, g, grad);
-	if (hvp != nullptr) {
-		for (int e = 0; e < 16; e++) { h[e] = conj(hz[e]); }
-		m4_adjoint(g, gh);
-		m4_symmetric_triple(z, gh, v, pd);
-		for (int e = 0; e < 16; e++) { h[e] -= pd[e]; }
-		m4_tangent_to_real(v, h, hvp);
-	}
-}
-
 }  // namespace rqc

@@ -33,7 +33,6 @@ struct CycArgs
 typedef int cyc_op_t __attribute__((ext_vector_type(16)));
 static_assert(sizeof(CycOp) == sizeof(cyc_op_t), "descriptor size");
 
-constexpr int cyc_log_threads(int K) { return 6 + 2 * (K - 4); }
 template <int K, bool DUAL> constexpr int cyc_state_bytes() { return (DUAL ? 32 : 16) << (2 * K); }
 constexpr int cyc_mats_per_op(bool dual) { return dual ? 4 : 2; }
 template <int K, bool DUAL> constexpr int cyc_lds_bytes()

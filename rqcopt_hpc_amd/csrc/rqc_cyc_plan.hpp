@@ -84,8 +84,6 @@ struct CycPlan
 	long ntrace = 0;          // tiles of the tracing launch (target evaluations)
 };
 
-// workgroup of a tile of 4^K elements: 4 elements per thread
-constexpr int cyc_threads(int K) { return 64 << (2 * (K - 4)); }
 // parts of a gate's partial trace: diagonal tiles times diagonal waves
 inline long cyc_parts(int L, int K) { return (1L << (L - K)) << (K - 4); }
 

@@ -1334,9 +1334,8 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 }
 
 // per-group sums of per-gate gradients / HVPs and the Riemannian projection
-// (reference src/target.c:526-535 and :650-671; m4_project_grad_hvp), one
-// workgroup per group, an entry of a 4x4 matrix per thread.  One thread per
-// group, with the sums and the six 4x4 products in series, took 28 us at 3
+// (reference src/target.c:526-535 and :650-671), one workgroup per group, an
+// entry of a 4x4 matrix per thread.  One thread per group, with the sums and the six 4x4 products in series, took 28 us at 3
 // groups of 3 gates and 60 us at 9 groups of 7; the entries' loads are
 // independent here (4 and 6 us).
 // res: f, dv[16 ng], hz[16 ng] (complex), grad[16 ng], hvp[16 ng] (double)
