@@ -74,17 +74,21 @@ int rqc_set_sweep_engine(int engine);
 /* tile-shape autotuning of batches (process-wide; default on, or the
    environment variable RQC_AUTOTUNE=0 switches it off): the tile height and
    the gates per pass are timed on whole steps of the batch, once per batch
-   structure and precision */
+   structure and precision.  Batches whose problems all fit as whole arrays
+   (rqc_last_tiles) have no tile to choose and are not timed */
 int rqc_set_autotune(int on);
 
 /* tile autotuning of single evaluations (process-wide; default off, or the environment
    variable RQC_EVAL_AUTOTUNE=1): the first target / gradient / HVP evaluation of a circuit
    structure times the tile height (2^10 or 2^9 FP64 elements, 2^11 or 2^10 FP32, which fixes the
    fused qubits K per pass) and the most gates per pass (8 or 6) on the evaluation itself and keeps
-   the fastest for that structure; on = 2 also forgets the choices made so far */
+   the fastest for that structure; on = 2 also forgets the choices made so far.  Only evaluations in
+   column blocks have a tile to choose: dense targets of 5 to 16 qubits take them where the arrays of
+   the whole target do not fit the workspace */
 int rqc_set_eval_autotune(int on);
 /* tile shape (2^rows x 2^cols amplitudes; 2^cols the elements of a contiguous run) and most gates
-   per pass of the last evaluation */
+   per pass of the last evaluation; an evaluation over the whole of a dense target has tiles of
+   2^rows x 2^rows elements (rows 5 or 6), runs of 16 elements (cols 4) and at most 8 gates */
 int rqc_last_tiles(int* tile_rows_log2, int* tile_cols_log2, int* gates_per_pass);
 
 /* device workspace: upper bound in bytes (0 = automatic, about 85% of free HBM);
@@ -108,13 +112,13 @@ void rqc_profile_reset(void);
 int rqc_profile_query(int kind, double* total_ms, long* launches, double* alg_bytes);
 /* algorithmic flops of the timed tile-pass launches of one kind (per amplitude and gate of the
    tiles a launch processes: forward 96, reverse 192 for the adjoint update and the outer
-   products, plain sweeps a third of these; a reverse launch that carries a forward pass adds
-   that pass's), and the flops the matrix cores issue for them: the reverse passes' state
-   recovery besides, in the forms the kernels use (FP64 dual: forward 72, reverse 240, with three
-   real products per complex gate product; FP32 the real 16 x 16 form: forward 128, reverse 384).
-   FP64 evaluations over the whole of a dense target sweep one array (U^dagger with the circuit's
-   gates on either side): its forward products count as forward (96, issued 72), a gate's
-   conjugation as reverse, by what it issues (144).
+   products, plain sweeps a third of these), and the flops the matrix cores issue for them: the
+   reverse passes' state recovery besides, in the forms the kernels use (column blocks, dual sweeps:
+   FP64 forward 72, reverse 240, with three real products per complex gate product; FP32 the real
+   16 x 16 form, forward 128, reverse 384).
+   Evaluations over the whole of a dense target, in FP64 and mixed precision, sweep one array
+   (U^dagger with the circuit's gates on either side): its forward products count as forward (96,
+   issued 72), a gate's conjugation as reverse, by what it issues (144).
    No reference counterpart: the library's own measurement. */
 int rqc_profile_query_flops(int kind, double* alg_flops, double* issued_flops);
 

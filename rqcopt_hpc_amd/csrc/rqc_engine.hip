@@ -13,8 +13,9 @@
 // (src/quantum_circuit.c:147-236) evaluated for all columns of the block, with
 // the tangent-forward folded into the forward sweep (dual numbers).
 // The column blocks cover all N columns; B is the largest power of two whose
-// checkpoints fit the device workspace.  FP64 evaluations over the whole of a dense target that
-// has room for its arrays sweep the product U^dagger W itself instead (rqc_cyc_plan.hpp).
+// checkpoints fit the device workspace.  Evaluations over the whole of a dense target, in FP64 and in
+// mixed precision, sweep the product U^dagger W itself instead where there is room for its arrays
+// (rqc_cyc_plan.hpp).
 
 #include <algorithm>
 #include <cstring>
@@ -1339,8 +1340,8 @@ static void run_cyc(Slot& s, const EvalPlan& pl, const zc* dU, zc* d_acc, zc* d_
 // groups of 3 gates and 60 us at 9 groups of 7; the entries' loads are
 // independent here (4 and 6 us).
 // res: f, dv[16 ng], hz[16 ng] (complex), grad[16 ng], hvp[16 ng] (double)
-// fcorr (FP32 sweeps with a gradient): the sweeps applied the gates rounded to
-// complex float, fl(V), so the accumulated f is f(fl(V)).  f(V) = f(fl(V)) +
+// fcorr (mixed precision with a gradient): the sweeps applied the gates rounded
+// to complex float, fl(V), so the accumulated f is f(fl(V)).  f(V) = f(fl(V)) +
 // sum_e dv[e] (V[e] - fl(V)[e]) + O(|V - fl(V)|^2), with dv = df/dV (f is
 // holomorphic in the gates for the trace targets: fcorr 1 corrects the complex
 // f; the block-encoding f is real with df = Re sum dv dV: fcorr 2 corrects its
@@ -2684,9 +2685,9 @@ extern "C" int brickwall_unitary_target_projected_hessian_vector_product(linear_
 // partial sums, tables, results) fits kScratchBytes, and no device memory is
 // allocated or freed.  U must be a device target (a host callback would need a
 // device copy of U).  Calls hold the library lock and synchronise before they
-// return, so they never overlap on the device; the scratch keeps the last
-// call's contents, and every buffer that must start at zero is cleared by the
-// evaluation's own fill kernels.
+// return, so they never overlap on the device.  The scratch keeps the last
+// call's contents: the sweeps store their first sums (per-gate engine: a fill
+// kernel clears them) and read nothing that they have not written.
 static EvalPlan plan_in_scratch(const Context& c, const Circuit& C, Mode mode, int per, bool fp32, bool project,
 	bool unitary)
 {

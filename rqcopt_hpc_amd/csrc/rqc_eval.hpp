@@ -58,7 +58,7 @@ struct TileChoice
 struct EvalPlan
 {
 	Mode mode = Mode::Target;
-	bool fp32 = false;     // complex FP32 sweeps (mixed precision)
+	bool fp32 = false;     // mixed precision: arrays in complex FP32 (products: FP64 with cyc, else FP32)
 	bool project = false;  // Riemannian projection of gradient and HVP
 	bool tiles = false;    // tile-pass engine (else one gate per pass)
 	bool cyc = false;      // cyclic-product sweeps (with tiles; rqc_cyc_plan.hpp)
@@ -84,9 +84,9 @@ struct EvalPlan
 	double state_bytes() const { return (double)nst * N * B * (fp32 ? 8.0 : 16.0); }
 };
 
-// In mixed precision (fp32) a target evaluation is planned as a gradient evaluation: the FP32
-// sweeps apply the gates rounded to complex float, and f is corrected to first order for that
-// rounding with the gate gradient (k_finalize), so that every mixed-precision f, with or without
+// In mixed precision (fp32) a target evaluation is planned as a gradient evaluation: the sweeps
+// apply the gates rounded to complex float (also those that multiply in FP64), and f is corrected
+// to first order for that rounding with the gate gradient (k_finalize), so that every mixed-precision f, with or without
 // a gradient, is computed the same way (a trust-region ratio compares f values of both kinds).
 // `unitary`: the gates pass gates_near_unitary (the tile-pass engine is used for
 // reverse sweeps only then; see sweep_unitary); `budget`: bytes for the state arrays
