@@ -120,7 +120,7 @@ def run(args):
     V, P, vec, Z = config_inputs(L, d, args.seed)
     Vt, Pt = ising_trotter_brickwall(L, 1.0, 0.75, 0.6, 0.5, 4)
     T = R.DeviceTarget.brickwall(Vt, Pt)
-    # tile shape and gates per pass timed on the first (warm-up) evaluation of each precision
+    # in column blocks, tile shape and gates per pass are timed on the first (warm-up) evaluation of each precision
     R.set_eval_autotune(not args.no_autotune)
 
     def one():
@@ -224,7 +224,7 @@ def run(args):
         "config": {"workload": f"brickwall grad+HVP eval, L={L}, depth {d}, periodic, Ising-Trotter U (t=0.5, 4 Strang steps)",
                    "L": L, "depth": d, "gates": G, "column_block": B, "sweep_engine": engine, "device": info,
                    "tiles": {"fp64": r64["tiles"], "mixed": r32["tiles"],
-                             "autotuned": not args.no_autotune,
+                             "autotuned": not args.no_autotune and engine == "tile_pass" and B < N,
                              "fields": "log2 tile rows (fused qubits K), log2 tile columns, most gates per pass"}},
         "roofline": ({"bound": "mfma", "achieved": achieved_tf, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                       "frac": achieved_tf / FP64_PEAK_TFLOPS, "traffic": traffic,
