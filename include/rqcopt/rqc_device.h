@@ -92,7 +92,7 @@ int rqc_set_eval_autotune(int on);
 int rqc_last_tiles(int* tile_rows_log2, int* tile_cols_log2, int* gates_per_pass);
 
 /* device workspace: upper bound in bytes (0 = automatic, about 85% of free HBM);
-   the workspace is kept between calls and released here */
+   the workspace is kept between calls and released here, with the plans kept of the last circuits */
 int rqc_set_workspace_limit(size_t bytes);
 void rqc_release_workspace(void);
 /* column-block width used by the last target evaluation */

@@ -440,10 +440,11 @@ static std::vector<int> structure_ints(const Circuit& C, std::initializer_list<i
 	return key;
 }
 
+static PlanCache<std::vector<Pass>> g_passes;
+
 static std::vector<Pass> cached_passes(const Circuit& C, int K, int gmax)
 {
-	static PlanCache<std::vector<Pass>> cache;
-	return *cache.get(structure_ints(C, {K, gmax}), [&] { return std::make_shared<const std::vector<Pass>>(plan_passes(C, K, gmax)); });
+	return *g_passes.get(structure_ints(C, {K, gmax}), [&] { return std::make_shared<const std::vector<Pass>>(plan_passes(C, K, gmax)); });
 }
 
 // Kernel arguments of a pass.  Tile-bit order: the two least used bits of the
@@ -839,10 +840,11 @@ struct CycCircuit
 	std::vector<CycPass> passes;
 };
 
+static PlanCache<CycCircuit> g_cyc_circuits;
+
 static std::shared_ptr<const CycCircuit> cyc_circuit(const Circuit& C, int K)
 {
-	static PlanCache<CycCircuit> cache;
-	return cache.get(structure_ints(C, {K}), [&] {
+	return g_cyc_circuits.get(structure_ints(C, {K}), [&] {
 		auto cc = std::make_shared<CycCircuit>();
 		std::vector<int> gi(C.ngates), gj(C.ngates);
 		for (int k = 0; k < C.ngates; k++) {
@@ -889,11 +891,12 @@ static std::shared_ptr<const TilePlan> make_cyc_tiles(const Context& dev, const 
 	return tp;
 }
 
+static PlanCache<TilePlan> g_cyc_plans;
+
 static std::shared_ptr<const TilePlan> plan_cyc(const Context& dev, const Circuit& C, const CycCircuit& cc, int split, bool dual, bool fp32,
 	bool target_only, int K)
 {
-	static PlanCache<TilePlan> cache;
-	return cache.get(structure_ints(C, {K, dual, fp32, target_only, dev.device}),
+	return g_cyc_plans.get(structure_ints(C, {K, dual, fp32, target_only, dev.device}),
 		[&] { return make_cyc_tiles(dev, C, cc, split, dual, fp32, target_only, K); });
 }
 
@@ -3540,6 +3543,9 @@ extern "C" void rqc_release_workspace(void)
 		c.vecs.release();
 		c.ubuf.release();
 		c.io.release();
+		g_passes.clear();
+		g_cyc_circuits.clear();
+		g_cyc_plans.clear();
 	} catch (...) {}
 }
 

@@ -1,6 +1,8 @@
 // Plans by circuit structure (host).  A program evaluates one structure many times with new gates; a
 // plan costs from 20 us (6 qubits, 3 layers) to 0.8 ms (14 qubits, 9 layers).  The last kMost plans are
-// kept (host memory only); the key holds the whole structure, nothing of the gates.
+// kept (host memory only, given back by clear), fewer of large circuits: a gate takes 2 integers of the
+// key and up to 1 KB of a plan, so that kMostInts bounds a cache at about 32 MB.  The key holds the
+// whole structure, nothing of the gates.
 #pragma once
 
 #include <cstddef>
@@ -26,13 +28,26 @@ public:
 		std::lock_guard<std::mutex> lk(mu_);
 		if (auto p = find_locked(key)) { return p; }
 		plans_.emplace_front(key, made);
-		if (plans_.size() > kMost) { plans_.pop_back(); }
+		ints_ += key.size();
+		while (plans_.size() > 1 && (plans_.size() > kMost || ints_ > kMostInts)) {
+			ints_ -= plans_.back().first.size();
+			plans_.pop_back();
+		}
 		return made;
 	}
 
+	// (plans in use stay with their users)
+	void clear()
+	{
+		std::lock_guard<std::mutex> lk(mu_);
+		plans_.clear();
+		ints_ = 0;
+	}
+
 private:
-	static constexpr size_t kMost = 64;
+	static constexpr size_t kMost = 64, kMostInts = (size_t)1 << 16;
 	std::mutex mu_;
+	size_t ints_ = 0;   // of the keys kept
 	std::list<std::pair<std::vector<int>, std::shared_ptr<const P>>> plans_;
 
 	std::shared_ptr<const P> find(const std::vector<int>& key)

@@ -55,6 +55,15 @@ int main()
 	for (int k = 100; k < 163; k++) { cache.get({k}, plan(k)); }
 	const int two = *cache.get({2}, plan(-2)), one = *cache.get({1}, plan(-2));
 	printf("%d %d\n", two, one);
+	// few of large circuits (keys of 20000 integers: three), the newest whatever its size
+	std::weak_ptr<const int> kept[5];
+	for (int k = 0; k < 4; k++) { kept[k] = cache.get(std::vector<int>(20000, k), plan(k)); }
+	kept[4] = cache.get(std::vector<int>(100000, 4), plan(4));
+	printf("%d%d%d%d%d", kept[0].expired(), kept[1].expired(), kept[2].expired(), kept[3].expired(), kept[4].expired());
+	for (int k = 0; k < 4; k++) { kept[k] = cache.get(std::vector<int>(20000, k), plan(k)); }
+	printf(" %d%d%d%d%d", kept[0].expired(), kept[1].expired(), kept[2].expired(), kept[3].expired(), kept[4].expired());
+	cache.clear();
+	printf(" %d%d%d%d\n", kept[0].expired(), kept[1].expired(), kept[2].expired(), kept[3].expired());
 }
 """
 
@@ -62,7 +71,7 @@ int main()
 def test_a_thread_that_plans_does_not_keep_others_from_their_plans(tmp_path):
     r = _run(_build(tmp_path, CACHE))
     assert r.returncode == 0, r.stderr
-    assert r.stdout.split("\n")[:2] == ["1 10 1 21", "21 -2"]
+    assert r.stdout.split("\n")[:3] == ["1 10 1 21", "21 -2", "11110 10001 1111"]
 
 
 PLAN = r"""
