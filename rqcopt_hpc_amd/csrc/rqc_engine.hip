@@ -1514,7 +1514,7 @@ void unpack_result(const EvalPlan& pl, const char* res, EvalResult& R)
 // dense U for a target evaluation: device-resident or assembled from the host callback
 static const zc* resolve_target(Context& c, linear_func ufunc, void* udata, int L);
 
-// Tile autotuning of single evaluations (rqc_set_eval_autotune): the first evaluation of a
+// Tile autotuning of single evaluations (rqc_set_eval_autotune): the first evaluation in column blocks of a
 // circuit structure (qubits, wires, groups, kind, precision, projection) times the tile
 // candidates on the evaluation itself (one untimed run, then the best of two, HIP events on the
 // library's stream) and keeps the fastest for every later evaluation of that structure.  The
@@ -1537,9 +1537,6 @@ static std::map<std::string, TileChoice>& tuned_choices()
 static TileChoice tune_eval(Context& c, const Circuit& C, Mode mode, int per, bool project, bool unitary, const zc* dU)
 {
 	const bool fp32 = c.precision == RQC_PRECISION_MIXED;
-	const std::string key = structure_key(C, mode, per, fp32, project);
-	auto it = tuned_choices().find(key);
-	if (it != tuned_choices().end()) { return it->second; }
 	const int base = fp32 ? 11 : 10;
 	const TileChoice cands[] = {{base, 8}, {base - 1, 8}, {base, 6}, {base - 1, 6}};
 	TileChoice best{0, 0};
@@ -1572,7 +1569,6 @@ static TileChoice tune_eval(Context& c, const Circuit& C, Mode mode, int per, bo
 	}
 	(void)hipEventDestroy(e0);
 	(void)hipEventDestroy(e1);
-	tuned_choices()[key] = best;
 	return best;
 }
 
@@ -1604,13 +1600,17 @@ static EvalResult eval_targets(const Circuit& C, linear_func ufunc, void* udata,
 	Context& c = ctx();
 	std::lock_guard<std::recursive_mutex> lk(c.mu);
 	const zc* dU = resolve_target(c, ufunc, udata, C.L);
-	const bool unitary = sweep_unitary(C, mode, c.precision == RQC_PRECISION_MIXED);
-	const bool fp32 = c.precision == RQC_PRECISION_MIXED;
-	EvalPlan pl = plan_eval(c, C, mode, per, fp32, project, unitary, c.ws_limit, c.work.bytes);
+	const bool fp32 = c.precision == RQC_PRECISION_MIXED, unitary = sweep_unitary(C, mode, fp32);
 	// (only column sweeps have a tile shape to choose; whether a structure takes them depends on the
 	// workspace limit, so that an evaluation of the other kind decides nothing for it)
-	if (c.eval_autotune && pl.tiles && !pl.cyc) {
-		const TileChoice tc = tune_eval(c, C, mode, per, project, unitary, dU);
+	const bool tune = c.eval_autotune && c.engine == RQC_ENGINE_TILE_PASS;
+	const std::string key = tune ? structure_key(C, mode, per, fp32, project) : std::string();
+	const auto it = tuned_choices().find(key);
+	const bool known = tune && it != tuned_choices().end();
+	TileChoice tc = known ? it->second : TileChoice{0, 0};
+	EvalPlan pl = plan_eval(c, C, mode, per, fp32, project, unitary, c.ws_limit, c.work.bytes, tc.logE > 0 ? &tc : nullptr);
+	if (tune && !known && pl.tiles && !pl.cyc) {
+		tc = tuned_choices()[key] = tune_eval(c, C, mode, per, project, unitary, dU);
 		if (tc.logE > 0) { pl = plan_eval(c, C, mode, per, fp32, project, unitary, c.ws_limit, c.work.bytes, &tc); }
 	}
 	return run_eval(c, pl, C, dU, nullptr, nullptr, nullptr);
