@@ -129,10 +129,23 @@ int main(int argc, char** argv)
 		}
 		best = std::min(best, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count());
 	}
-	printf("%.0f\n", best);
+	// the host's speed: a sort of 20000 numbers
+	double yard = 1e9;
+	for (int rep = 0; rep < 20; rep++) {
+		std::vector<unsigned> v(20000);
+		for (size_t i = 0; i < v.size(); i++) { v[i] = (unsigned)(i * 2654435761u); }
+		const auto t0 = std::chrono::steady_clock::now();
+		std::sort(v.begin(), v.end());
+		yard = std::min(yard, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count());
+		if (v[0] > v[1]) { return 7; }
+	}
+	printf("%.1f %.1f\n", best, yard);
 	return 0;
 }
 """
+
+
+YARD_US = 1000.0   # the program's yardstick where the bounds were measured; they grow with it on slower hosts
 
 
 @pytest.fixture(scope="module")
@@ -149,4 +162,5 @@ def plan(tmp_path_factory):
 def test_plans_hold_every_gate_in_order_and_are_quick(plan, L, layers, ngates, us):
     r = _run(plan, L, layers, ngates)
     assert r.returncode == 0, r.returncode
-    assert float(r.stdout) < us
+    took, yard = map(float, r.stdout.split())
+    assert took < us * max(1, yard / YARD_US)
